@@ -10,13 +10,13 @@
 // decode-time products use (decode_run, kdq_decode.hpp), so each weight byte is read once
 // per workgroup tile instead of once per 8 activation rows.
 //
-//   stage_rows_kernel  one workgroup per token row (rows up to the next multiple of 128,
+//   stage_rows_kernel  one workgroup per token row (rows up to the next whole token tile,
 //                      past m zero): the row's power-of-two scale sigma (max|x| / sigma in
 //                      [2^14, 2^15), 1 for a row whose maximum is below 2^-100, NaN for a
 //                      non-finite row) and fp16(x / sigma) in natural order
-//   rows_gemm_kernel   128 weight rows x 128 tokens per workgroup, four wavefronts each
-//                      owning one 32-row weight operand and all 128 tokens (four 32-token
-//                      blocks).  Per K group (256 values; 64 for BF16) the workgroup copies
+//   rows_gemm_kernel   128 weight rows x up to 128 tokens per workgroup, four wavefronts
+//                      each owning one 32-row weight operand and all the tokens (up to four
+//                      32-token blocks).  Per K group (256 values; 64 for BF16) the workgroup copies
 //                      its rows' raw block bytes into LDS with 16-byte loads (one group
 //                      ahead, double-buffered); per step of 32 values the activations pass
 //                      through LDS (double-buffered, swizzled; loaded up to four steps
@@ -44,7 +44,6 @@ namespace {
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int RM = 128;  // tokens per workgroup: four 32-token blocks
 constexpr int RN = 128;  // weight rows per workgroup: one 32-row operand per wavefront
 constexpr int RK = 32;   // K values per step: two 16-value MFMA sub-steps
 constexpr int kWaves = 4;
@@ -70,8 +69,10 @@ template <int ENC> constexpr unsigned lattice_rows_width = ENC == KDQ_IQ2_S ? 8 
 template <int ENC> constexpr size_t lattice_rows_bytes =
     size_t(lattice_rows_entries<ENC>) * lattice_rows_width<ENC>;
 
-template <int ENC> constexpr size_t rows_lds = 2 * size_t(RN) * RowsGroup<ENC>::pitch +
-                                               2 * size_t(RM) * RK * 2 + lattice_rows_bytes<ENC>;
+// LDS of a workgroup whose token tile is TB blocks of 32 tokens.
+template <int ENC, int TB> constexpr size_t rows_lds =
+    2 * size_t(RN) * RowsGroup<ENC>::pitch + 2 * size_t(32 * TB) * RK * 2 +
+    lattice_rows_bytes<ENC>;
 
 // Fills the LDS grid table (every thread of the workgroup; a barrier follows before use):
 // entry i's level indices (3 or 2 bits each, as iq_grids.inc encodes them) as the levels
@@ -103,15 +104,16 @@ template <int ENC> __device__ __forceinline__ void lattice_rows_table(uint8_t* t
 
 // A lane's 8 fp16 weights: fp16 of each value exactly as decode_run gives it (the same
 // fp32 operations in the same order), from the row's raw group bytes in LDS.  The
-// encodings below read whole code words and look values up four at a time; their range
+// encodings read whole code words and look values up four at a time; their range
 // flags are taken once per call from the block scale: `nonfinite` for a non-finite
 // scale, `wide` when the scale could take a weight past the fp16 range (the largest code
 // times |scale| above 65504, as the packed GEMM checks it); their fp16 scales convert in
-// hardware (exact for every finite half; a NaN stays a NaN).  Other encodings decode
-// value by value and check each value; BF16 checks its bits.
+// hardware (exact for every finite half; a NaN stays a NaN).  Q6_K checks its values and
+// BF16 its bits.
 struct RowFlags {
     bool nonfinite = false, wide = false;
     unsigned bf16_max = 0;  // BF16: the largest |bits| seen (two 16-bit lanes)
+    float peak = 0.f;       // Q6_K: the largest |weight| seen
 };
 
 typedef unsigned u32x2_a8 __attribute__((ext_vector_type(2), aligned(8)));
@@ -145,19 +147,32 @@ __device__ __forceinline__ void scale_signed(f16x8& a, int at, float step, unsig
         a[at + i] = _Float16(mul_rn(step, float(int8_t(q >> (8 * i)))));
 }
 
-template <int ENC> struct RowsDecode {
-    // every other encoding: decode_run, each value checked
+template <int ENC> struct RowsDecode;
+
+// One 210-byte super-block: low nibbles or high nibbles of eight ql bytes, two bits each
+// of eight qh bytes, four codes at a time.  The block scale alone does not bound the
+// weights tightly (codes reach -32 but rarely do), so the largest |weight| is kept.
+// (Value by value from decode_run, 512 x 4096 -> 4096 took 74.8 us; this way 57.1.)
+template <> struct RowsDecode<KDQ_Q6_K> {
     static __device__ __forceinline__ f16x8 run(const uint8_t* row, unsigned kk, RowFlags& f,
                                                 const uint8_t*) {
-        using F = Format<ENC>;
-        float v[8];
-        decode_run<ENC>(row + (kk / F::values) * F::bytes, kk % F::values, v);
+        const unsigned half = kk / 128, q = (kk % 128) / 32, at = kk % 32;
+        const float d = half_hw(lds_u16(row + 208));
+        const float step = mul_rn(d, float(int8_t(row[192 + kk / 16])));
+        f.nonfinite = f.nonfinite || !isfinite(step);
+        const u32x2_a8 l =
+            *reinterpret_cast<const u32x2_a8*>(row + 64 * half + 32 * (q & 1u) + at);
+        const u32x2_a8 h = *reinterpret_cast<const u32x2_a8*>(row + 128 + 32 * half + at);
+        const unsigned sh = q < 2 ? 0u : 4u;
+        const unsigned c[2] = {
+            ((l.x >> sh) & 0x0f0f0f0fu) | (((h.x >> (2 * q)) & 0x03030303u) << 4),
+            ((l.y >> sh) & 0x0f0f0f0fu) | (((h.y >> (2 * q)) & 0x03030303u) << 4)};
         f16x8 a;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            f.nonfinite = f.nonfinite || !isfinite(v[i]);
-            f.wide = f.wide || fabsf(v[i]) > 65504.f;
-            a[i] = _Float16(v[i]);
+            const float v = mul_rn(step, float(int((c[i / 4] >> (8 * (i % 4))) & 255u) - 32));
+            f.peak = fmaxf(f.peak, fabsf(v));
+            a[i] = _Float16(v);
         }
         return a;
     }
@@ -437,19 +452,22 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(const float* __restrict
     }
 }
 
-// Grid: ceil(n / RN) * ceil(m_pad / RM) * slices workgroups, rounded up to a multiple of 8
+// Grid: ceil(n / RN) * ceil(m / RM) * slices workgroups, rounded up to a multiple of 8
 // and ordered so that the token tiles of one weight tile (and K slice) run together on one
-// XCD (its L2 serves the weight bytes to all of them).  xs holds m_pad = ceil(m / RM) * RM
-// rows.  K slices (outputs too narrow to fill the compute units): slice `ks` runs groups
-// [ks * per, (ks + 1) * per) and writes its fp32 tile to part[ks] (m x n, already scaled
-// back by sigma, a power of two: exact), summed in slice order by slice_sum_kernel.
-template <int ENC>
+// XCD (its L2 serves the weight bytes to all of them).  A token tile is RM = 32 TB tokens
+// (rows_plan picks TB); xs holds m_pad = ceil(m / RM) * RM rows.  K slices (outputs too
+// narrow to fill the compute units): slice `ks` runs groups [ks * per, (ks + 1) * per) and
+// writes its fp32 tile to part + ks * part_stride (m x n, already scaled back by sigma, a
+// power of two: exact), summed in slice order by slice_sum_kernel.
+template <int ENC, int TB>
 __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
     const uint16_t* __restrict__ xs, const float* __restrict__ sigma,
     const uint8_t* __restrict__ w, size_t row_bytes, const uint8_t* __restrict__ tail,
     unsigned m, unsigned n, unsigned k, unsigned slices, unsigned per, float* __restrict__ y,
-    float* __restrict__ part, unsigned* __restrict__ status) {
+    float* __restrict__ part, size_t part_stride, unsigned* __restrict__ status) {
     using G = RowsGroup<ENC>;
+    constexpr int RM = 32 * TB;                              // tokens per workgroup
+    constexpr int XP = (RM * 4 + kThreads - 1) / kThreads;  // activation chunks per thread
     extern __shared__ __align__(16) uint8_t lds[];
     uint8_t* raw = lds;                        // [2][RN][pitch]
     uint8_t* xt = lds + 2 * RN * G::pitch;     // [2][RM][RK] fp16, 16-byte chunks swizzled
@@ -465,7 +483,7 @@ __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
         return;  // the whole workgroup, before any barrier
     const unsigned n0 = (linear / (m_tiles * slices)) * RN;
     const unsigned slice = (linear / m_tiles) % slices, m0 = (linear % m_tiles) * RM;
-    float* __restrict__ out_tile = slices > 1 ? part + size_t(slice) * m * n : y;
+    float* __restrict__ out_tile = slices > 1 ? part + slice * part_stride : y;
 
     const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const unsigned lane = threadIdx.x % 64, r = lane % 32, h = lane / 32;
@@ -503,33 +521,35 @@ __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
         for (int j = 0; j < G::per_thread; ++j)
             *reinterpret_cast<u32x4*>(raw + buf * RN * G::pitch + dst[j]) = v[j];
     };
-    // activation copy: thread i moves 16-byte chunks i and i + 256 of the step's RM x 64 B;
+    // activation copy: thread i moves 16-byte chunks i and i + 256 of the step's RM x 64 B
+    // (past the last one, the last one again: the same bytes to the same place);
     // chunk c of token t lands at t * 64 + 16 (c ^ swz(t)), swz(t) = ((t >> 1) ^ (t >> 3))
     // & 3: the 16-byte reads of 8 (or 16) consecutive tokens then cover distinct banks
     // whether a clock serves 128 or 256 bytes
-    const uint8_t* xrow[2];
-    unsigned xdst[2];
+    const uint8_t* xrow[XP];
+    unsigned xdst[XP];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const unsigned q = threadIdx.x + unsigned(j) * kThreads, t = q / 4, c = q % 4;
+    for (int j = 0; j < XP; ++j) {
+        const unsigned q = min(threadIdx.x + unsigned(j) * kThreads, unsigned(RM) * 4 - 1),
+                       t = q / 4, c = q % 4;
         xrow[j] = reinterpret_cast<const uint8_t*>(xs) + size_t(m0 + t) * k * 2 +
                   size_t(g0) * G::values * 2 + 16 * c;
         xdst[j] = t * 64 + 16 * (c ^ (((t >> 1) ^ (t >> 3)) & 3u));
     }
-    auto load_x = [&](unsigned s, u32x4 (&v)[2]) {
+    auto load_x = [&](unsigned s, u32x4 (&v)[XP]) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < XP; ++j)
             v[j] = load16(xrow[j] + size_t(s) * RK * 2);
     };
-    auto store_x = [&](unsigned buf, const u32x4 (&v)[2]) {
+    auto store_x = [&](unsigned buf, const u32x4 (&v)[XP]) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < XP; ++j)
             *reinterpret_cast<u32x4*>(xt + buf * RM * RK * 2 + xdst[j]) = v[j];
     };
 
-    f32x16 acc[4];
+    f32x16 acc[TB];
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < TB; ++b)
         acc[b] = f32x16{};
     RowFlags flags;
 
@@ -548,7 +568,7 @@ __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
     constexpr int kAhead = PG < 4 || ENC == KDQ_Q8_0 || ENC == KDQ_Q6_K ? 2 : 4;
     constexpr int kUnroll = kAhead;
     static_assert(PG % kAhead == 0, "a group is whole turns of the ring");
-    u32x4 rv[G::per_thread], xv[kAhead][2];
+    u32x4 rv[G::per_thread], xv[kAhead][XP];
     load_x(0, xv[0]);
     load_raw(0, rv);
 #pragma unroll
@@ -583,7 +603,7 @@ __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
             const f16x8 a = RowsDecode<ENC>::run(row, kk, flags, table);
             const unsigned c = 2 * sub + h;  // 16-byte chunk of the token's 64 bytes
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
+            for (int b = 0; b < TB; ++b) {
                 const unsigned t = 32 * b + r;
                 const f16x8 xf =
                     *reinterpret_cast<const f16x8*>(xb + t * 64 +
@@ -606,7 +626,7 @@ __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
     // wavefront's 32; scaled back by the token's sigma
     const bool vec = n % 4 == 0;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
+    for (int b = 0; b < TB; ++b) {
         const unsigned tok = m0 + 32 * b + r;
         if (tok >= m)
             continue;
@@ -633,60 +653,105 @@ __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
             flags.nonfinite = mx >= 0x7f80u;
             flags.wide = mx >= 0x4780u && mx < 0x7f80u;
         }
+        if constexpr (ENC == KDQ_Q6_K)
+            flags.wide = flags.peak > 65504.f;
         const unsigned f = (__any(flags.nonfinite) ? 1u : 0u) | (__any(flags.wide) ? 2u : 0u);
         if (f && lane == 0)
             atomicOr(status, f);
     }
 }
 
-// y = sum over the slices of part[s], in slice order; one thread per 4 outputs (m * n % 4
-// == 0 when slices run).
+// y = sum over the slices of part + s * stride, in slice order; one thread per 4 outputs
+// (stride % 4 == 0; the last count % 4 outputs one by one).
 __global__ __launch_bounds__(256) void slice_sum_kernel(const float* __restrict__ part,
-                                                        size_t count, unsigned slices,
-                                                        float* __restrict__ y) {
-    const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= count / 4)
+                                                        size_t count, size_t stride,
+                                                        unsigned slices, float* __restrict__ y) {
+    const size_t i = (size_t(blockIdx.x) * 256 + threadIdx.x) * 4;
+    if (i >= count)
         return;
-    float4 acc = reinterpret_cast<const float4*>(part)[i];
+    float4 acc = *reinterpret_cast<const float4*>(part + i);
     for (unsigned s = 1; s < slices; ++s) {
-        const float4 v = reinterpret_cast<const float4*>(part + s * count)[i];
+        const float4 v = *reinterpret_cast<const float4*>(part + s * stride + i);
         acc.x += v.x;
         acc.y += v.y;
         acc.z += v.z;
         acc.w += v.w;
     }
-    reinterpret_cast<float4*>(y)[i] = acc;
+    if (i + 4 <= count) {
+        *reinterpret_cast<float4*>(y + i) = acc;
+        return;
+    }
+    const float last[3] = {acc.x, acc.y, acc.z};
+    for (unsigned j = 0; i + j < count; ++j)
+        y[i + j] = last[j];
 }
 
-// K slices: enough workgroups for about two per compute unit when the output tiles are
-// fewer; whole groups, none empty, and only where m * n % 4 == 0.
+// The token tile (TB blocks of 32) and the K slices of one call.
 struct RowsPlan {
-    unsigned slices, per;
+    unsigned blocks, slices, per;
 };
 
+// Token tile: the fewest (32-token blocks multiplied + weight passes); a pass decodes the
+// weights once, which costs about as much as multiplying two blocks.  So up to 128 tokens
+// take one pass over no more blocks than they fill (32 x 4096 -> 14336 IQ4_XS: 40.3 us in
+// a 128-token tile, 32.9 in a 32-token one).
+// K slices: enough workgroups for about two per compute unit when the output tiles are
+// fewer; whole groups, none empty; the partials' stride is padded, so m * n may be odd
+// (61 x 13824 -> 3253 Q3_K, 26 output tiles: 324 us in one slice, 51.5 in 18).
 RowsPlan rows_plan(size_t m, size_t n, size_t groups) {
-    const size_t tiles = (m + RM - 1) / RM * ((n + RN - 1) / RN);
+    const size_t need = (m + 31) / 32;
+    size_t blocks = 4, best = ~size_t(0);
+    for (size_t tb : {4, 3, 2, 1}) {
+        const size_t passes = (need + tb - 1) / tb, cost = passes * (tb + 2);
+        if (cost < best) {
+            best = cost;
+            blocks = tb;
+        }
+    }
+    const size_t tiles = (need + blocks - 1) / blocks * ((n + RN - 1) / RN);
     const size_t target = 2 * size_t(compute_units());
-    size_t slices = (m * n) % 4 ? 1 : std::max<size_t>(1, target / tiles);
-    slices = std::min(slices, groups);
+    const size_t slices = std::min(std::max<size_t>(1, target / tiles), groups);
     const size_t per = (groups + slices - 1) / slices;
-    return RowsPlan{unsigned((groups + per - 1) / per), unsigned(per)};
+    return RowsPlan{unsigned(blocks), unsigned((groups + per - 1) / per), unsigned(per)};
 }
 
 struct RowsScratch {
-    size_t m_pad, xs, sigma, tail, total;
+    size_t m_pad, xs, sigma, tail, part_stride, total;
 };
 
 constexpr unsigned kTailSize = 512;  // >= every RowsGroup pitch
 
-RowsScratch rows_scratch(size_t m, size_t n, size_t k, size_t row_bytes, unsigned slices) {
+RowsScratch rows_scratch(size_t m, size_t n, size_t k, const RowsPlan& plan) {
+    const size_t rm = 32 * size_t(plan.blocks);
     RowsScratch s;
-    s.m_pad = (m + RM - 1) / RM * RM;
+    s.m_pad = (m + rm - 1) / rm * rm;
     s.xs = (s.m_pad * k * 2 + 255) / 256 * 256;
     s.sigma = (s.m_pad * 4 + 255) / 256 * 256;
     s.tail = kTailSize;
-    s.total = s.xs + s.sigma + s.tail + (slices > 1 ? size_t(slices) * m * n * 4 : 0);
+    s.part_stride = (m * n + 3) / 4 * 4;
+    s.total = s.xs + s.sigma + s.tail + (plan.slices > 1 ? plan.slices * s.part_stride * 4 : 0);
     return s;
+}
+
+template <int ENC, int TB>
+int launch_rows_gemm(const uint8_t* w, size_t row_bytes, size_t n, size_t k, size_t m,
+                     const RowsPlan& plan, const RowsScratch& s, const uint16_t* xs,
+                     const float* sigma, const uint8_t* tail, float* part, float* y,
+                     unsigned* status, hipStream_t st) {
+    static bool configured = false;  // one attribute call per instantiation
+    constexpr size_t lds = rows_lds<ENC, TB>;
+    if (!configured) {
+        KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&rows_gemm_kernel<ENC, TB>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+        configured = true;
+    }
+    const size_t tiles = s.m_pad / (32 * TB) * ((n + RN - 1) / RN) * plan.slices;
+    hipLaunchKernelGGL((rows_gemm_kernel<ENC, TB>), dim3(unsigned((tiles + 7) / 8 * 8)),
+                       dim3(kThreads), lds, st, xs, sigma, w, row_bytes, tail,
+                       unsigned(m), unsigned(n), unsigned(k), plan.slices, plan.per, y, part,
+                       s.part_stride, status);
+    KDQ_HIP(hipGetLastError());
+    return KDQ_OK;
 }
 
 template <int ENC>
@@ -695,15 +760,8 @@ int launch_rows(const uint8_t* w, size_t row_bytes, size_t n, size_t k, const fl
     using G = RowsGroup<ENC>;
     if (k % G::values)
         return KDQ_ERR_SHAPE;
-    static bool configured = false;  // one attribute call per instantiation
-    if (!configured) {
-        KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&rows_gemm_kernel<ENC>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    int(rows_lds<ENC>)));
-        configured = true;
-    }
     const RowsPlan plan = rows_plan(m, n, k / G::values);
-    const RowsScratch s = rows_scratch(m, n, k, row_bytes, plan.slices);
+    const RowsScratch s = rows_scratch(m, n, k, plan);
     auto* xs = reinterpret_cast<uint16_t*>(scratch);
     auto* sigma = reinterpret_cast<float*>(scratch + s.xs);
     uint8_t* tail = scratch + s.xs + s.sigma;
@@ -714,16 +772,19 @@ int launch_rows(const uint8_t* w, size_t row_bytes, size_t n, size_t k, const fl
                        unsigned(m), unsigned(s.m_pad), unsigned(k), xs, sigma, tail_src,
                        unsigned(G::bytes), unsigned(G::pitch), tail);
     KDQ_HIP(hipGetLastError());
-    const size_t tiles = (s.m_pad / RM) * ((n + RN - 1) / RN) * plan.slices;
-    hipLaunchKernelGGL(rows_gemm_kernel<ENC>, dim3(unsigned((tiles + 7) / 8 * 8)),
-                       dim3(kThreads), rows_lds<ENC>, st, xs, sigma, w, row_bytes, tail,
-                       unsigned(m), unsigned(n), unsigned(k), plan.slices, plan.per, y, part,
-                       status);
-    KDQ_HIP(hipGetLastError());
+    auto run = [&](auto launch) {
+        return launch(w, row_bytes, n, k, m, plan, s, xs, sigma, tail, part, y, status, st);
+    };
+    const int rc = plan.blocks == 1   ? run(launch_rows_gemm<ENC, 1>)
+                   : plan.blocks == 2 ? run(launch_rows_gemm<ENC, 2>)
+                   : plan.blocks == 3 ? run(launch_rows_gemm<ENC, 3>)
+                                      : run(launch_rows_gemm<ENC, 4>);
+    if (rc)
+        return rc;
     if (plan.slices > 1) {
         const size_t count = m * n;
-        hipLaunchKernelGGL(slice_sum_kernel, dim3(unsigned((count / 4 + 255) / 256)), dim3(256),
-                           0, st, part, count, plan.slices, y);
+        hipLaunchKernelGGL(slice_sum_kernel, dim3(unsigned((count + 1023) / 1024)), dim3(256), 0,
+                           st, part, count, s.part_stride, plan.slices, y);
         KDQ_HIP(hipGetLastError());
     }
     return KDQ_OK;
@@ -798,7 +859,7 @@ extern "C" int kdq_gemm_rows(int encoding, const void* weights, size_t row_bytes
         return KDQ_ERR_ALIAS;
     int rc;
     void* scratch = workspace(
-        rows_scratch(m, n, k, row_bytes, rows_plan(m, n, k / values).slices).total, &rc);
+        rows_scratch(m, n, k, rows_plan(m, n, k / values)).total, &rc);
     if (rc)
         return rc;
     return rows_gemm(encoding, static_cast<const uint8_t*>(weights), row_bytes, n, k, x, m, y,

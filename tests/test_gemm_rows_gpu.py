@@ -50,6 +50,14 @@ def test_gemm_rows_shapes(device, oracle, enc, m, k, n):
     run(device, oracle, enc, m, k, n, seed=0xA0 + enc + m + n)
 
 
+@pytest.mark.parametrize("enc", [Q3_K, Q6_K, BF16, Q8_0])
+@pytest.mark.parametrize("m,n", [(1, 1), (31, 129), (33, 127), (65, 131), (97, 301), (161, 257)])
+def test_gemm_rows_token_tiles_and_odd_slices(device, oracle, enc, m, n):
+    """Token tiles of one to four 32-token blocks at their edges, and K slices of an odd
+    m * n (the partials' padded stride, the sum's last outputs)."""
+    run(device, oracle, enc, m, 1280, n, seed=0x1A0 + enc + m)
+
+
 def test_gemm_rows_bf16_k64(device, oracle):
     """BF16 stages 64-value groups: a k that is a multiple of 64 but not of 256."""
     run(device, oracle, BF16, 40, 192, 96, seed=0xA7)
