@@ -16,6 +16,8 @@
 //   stage_kernel<ENC>  one workgroup per token row: the row's power-of-two scale, and the
 //                      row as fp16 in the order the weight lanes consume each 256-value
 //                      group (the permutation depends on the format's packed lane image)
+//   stream_gemm_kernel<ENC, PAIR>  short chunks and grouped (MoE) layers: 64-token tiles,
+//                      the weights of two groups in flight
 //   gemm_kernel<ENC, W> 128 tokens x 256 weight rows per workgroup, W = 4 wavefronts
 //                      each owning two 32-row weight operands (W = 8: one) and all 128
 //                      tokens; weights go from HBM straight into operand registers
@@ -40,13 +42,11 @@ constexpr int kTiles = 8 * NB;               // 16-row packed tiles per workgrou
 constexpr int kStageRow = 512;               // LDS bytes per token of one staged group
 constexpr int kDmaRows = 1024 / kStageRow;   // token rows per 64-lane 16-byte DMA
 constexpr int kOutPitch = kTiles * 16 * 4 + 16;  // fp32 output row in LDS (+16: banks)
-// LDS of a workgroup with TM-token tiles: two activation stages, reused for the output
-template <int TM> constexpr size_t gemm_lds =
-    std::max(size_t(TM) * kOutPitch, 2 * size_t(TM) * kStageRow);
-constexpr size_t kLds = gemm_lds<PM>;
+constexpr int kStreamTM = int(kGroupedTileRows);  // tokens per tile of the streaming kernel
+// LDS of a workgroup: two activation stages, reused for the output
+constexpr size_t kLds = std::max(size_t(PM) * kOutPitch, 2 * size_t(PM) * kStageRow);
 
 typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) void global_void;
 
 // ------------------------------------------------------------------ formats
 //
@@ -265,14 +265,16 @@ __device__ __forceinline__ f16x8 dequant<KDQ_Q6_K>(const GemmFormat<KDQ_Q6_K>::R
     return f16x8{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
 }
 
-// Weight load i (0 .. loads - 1) of one operand's group into its registers.  `base` is
-// the operand's lane address in group 0 (tile, plus 16 * (16h + r % 16)).
+// Weight load i (0 .. loads - 1) of one operand's group into its registers, from p + the
+// item's place in the unit: `p` is the operand's lane address in the group (the tile's
+// unit, plus lane_code(r, h) bytes).
+__device__ __forceinline__ unsigned lane_code(unsigned r, unsigned h) {
+    return 16 * (16 * h + r % 16);
+}
 template <int ENC>
-__device__ __forceinline__ void load_item(const uint8_t* base, size_t off, unsigned h,
-                                          unsigned r, typename GemmFormat<ENC>::Regs& g,
-                                          int i) {
-    const uint8_t* p = base + off;
-    const unsigned lane_bytes = 16 * (16 * h + r % 16);  // already in `base`
+__device__ __forceinline__ void load_item(const uint8_t* p, unsigned h, unsigned r,
+                                          typename GemmFormat<ENC>::Regs& g, int i) {
+    const unsigned lane_bytes = lane_code(r, h);  // already in `p`
     if constexpr (ENC == KDQ_Q4_K) {
         if (i < 4)
             g.code[i / 2][i % 2] = load16(p + 1024 * (i % 2) + 512 * (i / 2));
@@ -295,6 +297,16 @@ __device__ __forceinline__ void load_item(const uint8_t* base, size_t off, unsig
     }
 }
 
+// The sub-step after which load i's registers hold nothing that the group still needs (the
+// dequantisation of sub-step s runs one sub-step before it; scales are read out first).
+template <int ENC> constexpr int free_at(int i) {
+    if (ENC == KDQ_Q4_K)
+        return i < 4 ? 4 * i + 3 : 0;
+    if (ENC == KDQ_Q8_0)
+        return i < 8 ? 2 * i + 1 : 0;
+    return i < 4 ? 4 * i + 3 : i < 6 ? 8 * (i - 4) + 7 : 0;
+}
+
 // The GEMM's scale checks over a whole packed matrix, without the product: 32 threads
 // per (16-row tile, 256-value group), lane (r = s, h) of the GEMM's operand lanes for row
 // slot s, each loading that lane's registers as the GEMM does and running the same
@@ -313,7 +325,7 @@ __global__ __launch_bounds__(256) void check_kernel(const uint8_t* __restrict__ 
     typename F::Regs g;
 #pragma unroll
     for (int i = 0; i < F::loads; ++i)
-        load_item<ENC>(base, 0, h, s, g, i);
+        load_item<ENC>(base, h, s, g, i);
     unsigned f = 0;
     Scales<ENC> sc;
     sc.prepare(g, ENC == KDQ_Q6_K ? s : h, f);
@@ -328,27 +340,23 @@ __global__ __launch_bounds__(256) void check_kernel(const uint8_t* __restrict__ 
 // (1 for an all-zero row), and fp16(x / sigma) permuted per 256-value group: logical
 // 16-byte chunk q = 16j + 8h + 4p + u of a group holds operand elements 0..7 of sub-step
 // s = 8j + 4p + u for lane half h.  One 256-thread workgroup per row; the row passes
-// through LDS.  Grouped (MoE) form: row t is x[slot_of[t] / topk] (a zero row when
-// slot_of[t] < 0) and rows from *used on are not staged.
+// through LDS.  With `slot_of` (rows are positions of a grouped layer), rows from *used on
+// and rows with slot_of[t] < 0 are not staged.
 template <int ENC>
 __global__ __launch_bounds__(256) void stage_kernel(const float* __restrict__ x, unsigned k,
                                                     uint16_t* __restrict__ xs,
                                                     float* __restrict__ sigma,
                                                     const int32_t* __restrict__ slot_of,
-                                                    unsigned topk,
                                                     const unsigned* __restrict__ used) {
     extern __shared__ __align__(16) float row[];
     __shared__ float wave_max[4];
     const unsigned t = blockIdx.x;
-    if (used && t >= *used)
+    if (slot_of && (t >= *used || slot_of[t] < 0))
         return;
-    const int slot = slot_of ? slot_of[t] : 0;
-    const bool zero = slot < 0;
-    const float* src = x + (slot_of ? size_t(zero ? 0 : slot / int(topk)) : size_t(t)) * k;
+    const float* src = x + size_t(t) * k;
     float amax = 0.f;
     for (unsigned i = threadIdx.x; i < k / 4; i += 256) {
-        const float4 v = zero ? make_float4(0.f, 0.f, 0.f, 0.f)
-                              : reinterpret_cast<const float4*>(src)[i];
+        const float4 v = reinterpret_cast<const float4*>(src)[i];
         reinterpret_cast<float4*>(row)[i] = v;
         amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
         if (!(isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w)))
@@ -390,6 +398,14 @@ __global__ __launch_bounds__(256) void stage_kernel(const float* __restrict__ x,
 
 // ------------------------------------------------------------------- GEMM
 
+// The staged rows from `xs` on, for the DMAs into LDS.  These go out as buffer loads: the
+// compiler takes a global load to LDS for a flat access, whose return order it does not
+// trust, and would wait for every load and LDS read in flight wherever it needs one.
+__device__ __forceinline__ auto activation_resource(const uint16_t* xs) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(xs), 0, int(0xffffffffu),
+                                             0x00027000);
+}
+
 // Workgroup tile: 128 tokens x 256 weight rows (16 packed tiles); wavefront w owns tiles
 // 4w .. 4w + 3 as two 32-row operands.  K runs over 256-value groups; each group's 128
 // tokens x 512 bytes of permuted activations are staged into LDS by 16-byte DMA
@@ -403,36 +419,21 @@ __global__ __launch_bounds__(256) void stage_kernel(const float* __restrict__ x,
 // runs groups [ks * per, (ks + 1) * per) and writes its fp32 tile to part[ks] (m x n);
 // reduce_kernel then sums the slices in order.
 //
-// Grouped (MoE) form, `tile_expert` given: token tile t multiplies the weights of expert
-// tile_expert[t] of a stack of packed experts `expert_bytes` apart; tiles whose entry is
-// negative are skipped (the whole workgroup returns before any barrier).
-//
-// TM = 64 (the grouped form's token tiles: experts average a few dozen rows) halves the
-// token tile: two token blocks per operand, two workgroups per compute unit (Q8_0: one;
-// at two its registers spill).
-//
-// PAIR (grouped, four wavefronts): a workgroup takes 128 output rows of two matrices
-// stored alike, `w` (gate) and `w2` (up); wavefront w's operand 0 is gate rows
-// 32w .. 32w + 31 of the tile and operand 1 the same rows of up, and the epilogue writes
-// silu(gate) * up (the reference's silu, on the scaled-back fp32 values) — one staging
-// of x and no SwiGLU pass, the same bits as the two products and the pass.
-template <int ENC, int W, int TM, bool PAIR = false>
-__global__ __launch_bounds__(W * 64, TM == PM || ENC == KDQ_Q8_0 ? 1 : 2) void gemm_kernel(
+template <int ENC, int W>
+__global__ __launch_bounds__(W * 64, 1) void gemm_kernel(
     const uint16_t* __restrict__ xs, const float* __restrict__ sigma,
     const uint8_t* __restrict__ w, unsigned m, unsigned n, unsigned k, unsigned slices,
-    unsigned per, float* __restrict__ y, float* __restrict__ part, unsigned* __restrict__ status,
-    const int32_t* __restrict__ tile_expert, size_t expert_bytes,
-    const uint8_t* __restrict__ w2 = nullptr) {
+    unsigned per, float* __restrict__ y, float* __restrict__ part,
+    unsigned* __restrict__ status) {
     using F = GemmFormat<ENC>;
     using Regs = typename F::Regs;
     extern __shared__ __align__(16) uint8_t lds[];
     // W wavefronts of NBW 32-row operands each (8 operands, 256 rows, per workgroup), TB
     // token blocks of 32
-    constexpr int NBW = 8 / W, TB = TM / 32;
+    constexpr int TM = PM, NBW = 8 / W, TB = TM / 32;
     constexpr int DMAS = TM / kDmaRows / W;  // DMA instructions per wavefront per group
     constexpr int SB = TM * kStageRow;       // bytes of one activation stage
-    static_assert(!PAIR || NBW == 2, "a pair is two operands of one wavefront");
-    constexpr int TILES = PAIR ? kTiles / 2 : kTiles;  // 16-row output tiles per workgroup
+    constexpr int TILES = kTiles;            // 16-row output tiles per workgroup
 
     const unsigned groups = k / 256, wtiles = (n + 15) / 16;
     const unsigned m_tiles = (m + TM - 1) / TM, n_tiles = (wtiles + TILES - 1) / TILES;
@@ -445,14 +446,6 @@ __global__ __launch_bounds__(W * 64, TM == PM || ENC == KDQ_Q8_0 ? 1 : 2) void g
         return;
     const unsigned n_tile = linear / (m_tiles * slices);
     const unsigned slice = (linear / m_tiles) % slices, m0 = (linear % m_tiles) * TM;
-    if (tile_expert) {
-        const int e = tile_expert[m0 / TM];
-        if (e < 0)
-            return;
-        w += size_t(e) * expert_bytes;
-        if constexpr (PAIR)
-            w2 += size_t(e) * expert_bytes;
-    }
     // slices = ceil(groups / per), so every slice has at least one group
     const unsigned g_begin = slice * per, g_end = min(groups, g_begin + per);
     float* __restrict__ dst_base = slices > 1 ? part + size_t(slice) * m * n : y;
@@ -464,16 +457,14 @@ __global__ __launch_bounds__(W * 64, TM == PM || ENC == KDQ_Q8_0 ? 1 : 2) void g
 
     // operand c = tiles tile0 + 2c (rows 0-15) and tile0 + 2c + 1 (rows 16-31); tiles
     // past the end load the last tile, and their results are never stored
-    const unsigned tile0 = n_tile * TILES + wave * 2 * (PAIR ? 1 : NBW);
+    const unsigned tile0 = n_tile * TILES + wave * 2 * NBW;
     const uint8_t* base[NBW];
 #pragma unroll
     for (int c = 0; c < NBW; ++c)
-        base[c] = (PAIR && c == 1 ? w2 : w) +
-                  size_t(min(tile0 + (PAIR ? 0 : 2 * c) + r / 16, wtiles - 1)) * groups *
-                      F::unit +
-                  16 * (16 * h + r % 16);
+        base[c] = w + size_t(min(tile0 + 2 * c + r / 16, wtiles - 1)) * groups * F::unit +
+                  lane_code(r, h);
     auto load_weight = [&](unsigned g, Regs* rg, int i) {
-        load_item<ENC>(base[i / F::loads], size_t(g) * F::unit, h, r, rg[i / F::loads],
+        load_item<ENC>(base[i / F::loads] + size_t(g) * F::unit, h, r, rg[i / F::loads],
                        i % F::loads);
     };
 
@@ -485,12 +476,12 @@ __global__ __launch_bounds__(W * 64, TM == PM || ENC == KDQ_Q8_0 ? 1 : 2) void g
         const unsigned tok = kDmaRows * jm + lane / 32;
         xlane[jm] = unsigned(tok * row_pitch) + 16 * ((lane % 32) ^ tok);
     }
-    const uint8_t* xtile = reinterpret_cast<const uint8_t*>(xs) + size_t(m0) * row_pitch;
+    const auto x_rsrc = activation_resource(xs + size_t(m0) * k);
     auto stage_one = [&](unsigned g, unsigned buf, int j) {
         const unsigned J = wave * DMAS + j;
-        __builtin_amdgcn_global_load_lds(
-            (global_void*)(xtile + size_t(g) * 512 + (J / 8) * (16 * row_pitch) + xlane[J % 8]),
-            (lds_void*)(lds + buf * SB + J * 1024), 16, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            x_rsrc, (lds_void*)(lds + buf * SB + J * 1024), 16, int(xlane[J % 8]),
+            int(g * 512 + (J / 8) * (16 * unsigned(row_pitch))), 0, 0);
     };
     constexpr int kLoads = DMAS + F::loads * NBW, kPerStep = 4;
     static_assert(kLoads <= 16 * kPerStep, "the loads must fit the group's sub-steps");
@@ -608,32 +599,17 @@ __global__ __launch_bounds__(W * 64, TM == PM || ENC == KDQ_Q8_0 ? 1 : 2) void g
         sig[b] = tok < m ? sigma[tok] : 1.f;
     }
     __syncthreads();  // every wavefront is done reading the activation stages
-    if constexpr (PAIR) {
+#pragma unroll
+    for (int c = 0; c < NBW; ++c)
 #pragma unroll
         for (int b = 0; b < TB; ++b)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const unsigned row = wave * 32 + 8 * q + 4 * h;
-                float v[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    v[i] = silu_of(acc[0][b][4 * q + i] * sig[b]) * (acc[1][b][4 * q + i] * sig[b]);
+                const unsigned row = (wave * NBW + c) * 32 + 8 * q + 4 * h;
                 *reinterpret_cast<float4*>(lds + (32 * b + r) * kOutPitch + 4 * row) =
-                    make_float4(v[0], v[1], v[2], v[3]);
+                    make_float4(acc[c][b][4 * q] * sig[b], acc[c][b][4 * q + 1] * sig[b],
+                                acc[c][b][4 * q + 2] * sig[b], acc[c][b][4 * q + 3] * sig[b]);
             }
-    } else {
-#pragma unroll
-        for (int c = 0; c < NBW; ++c)
-#pragma unroll
-            for (int b = 0; b < TB; ++b)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const unsigned row = (wave * NBW + c) * 32 + 8 * q + 4 * h;
-                    *reinterpret_cast<float4*>(lds + (32 * b + r) * kOutPitch + 4 * row) =
-                        make_float4(acc[c][b][4 * q] * sig[b], acc[c][b][4 * q + 1] * sig[b],
-                                    acc[c][b][4 * q + 2] * sig[b], acc[c][b][4 * q + 3] * sig[b]);
-                }
-    }
     __syncthreads();
     const unsigned f0 = n_tile * TILES * 16;       // first weight row of the tile
     constexpr int kChunks = TILES * 16 * 4 / 16;  // 16-byte chunks per token row
@@ -643,6 +619,318 @@ __global__ __launch_bounds__(W * 64, TM == PM || ENC == KDQ_Q8_0 ? 1 : 2) void g
             continue;
         const float4 v = *reinterpret_cast<const float4*>(lds + t * kOutPitch + 16 * ch);
         float* dst = dst_base + size_t(tok) * n + f;
+        if (f + 3 < n && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
+            *reinterpret_cast<float4*>(dst) = v;
+        } else {
+            const float vals[4] = {v.x, v.y, v.z, v.w};
+            for (unsigned j = 0; j < 4 && f + j < n; ++j)
+                dst[j] = vals[j];
+        }
+    }
+    if (status) {
+        unsigned all = flags;
+        for (int o = 32; o > 0; o >>= 1)
+            all |= __shfl_xor(all, o, 64);
+        if (lane == 0 && all)
+            atomicOr(status, all);
+    }
+}
+
+// The weight-streaming form, for few tokens per weight matrix (grouped MoE layers, short
+// chunks): 64 tokens per workgroup of four wavefronts, each with NBW 32-row weight operands
+// (stream_operands: as many as leave room for two workgroups per compute unit).  What bounds it is the wait for the weights: a
+// workgroup has few groups (8 of a 2048-value row), each multiplied in a fraction of the
+// time its bytes take to arrive.  So a group's registers are reloaded with the group
+// after the next as soon as each is read out (free_at), which keeps between one and two
+// groups per wavefront in flight in two groups' registers, and a group ends by waiting only
+// for its activation DMA, which goes out first (the counted wait below).  Past the last
+// group the loads go on, all lanes to one line: the count stays the same and nothing is read
+// twice.  (Before, the next group's loads were spread over a group and waited for at its
+// end, most of their latency showing; at 4096 slots over 128 experts, Q4_K gate / up 2048 ->
+// 768: 90 -> 68 us, the 226 MB of weights at 3.3 TB/s; Q6_K down 768 -> 2048: 72 -> 58.)
+// Only the tile's live tokens cost anything: the DMA of a dead one repeats token 0's lines,
+// and a tile of at most 32 live tokens runs one 32-token block.
+//
+// Dense form: token t of tile m0 is staged row m0 + t, K slices as in gemm_kernel.
+// Grouped (MoE) form, `tile_expert` given: token tile t multiplies the weights of expert
+// tile_expert[t] of a stack of packed experts `expert_bytes` apart; tiles whose entry is
+// negative are skipped (the whole workgroup returns before any barrier).  Position p holds
+// slot slot_of[p] (negative: dead; a tile's live positions come first), whose staged row is
+// slot / topk, or p itself when topk is 0.
+//
+// PAIR: a workgroup takes the same output rows of two matrices stored alike, `w` (gate) and
+// `w2` (up), and the epilogue writes silu(gate) * up (the reference's silu, on the
+// scaled-back fp32 values): one staging of x and no SwiGLU pass, the same bits as the two
+// products and the pass.  With two operands a wavefront holds both matrices' rows (128 per
+// workgroup); with one, wavefronts 0 and 1 hold the gate's and 2 and 3 the up's (64), which
+// meet in LDS.
+template <int ENC> constexpr int stream_operands = ENC == KDQ_Q4_K ? 2 : 1;
+constexpr int kStreamWaves = 4;
+template <int ENC, bool PAIR> constexpr int stream_tiles =
+    2 * kStreamWaves * stream_operands<ENC> / (PAIR ? 2 : 1);
+// fp32 output row of the tile in LDS (+16: banks), and a workgroup's LDS
+template <int ENC> constexpr int kStreamOutPitch =
+    kStreamWaves * stream_operands<ENC> * 32 * 4 + 16;
+template <int ENC> constexpr size_t kStreamLds =
+    std::max(size_t(kStreamTM) * kStreamOutPitch<ENC>, 2 * size_t(kStreamTM) * kStageRow);
+
+template <int ENC, bool PAIR>
+__global__ __launch_bounds__(kStreamWaves * 64, 2) void stream_gemm_kernel(
+    const uint16_t* __restrict__ xs, const float* __restrict__ sigma,
+    const uint8_t* __restrict__ w, unsigned m, unsigned n, unsigned k, unsigned slices,
+    unsigned per, float* __restrict__ y, float* __restrict__ part, unsigned* __restrict__ status,
+    const int32_t* __restrict__ tile_expert, size_t expert_bytes, const uint8_t* __restrict__ w2,
+    const int32_t* __restrict__ slot_of, unsigned topk, const unsigned* __restrict__ used) {
+    using F = GemmFormat<ENC>;
+    using Regs = typename F::Regs;
+    extern __shared__ __align__(16) uint8_t lds[];
+    constexpr int TM = kStreamTM, W = kStreamWaves, NBW = stream_operands<ENC>;
+    constexpr int SB = TM * kStageRow;  // bytes of one activation stage
+    constexpr int TILES = stream_tiles<ENC, PAIR>;  // 16-row output tiles per workgroup
+    constexpr int kOutPitch = kStreamOutPitch<ENC>;
+    constexpr int kWeightLoads = F::loads * NBW;       // per wavefront and group
+
+    const unsigned groups = k / 256, wtiles = (n + 15) / 16;
+    // (grouped: the used token tiles only, so that every XCD gets the same share of them)
+    const unsigned m_tiles = used ? max(*used / TM, 1u) : (m + TM - 1) / TM;
+    const unsigned n_tiles = (wtiles + TILES - 1) / TILES;
+    // XCD-aware order: the M tiles of one weight tile (and K slice) run together on one XCD
+    const unsigned id = blockIdx.x, xcd = id % 8, local = id / 8;
+    const unsigned per_xcd = (m_tiles * n_tiles * slices + 7) / 8;
+    const unsigned linear = xcd * per_xcd + local;
+    if (local >= per_xcd || linear >= m_tiles * n_tiles * slices)
+        return;
+    const unsigned n_tile = linear / (m_tiles * slices);
+    const unsigned slice = (linear / m_tiles) % slices, m0 = (linear % m_tiles) * TM;
+    if (tile_expert) {
+        const int e = tile_expert[m0 / TM];
+        if (e < 0)
+            return;
+        w += size_t(e) * expert_bytes;
+        if constexpr (PAIR)
+            w2 += size_t(e) * expert_bytes;
+    }
+    const unsigned g_begin = slice * per, g_end = min(groups, g_begin + per);
+    float* __restrict__ dst_base = slices > 1 ? part + size_t(slice) * m * n : y;
+
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const unsigned lane = threadIdx.x % 64;
+    const unsigned r = lane % 32, h = lane / 32;
+    const unsigned row_pitch = k * 2;
+    // live tokens of the tile (at least one), and lane t's: the staged row of token t
+    unsigned live = min(m - m0, unsigned(TM)), row_of_lane = m0 + lane;
+    if (slot_of) {
+        const int slot = slot_of[m0 + lane];
+        live = __popcll(__ballot(slot >= 0));
+        if (topk)
+            row_of_lane = unsigned(max(slot, 0)) / topk;
+    }
+    auto staged_row = [&](unsigned t) {  // by the whole wavefront; dead tokens: token 0's
+        return unsigned(__shfl(int(row_of_lane), int(t < live ? t : 0), 64));
+    };
+
+    // an operand is two packed tiles (rows 0-15, rows 16-31); tiles past the end load the
+    // last tile, and their results are never stored.  ubase: the uniform
+    // address of the first one in group 0; lane_at: the lane's bytes from there.
+    const uint8_t* ubase[NBW];
+    unsigned lane_at[NBW];
+#pragma unroll
+    for (int c = 0; c < NBW; ++c) {
+        const unsigned operand = PAIR ? (NBW == 2 ? wave : wave % (W / 2)) : wave * NBW + c;
+        const bool second = PAIR && (NBW == 2 ? c == 1 : wave >= W / 2);
+        const unsigned first = min(n_tile * TILES + 2 * operand, wtiles - 1);
+        ubase[c] = (second ? w2 : w) + size_t(first) * groups * F::unit;
+        lane_at[c] = (min(n_tile * TILES + 2 * operand + r / 16, wtiles - 1) - first) * groups *
+                         F::unit +
+                     lane_code(r, h);
+    }
+
+    const auto x_rsrc = activation_resource(xs);
+
+    unsigned flags = 0;
+    unsigned magic = 0x64006400u;  // kept in a VGPR: the mask-and-or takes one SGPR only
+    asm volatile("" : "+v"(magic));
+
+    auto run = [&]<int TB>() {
+        constexpr int DMAS = 32 * TB / kDmaRows / W;  // DMA instructions per wavefront and group
+        static_assert(DMAS <= 8, "the DMAs of a group go out in two sub-steps");
+        // instruction J = wave * DMAS + j covers tokens 2J, 2J + 1 of the tile; lane L fills
+        // LDS chunk L % 32 of token 2J + L / 32 from logical chunk (L % 32) ^ (token % 16)
+        unsigned xlane[DMAS];
+#pragma unroll
+        for (int j = 0; j < DMAS; ++j) {
+            const unsigned tok = 2 * (wave * DMAS + j) + lane / 32;
+            xlane[j] = staged_row(tok) * row_pitch +
+                       (tok < live ? 16 * ((lane % 32) ^ (tok % 16)) : 0u);
+        }
+        auto stage_x = [&](unsigned g, unsigned buf, int j0, int j1) {
+            const bool more = g < g_end;
+            const int from = more ? int(g * 512) : 0;
+#pragma unroll
+            for (int j = j0; j < j1; ++j)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    x_rsrc, (lds_void*)(lds + buf * SB + (wave * DMAS + j) * 1024), 16,
+                    more ? int(xlane[j]) : 0, from, 0, 0);
+        };
+        struct Source {
+            const uint8_t* base[NBW];
+            unsigned at[NBW];
+        };
+        auto source = [&](unsigned g) {
+            Source s;
+            const bool more = g < g_end;
+#pragma unroll
+            for (int c = 0; c < NBW; ++c) {
+                s.base[c] = ubase[c] + (more ? size_t(g) * F::unit : 0);
+                s.at[c] = more ? lane_at[c] : lane_code(r, h);
+            }
+            return s;
+        };
+        f32x16 acc[NBW][TB];
+#pragma unroll
+        for (int c = 0; c < NBW; ++c)
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+                acc[c][b] = f32x16{};
+
+        // group g from stage `buf` and registers rg: the DMAs of g + 1 into the other stage
+        // first, then rg's reloads (group g + 2)
+        auto compute = [&](unsigned g, unsigned buf, Regs* rg) {
+            const uint8_t* a = lds + buf * SB + r * kStageRow;
+            auto read_x = [&](int s, f16x8* xf) {
+                const unsigned q = 16 * (s / 8) + 8 * h + 4 * ((s / 4) % 2) + s % 4;
+#pragma unroll
+                for (int b = 0; b < TB; ++b)
+                    xf[b] = *reinterpret_cast<const f16x8*>(a + b * 32 * kStageRow +
+                                                             16 * (q ^ (r % 16)));
+            };
+            Scales<ENC> sc[NBW];
+#pragma unroll
+            for (int c = 0; c < NBW; ++c)
+                sc[c].prepare(rg[c], ENC == KDQ_Q6_K ? r : h, flags);
+            const Source next = source(g + 2);
+            f16x8 xf[2][TB], wf[2][NBW];
+            read_x(0, xf[0]);
+#pragma unroll
+            for (int c = 0; c < NBW; ++c)
+                wf[0][c] = dequant<ENC>(rg[c], sc[c], 0, magic);
+#pragma unroll
+            for (int s = 0; s < 16; ++s) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (s < 2)
+                    stage_x(g + 1, buf ^ 1u, s * (DMAS / 2), s ? DMAS : DMAS / 2);
+#pragma unroll
+                for (int c = 0; c < NBW; ++c)
+#pragma unroll
+                    for (int i = 0; i < F::loads; ++i)
+                        if (s == (free_at<ENC>(i) < 2 ? 2 : free_at<ENC>(i)))
+                            load_item<ENC>(next.base[c] + next.at[c], h, r, rg[c], i);
+                if (s + 1 < 16) {
+                    read_x(s + 1, xf[(s + 1) % 2]);
+#pragma unroll
+                    for (int c = 0; c < NBW; ++c)
+                        wf[(s + 1) % 2][c] = dequant<ENC>(rg[c], sc[c], s + 1, magic);
+                }
+#pragma unroll
+                for (int c = 0; c < NBW; ++c)
+#pragma unroll
+                    for (int b = 0; b < TB; ++b) {
+                        acc[c][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                            wf[s % 2][c], xf[s % 2][b], acc[c][b], 0, 0, 0);
+                        if constexpr (NBW == 1)  // the MFMAs stay in their sub-step (else the
+                            asm volatile("" : "+v"(acc[c][b]));  // compiler sinks them all)
+                    }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // every load but the newest group's weights has arrived (so the DMAs have), for every
+        // wavefront
+        auto arrive = [&]() {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kWeightLoads) : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        static_assert(kWeightLoads < 64, "vmcnt holds six bits");
+        Regs ra[NBW], rb[NBW];
+        auto load_all = [&](unsigned g, Regs* rg) {
+            const Source s = source(g);
+#pragma unroll
+            for (int c = 0; c < NBW; ++c)
+#pragma unroll
+                for (int i = 0; i < F::loads; ++i)
+                    load_item<ENC>(s.base[c] + s.at[c], h, r, rg[c], i);
+        };
+        stage_x(g_begin, 0, 0, DMAS);
+        __builtin_amdgcn_sched_barrier(0);
+        load_all(g_begin, ra);
+        __builtin_amdgcn_sched_barrier(0);
+        load_all(g_begin + 1, rb);
+        __builtin_amdgcn_sched_barrier(0);
+        unsigned g = g_begin;
+        for (; g + 1 < g_end; g += 2) {
+            arrive();
+            compute(g, 0, ra);
+            arrive();
+            compute(g + 1, 1, rb);
+        }
+        if (g < g_end) {  // odd group count
+            arrive();
+            compute(g, 0, ra);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no DMA outlives the workgroup
+
+        // Output tile through LDS (free after the K loop), scaled back by the token's sigma,
+        // as [token][row] fp32: D of operand c, token block b holds token 32b + r and weight
+        // rows 8(v / 4) + 4h + v % 4 of the operand's 32.
+        float sig[TB];
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+            sig[b] = sigma[staged_row(32 * b + r)];
+        __syncthreads();  // every wavefront is done reading the activation stages
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float* out = reinterpret_cast<float*>(lds + (32 * b + r) * kOutPitch);
+                if constexpr (PAIR && NBW == 2) {
+                    float v[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        v[i] = silu_of(acc[0][b][4 * q + i] * sig[b]) *
+                               (acc[1][b][4 * q + i] * sig[b]);
+                    *reinterpret_cast<float4*>(out + wave * 32 + 8 * q + 4 * h) =
+                        make_float4(v[0], v[1], v[2], v[3]);
+                } else {
+#pragma unroll
+                    for (int c = 0; c < NBW; ++c)
+                        *reinterpret_cast<float4*>(out + (wave * NBW + c) * 32 + 8 * q + 4 * h) =
+                            make_float4(acc[c][b][4 * q] * sig[b], acc[c][b][4 * q + 1] * sig[b],
+                                        acc[c][b][4 * q + 2] * sig[b],
+                                        acc[c][b][4 * q + 3] * sig[b]);
+                }
+            }
+        __syncthreads();
+    };
+    if (live <= 32)
+        run.template operator()<1>();
+    else
+        run.template operator()<2>();
+
+    const unsigned f0 = n_tile * TILES * 16;       // first weight row of the tile
+    constexpr unsigned kChunks = TILES * 16 * 4 / 16;  // 16-byte chunks per token row
+    for (unsigned e = threadIdx.x; e < live * kChunks; e += W * 64) {
+        const unsigned t = e / kChunks, ch = e % kChunks, f = f0 + 4 * ch;
+        if (f >= n)
+            continue;
+        float4 v = *reinterpret_cast<const float4*>(lds + t * kOutPitch + 16 * ch);
+        if constexpr (PAIR && NBW == 1) {
+            const float4 u =
+                *reinterpret_cast<const float4*>(lds + t * kOutPitch + 16 * (kChunks + ch));
+            v = make_float4(silu_of(v.x) * u.x, silu_of(v.y) * u.y, silu_of(v.z) * u.z,
+                            silu_of(v.w) * u.w);
+        }
+        float* dst = dst_base + size_t(m0 + t) * n + f;
         if (f + 3 < n && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
             *reinterpret_cast<float4*>(dst) = v;
         } else {
@@ -703,70 +991,90 @@ unsigned gemm_slice_depth(size_t m, size_t n, size_t k) {
 // tokens 125 -> 83 us with 8), else 4 (Q4_K and Q8_0 measured 2-4 % slower with 8).
 template <int ENC> constexpr int gemm_waves = ENC == KDQ_Q6_K ? 8 : 4;
 
-// Token tile of the grouped (MoE) form: an expert's rows are padded to whole tiles, and
-// experts average a few dozen rows in a prefill chunk, so its tiles are 64 tokens.
-constexpr int kGroupTM = int(kGroupedTileRows);
+// Dense calls of up to this many rows run on the streaming kernel, one 64-token tile: 64 x
+// 4096 -> 14336 Q8_0 31.5 us against 36.4 in a 128-token tile, 16 x 4096 -> 4096 Q6_K 15.7
+// against 20.2.  Two such tiles read the weights twice: 128 x 4096 -> 14336 Q4_K 39.6 us
+// against 38.5, 77 x 14336 -> 4096 Q6_K 47.9 against 42.0.
+constexpr size_t kStreamRows = 64;
 
 template <int ENC>
 int configure() {
     static bool configured = false;  // one attribute call per instantiation
     if (!configured) {
+        constexpr int W = gemm_waves<ENC>;
         KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&stage_kernel<ENC>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024));
-        KDQ_HIP(hipFuncSetAttribute(
-            reinterpret_cast<const void*>(&gemm_kernel<ENC, gemm_waves<ENC>, PM>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds)));
-        KDQ_HIP(hipFuncSetAttribute(
-            reinterpret_cast<const void*>(&gemm_kernel<ENC, gemm_waves<ENC>, kGroupTM>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, int(gemm_lds<kGroupTM>)));
-        if constexpr (gemm_waves<ENC> == 4)
-            KDQ_HIP(hipFuncSetAttribute(
-                reinterpret_cast<const void*>(&gemm_kernel<ENC, 4, kGroupTM, true>),
-                hipFuncAttributeMaxDynamicSharedMemorySize, int(gemm_lds<kGroupTM>)));
+        KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<ENC, W>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds)));
+        for (const void* f : {reinterpret_cast<const void*>(&stream_gemm_kernel<ENC, false>),
+                              reinterpret_cast<const void*>(&stream_gemm_kernel<ENC, true>)})
+            KDQ_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        int(kStreamLds<ENC>)));
         configured = true;
     }
     return KDQ_OK;
 }
 
-// Grouped form: x staged through the position -> slot map, then one GEMM launch over the
-// token tiles; `up` given (four-wavefront encodings): the paired launch writing
-// silu(gate x) * (up x).
+// One launch of the streaming kernel over m rows (64-token tiles); `up` given: the paired
+// form.
+template <int ENC>
+int launch_stream(const uint16_t* xs, const float* sigma, const void* packed, const void* up,
+                  size_t m, size_t n, size_t k, unsigned slices, unsigned per, float* y,
+                  float* part, unsigned* status, const int32_t* tile_expert, size_t expert_bytes,
+                  const int32_t* slot_of, unsigned topk, const unsigned* used, hipStream_t st) {
+    const size_t per_tile = up ? stream_tiles<ENC, true> : stream_tiles<ENC, false>;
+    const size_t tiles =
+        (m + kStreamTM - 1) / kStreamTM * (((n + 15) / 16 + per_tile - 1) / per_tile) * slices;
+    auto kernel = up ? stream_gemm_kernel<ENC, true> : stream_gemm_kernel<ENC, false>;
+    hipLaunchKernelGGL(kernel, dim3(unsigned((tiles + 7) / 8 * 8)), dim3(kStreamWaves * 64),
+                       kStreamLds<ENC>, st, xs, sigma, static_cast<const uint8_t*>(packed),
+                       unsigned(m), unsigned(n), unsigned(k), slices, per, y, part, status,
+                       tile_expert, expert_bytes, static_cast<const uint8_t*>(up), slot_of, topk,
+                       used);
+    KDQ_HIP(hipGetLastError());
+    return KDQ_OK;
+}
+
+// Grouped form: the rows of x staged (topk > 0: each token once; topk == 0: the live
+// positions), then one launch over the token tiles.
 template <int ENC>
 int launch_grouped(const void* packed, const void* up, size_t expert_bytes,
-                   const int32_t* tile_expert, size_t n, size_t k, const float* x,
+                   const int32_t* tile_expert, size_t n, size_t k, const float* x, size_t x_rows,
                    const int32_t* inv, unsigned topk, const unsigned* used, size_t positions,
                    float* y, unsigned* status, uint16_t* xs, float* sigma, hipStream_t st) {
     int rc;
     if ((rc = configure<ENC>()))
         return rc;
-    hipLaunchKernelGGL(stage_kernel<ENC>, dim3(unsigned(positions)), dim3(256), k * 4, st, x,
-                       unsigned(k), xs, sigma, inv, topk, used);
+    hipLaunchKernelGGL(stage_kernel<ENC>, dim3(unsigned(x_rows)), dim3(256), k * 4, st, x,
+                       unsigned(k), xs, sigma, topk ? nullptr : inv, used);
     KDQ_HIP(hipGetLastError());
-    const size_t wtiles = (n + 15) / 16;
-    const auto* w = static_cast<const uint8_t*>(packed);
-    if (up) {
-        if constexpr (gemm_waves<ENC> == 4) {
-            constexpr size_t pair_tiles = kTiles / 2;
-            const size_t tiles = (positions / kGroupTM) * ((wtiles + pair_tiles - 1) / pair_tiles);
-            hipLaunchKernelGGL((gemm_kernel<ENC, 4, kGroupTM, true>),
-                               dim3(unsigned((tiles + 7) / 8 * 8)), dim3(4 * 64),
-                               gemm_lds<kGroupTM>, st, xs, sigma, w, unsigned(positions),
-                               unsigned(n), unsigned(k), 1u, unsigned(k / 256), y, nullptr,
-                               status, tile_expert, expert_bytes,
-                               static_cast<const uint8_t*>(up));
-            KDQ_HIP(hipGetLastError());
-            return KDQ_OK;
-        }
-        return KDQ_ERR_UNSUPPORTED;
+    return launch_stream<ENC>(xs, sigma, packed, up, positions, n, k, 1u, unsigned(k / 256), y,
+                              nullptr, status, tile_expert, expert_bytes, inv, topk, used, st);
+}
+
+// How one dense call runs: on 64-token tiles of the streaming kernel or 128-token tiles, and
+// its K slices (groups per slice; the count is ceil(groups / per)).
+struct GemmPlan {
+    bool stream;
+    unsigned per, slices;
+};
+
+GemmPlan gemm_plan(int encoding, size_t m, size_t n, size_t k) {
+    GemmPlan p;
+    p.stream = m <= kStreamRows;
+    const size_t groups = k / 256;
+    if (p.stream) {
+        const size_t wt = encoding == KDQ_Q4_K ? stream_tiles<KDQ_Q4_K, false>
+                                               : stream_tiles<KDQ_Q8_0, false>;
+        const size_t tiles = (m + kStreamTM - 1) / kStreamTM * (((n + 15) / 16 + wt - 1) / wt);
+        const size_t ks = std::max<size_t>(1, 2 * compute_units() / tiles);
+        p.per = unsigned((groups + ks - 1) / ks);
+        p.per = unsigned(std::min<size_t>(groups, std::max<size_t>(p.per, 2)));
+    } else {
+        p.per = gemm_slice_depth(m, n, k);
     }
-    const size_t tiles = (positions / kGroupTM) * ((wtiles + kTiles - 1) / kTiles);
-    const unsigned grid = unsigned((tiles + 7) / 8 * 8);
-    hipLaunchKernelGGL((gemm_kernel<ENC, gemm_waves<ENC>, kGroupTM>), dim3(grid),
-                       dim3(gemm_waves<ENC> * 64), gemm_lds<kGroupTM>, st, xs, sigma, w,
-                       unsigned(positions), unsigned(n), unsigned(k), 1u, unsigned(k / 256), y,
-                       nullptr, status, tile_expert, expert_bytes, nullptr);
-    KDQ_HIP(hipGetLastError());
-    return KDQ_OK;
+    p.slices = unsigned((groups + p.per - 1) / p.per);
+    return p;
 }
 
 // Scratch of one dense GEMM call: x staged as fp16 rows padded to whole token tiles, the
@@ -775,10 +1083,9 @@ struct GemmScratch {
     size_t xs, sigma, part, total;
 };
 
-GemmScratch gemm_scratch(size_t m, size_t n, size_t k) {
+GemmScratch gemm_scratch(int encoding, size_t m, size_t n, size_t k) {
     const size_t m_pad = (m + PM - 1) / PM * PM;
-    const unsigned per = gemm_slice_depth(m, n, k);
-    const unsigned slices = unsigned((k / 256 + per - 1) / per);
+    const unsigned slices = gemm_plan(encoding, m, n, k).slices;
     GemmScratch g;
     g.xs = (m_pad * k * 2 + 255) & ~size_t(255);
     g.sigma = (m * 4 + 255) & ~size_t(255);
@@ -791,25 +1098,30 @@ template <int ENC>
 int launch_gemm(const float* x, const uint8_t* packed, size_t m, size_t n, size_t k, float* y,
                 unsigned* status, uint8_t* scratch, hipStream_t st) {
     int rc;
-    const size_t m_pad = (m + PM - 1) / PM * PM;
-    const unsigned per = gemm_slice_depth(m, n, k);
-    const unsigned slices = unsigned((k / 256 + per - 1) / per);
-    const GemmScratch g = gemm_scratch(m, n, k);
+    const GemmPlan plan = gemm_plan(ENC, m, n, k);
+    const unsigned per = plan.per, slices = plan.slices;
+    const GemmScratch g = gemm_scratch(ENC, m, n, k);
     auto* xs = reinterpret_cast<uint16_t*>(scratch);
     auto* sigma = reinterpret_cast<float*>(scratch + g.xs);
     auto* part = slices > 1 ? reinterpret_cast<float*>(scratch + g.xs + g.sigma) : nullptr;
     if ((rc = configure<ENC>()))
         return rc;
     hipLaunchKernelGGL(stage_kernel<ENC>, dim3(unsigned(m)), dim3(256), k * 4, st, x,
-                       unsigned(k), xs, sigma, nullptr, 1u, nullptr);
+                       unsigned(k), xs, sigma, nullptr, nullptr);
     KDQ_HIP(hipGetLastError());
-    const size_t wtiles = (n + 15) / 16;
-    const size_t tiles = (m_pad / PM) * ((wtiles + kTiles - 1) / kTiles) * slices;
-    const unsigned grid = unsigned((tiles + 7) / 8 * 8);
-    hipLaunchKernelGGL((gemm_kernel<ENC, gemm_waves<ENC>, PM>), dim3(grid), dim3(gemm_waves<ENC> * 64), kLds, st, xs, sigma, packed,
-                       unsigned(m), unsigned(n), unsigned(k), slices, per, y, part, status,
-                       nullptr, size_t(0));
-    KDQ_HIP(hipGetLastError());
+    if (plan.stream) {
+        if ((rc = launch_stream<ENC>(xs, sigma, packed, nullptr, m, n, k, slices, per, y, part,
+                                     status, nullptr, 0, nullptr, 0u, nullptr, st)))
+            return rc;
+    } else {
+        constexpr int W = gemm_waves<ENC>;
+        const size_t tiles = (m + PM - 1) / PM * (((n + 15) / 16 + kTiles - 1) / kTiles) * slices;
+        auto kernel = gemm_kernel<ENC, W>;
+        hipLaunchKernelGGL(kernel, dim3(unsigned((tiles + 7) / 8 * 8)), dim3(W * 64), kLds, st,
+                           xs, sigma, packed, unsigned(m), unsigned(n), unsigned(k), slices, per,
+                           y, part, status);
+        KDQ_HIP(hipGetLastError());
+    }
     if (slices > 1) {
         const size_t count = m * n;
         hipLaunchKernelGGL(reduce_kernel, dim3(unsigned((count / 4 + 256) / 256)), dim3(256), 0,
@@ -846,8 +1158,8 @@ int gemm_check(int encoding, const void* packed, size_t n, size_t k, unsigned* f
     return KDQ_OK;
 }
 
-size_t dense_gemm_scratch(size_t m, size_t n, size_t k) {
-    return gemm_scratch(m, n, k).total;
+size_t dense_gemm_scratch(int encoding, size_t m, size_t n, size_t k) {
+    return gemm_scratch(encoding, m, n, k).total;
 }
 
 int dense_gemm(int encoding, const void* packed, size_t n, size_t k, const float* x, size_t m,
@@ -869,31 +1181,25 @@ int dense_gemm(int encoding, const void* packed, size_t n, size_t k, const float
 int dense_gemm_pair(int encoding, const void* gate, const void* up, size_t n, size_t k,
                     const float* x, size_t m, float* y, unsigned* status, void* scratch,
                     hipStream_t st) {
-    if (!grouped_gemm_takes(encoding, k) || !grouped_gemm_pairs(encoding))
+    if (!grouped_gemm_takes(encoding, k))
         return KDQ_ERR_UNSUPPORTED;
     auto* sc = static_cast<uint8_t*>(scratch);
-    const GemmScratch g = gemm_scratch(m, n, k);  // covers m rounded up to 128 rows
-    auto launch = [&](auto kernel, auto stage) -> int {
+    const GemmScratch g = gemm_scratch(encoding, m, n, k);
+    auto launch = [&]<int ENC>() -> int {
         int rc;
-        if ((rc = encoding == KDQ_Q4_K ? configure<KDQ_Q4_K>() : configure<KDQ_Q8_0>()))
+        if ((rc = configure<ENC>()))
             return rc;
         auto* xs = reinterpret_cast<uint16_t*>(sc);
         auto* sigma = reinterpret_cast<float*>(sc + g.xs);
-        hipLaunchKernelGGL(stage, dim3(unsigned(m)), dim3(256), k * 4, st, x, unsigned(k), xs,
-                           sigma, nullptr, 1u, nullptr);
+        hipLaunchKernelGGL(stage_kernel<ENC>, dim3(unsigned(m)), dim3(256), k * 4, st, x,
+                           unsigned(k), xs, sigma, nullptr, nullptr);
         KDQ_HIP(hipGetLastError());
-        const size_t tiles = (m + kGroupTM - 1) / kGroupTM * (((n + 15) / 16 + 7) / 8);
-        hipLaunchKernelGGL(kernel, dim3(unsigned((tiles + 7) / 8 * 8)), dim3(4 * 64),
-                           gemm_lds<kGroupTM>, st, xs, sigma, static_cast<const uint8_t*>(gate),
-                           unsigned(m), unsigned(n), unsigned(k), 1u, unsigned(k / 256), y,
-                           nullptr, status, nullptr, size_t(0),
-                           static_cast<const uint8_t*>(up));
-        KDQ_HIP(hipGetLastError());
-        return KDQ_OK;
+        return launch_stream<ENC>(xs, sigma, gate, up, m, n, k, 1u, unsigned(k / 256), y, nullptr,
+                                  status, nullptr, 0, nullptr, 0u, nullptr, st);
     };
-    return encoding == KDQ_Q4_K
-               ? launch(gemm_kernel<KDQ_Q4_K, 4, kGroupTM, true>, stage_kernel<KDQ_Q4_K>)
-               : launch(gemm_kernel<KDQ_Q8_0, 4, kGroupTM, true>, stage_kernel<KDQ_Q8_0>);
+    return encoding == KDQ_Q4_K   ? launch.template operator()<KDQ_Q4_K>()
+           : encoding == KDQ_Q8_0 ? launch.template operator()<KDQ_Q8_0>()
+                                  : launch.template operator()<KDQ_Q6_K>();
 }
 
 bool grouped_gemm_takes(int encoding, size_t k) {
@@ -902,28 +1208,19 @@ bool grouped_gemm_takes(int encoding, size_t k) {
 }
 
 int grouped_gemm(int encoding, const void* packed, size_t expert_bytes,
-                 const int32_t* tile_expert, size_t n, size_t k, const float* x,
+                 const int32_t* tile_expert, size_t n, size_t k, const float* x, size_t x_rows,
                  const int32_t* inv, unsigned topk, const unsigned* used, size_t positions,
                  float* y, unsigned* status, uint16_t* xs, float* sigma, hipStream_t st,
                  const void* up) {
-    if (!grouped_gemm_takes(encoding, k) || positions % kGroupTM ||
-        (up && !grouped_gemm_pairs(encoding)))
+    if (!grouped_gemm_takes(encoding, k) || positions % kStreamTM)
         return KDQ_ERR_UNSUPPORTED;
-    switch (encoding) {
-    case KDQ_Q4_K:
-        return launch_grouped<KDQ_Q4_K>(packed, up, expert_bytes, tile_expert, n, k, x, inv,
-                                        topk, used, positions, y, status, xs, sigma, st);
-    case KDQ_Q8_0:
-        return launch_grouped<KDQ_Q8_0>(packed, up, expert_bytes, tile_expert, n, k, x, inv,
-                                        topk, used, positions, y, status, xs, sigma, st);
-    default:
-        return launch_grouped<KDQ_Q6_K>(packed, up, expert_bytes, tile_expert, n, k, x, inv,
-                                        topk, used, positions, y, status, xs, sigma, st);
-    }
-}
-
-bool grouped_gemm_pairs(int encoding) {
-    return encoding == KDQ_Q4_K || encoding == KDQ_Q8_0;
+    auto launch = [&](auto go) {
+        return go(packed, up, expert_bytes, tile_expert, n, k, x, x_rows, inv, topk, used,
+                  positions, y, status, xs, sigma, st);
+    };
+    return encoding == KDQ_Q4_K   ? launch(launch_grouped<KDQ_Q4_K>)
+           : encoding == KDQ_Q8_0 ? launch(launch_grouped<KDQ_Q8_0>)
+                                  : launch(launch_grouped<KDQ_Q6_K>);
 }
 
 }  // namespace kdq
@@ -946,7 +1243,7 @@ extern "C" int kdq_gemm_packed(int encoding, const void* packed, size_t n, size_
     if (overlaps(y, m * n * 4, x, m * k * 4) || overlaps(y, m * n * 4, packed, packed_bytes))
         return KDQ_ERR_ALIAS;
     int rc;
-    void* scratch = workspace(dense_gemm_scratch(m, n, k), &rc);
+    void* scratch = workspace(dense_gemm_scratch(encoding, m, n, k), &rc);
     if (rc)
         return rc;
     return dense_gemm(encoding, packed, n, k, x, m, y, status, scratch,

@@ -230,28 +230,27 @@ __device__ __forceinline__ float sigmoid_of(float v) {
 // Grouped prefill GEMM (gguf_gemm.hip): y[p, :] = W_{e(p)} x_p for positions p in token
 // tiles of kGroupedTileRows (positions a multiple of it), tile t's weights expert tile_expert[t] of a
 // stack of tile-packed experts expert_bytes apart (tiles with a negative entry skipped);
-// x_p = x[inv[p] / topk] (zero rows where inv[p] < 0), rows from *used on unstaged.
+// x_p = x[inv[p] / topk], or x[p] when topk is 0; positions with inv[p] < 0 (the last ones
+// of a tile) and those from *used on are not computed.  x has x_rows rows.
 // xs (positions * k * 2 bytes) and sigma (positions * 4) are the caller's scratch.
 // Q4_K / Q8_0 / Q6_K, k % 256 == 0, k <= 32768.
 constexpr unsigned kGroupedTileRows = 64;
 bool grouped_gemm_takes(int encoding, size_t k);
-// `up` (another stack stored alike; grouped_gemm_pairs(encoding)): one launch writing
+// `up` (another stack stored alike): one launch writing
 // y = silu(W_gate x) * (W_up x) with the reference's silu, bit-identical to the two
 // products followed by that SwiGLU.
 int grouped_gemm(int encoding, const void* packed, size_t expert_bytes,
-                 const int32_t* tile_expert, size_t n, size_t k, const float* x,
+                 const int32_t* tile_expert, size_t n, size_t k, const float* x, size_t x_rows,
                  const int32_t* inv, unsigned topk, const unsigned* used, size_t positions,
                  float* y, unsigned* status, uint16_t* xs, float* sigma, hipStream_t st,
                  const void* up = nullptr);
-bool grouped_gemm_pairs(int encoding);
 int route_selection(const float* logits, size_t tokens, size_t experts, size_t top_k,
                     int32_t* idx, float* w, hipStream_t stream);
 // Dense prefill GEMM over one tile-packed matrix (kdq_gemm_packed's product) with the
-// caller's scratch of dense_gemm_scratch(m, n, k) bytes: y[m x n] = x[m x k] W^T.
-size_t dense_gemm_scratch(size_t m, size_t n, size_t k);
+// caller's scratch of dense_gemm_scratch(encoding, m, n, k) bytes: y[m x n] = x[m x k] W^T.
+size_t dense_gemm_scratch(int encoding, size_t m, size_t n, size_t k);
 // y[m x n] = silu(x Wg^T) * (x Wu^T) for two tile-packed matrices stored alike
-// (grouped_gemm_pairs(encoding)), one launch on 64-token tiles, no K slices; the same
-// scratch as dense_gemm.
+// one launch on 64-token tiles, no K slices; the same scratch as dense_gemm.
 int dense_gemm_pair(int encoding, const void* gate, const void* up, size_t n, size_t k,
                     const float* x, size_t m, float* y, unsigned* status, void* scratch,
                     hipStream_t st);

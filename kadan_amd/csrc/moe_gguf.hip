@@ -205,6 +205,70 @@ __global__ __launch_bounds__(1024) void group_kernel(const int32_t* __restrict__
     }
 }
 
+// Router logits of a prefill batch: logits[t, e] = w_e . x_t in fp32 on
+// v_mfma_f32_16x16x4_f32, 16 tokens x 16 experts per workgroup of 8 wavefronts, which take
+// 16-value pieces of K in turn and meet in LDS, summed in wavefront order.
+// Bound by the latency of its loads: x and w come from L2, and 16-wide tiles give a
+// 512-token batch over 128 experts 256 workgroups.  Each of a wavefront's four accumulators
+// chains H / 512 steps of four products, shorter than the H / 64 of one lane of the exact
+// GEMV this replaces here (512 x 2048 x 128: 26.8 us in rows of 8 through it, 10.8 this way).
+// A non-finite weight sets bit 1 of `status`.  H % 8 == 0; x and the rows of w 16-byte
+// aligned.
+__global__ __launch_bounds__(512) void router_kernel(const float* __restrict__ x, unsigned rows,
+                                                     unsigned hidden,
+                                                     const uint8_t* __restrict__ w,
+                                                     size_t row_bytes, unsigned experts,
+                                                     float* __restrict__ logits,
+                                                     unsigned* __restrict__ status) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    constexpr unsigned kPitch = 17;
+    __shared__ float partial[8][16][kPitch];
+    const unsigned wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const unsigned r = lane % 16, quarter = lane / 16;
+    const unsigned t0 = blockIdx.y * 16, e0 = blockIdx.x * 16;
+    const auto* xr = reinterpret_cast<const f32x4*>(x + size_t(min(t0 + r, rows - 1)) * hidden);
+    const auto* wr =
+        reinterpret_cast<const f32x4*>(w + size_t(min(e0 + r, experts - 1)) * row_bytes);
+    f32x4 acc[4] = {};
+    bool finite = true;
+    const unsigned quads = hidden / 4;
+    constexpr unsigned kAhead = 4;  // pieces of 16 values (four a lane) loaded together
+    for (unsigned q0 = wave * 4; q0 < quads; q0 += 32 * kAhead) {
+        f32x4 a[kAhead], b[kAhead];
+#pragma unroll
+        for (unsigned p = 0; p < kAhead; ++p) {
+            const unsigned q = q0 + 32 * p + quarter;
+            a[p] = xr[min(q, quads - 1)];
+            b[p] = wr[min(q, quads - 1)];
+        }
+#pragma unroll
+        for (unsigned p = 0; p < kAhead; ++p) {
+            const bool in = q0 + 32 * p + quarter < quads;
+            finite = finite && isfinite(b[p].x) && isfinite(b[p].y) && isfinite(b[p].z) &&
+                     isfinite(b[p].w);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? a[p][i] : 0.f,
+                                                              in ? b[p][i] : 0.f, acc[i], 0, 0, 0);
+        }
+    }
+    const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)  // token 4 quarter + i, expert r
+        partial[wave][4 * quarter + i][r] = sum[i];
+    if (status && blockIdx.y == 0 && __any(!finite) && lane == 0)
+        atomicOr(status, 1u);
+    __syncthreads();
+    const unsigned t = threadIdx.x / 16, e = threadIdx.x % 16;
+    if (t < 16 && t0 + t < rows && e0 + e < experts) {
+        float s = partial[0][t][e];
+#pragma unroll
+        for (int v = 1; v < 8; ++v)
+            s += partial[v][t][e];
+        logits[size_t(t0 + t) * experts + e0 + e] = s;
+    }
+}
+
 // xp[p] = x[inv[p] / k] (zero for padding rows), positions below *used; 4 values a thread.
 __global__ __launch_bounds__(256) void gather_kernel(const float* __restrict__ x,
                                                      const int32_t* __restrict__ inv,
@@ -375,7 +439,10 @@ int moe_gguf(const kdq_moe_gguf_layer* layer, const kdq_moe_gguf_packed_stacks* 
     const size_t shu_bytes = sh_pack(L.up_shexp, pk.up_shexp, S, H);
     const size_t shd_bytes = sh_pack(L.down_shexp, pk.down_shexp, H, S);
     const size_t sh_scratch =
-        gemm_sh ? std::max(dense_gemm_scratch(rows, S, H), dense_gemm_scratch(rows, H, S)) : 0;
+        gemm_sh ? std::max({dense_gemm_scratch(L.gate_shexp.encoding, rows, S, H),
+                            dense_gemm_scratch(L.up_shexp.encoding, rows, S, H),
+                            dense_gemm_scratch(L.down_shexp.encoding, rows, H, S)})
+                : 0;
     const size_t sizes[] = {rows * E * 4,      rows * S * 4,      rows * S * 4,
                             size_t(0),         slots * 4,         slots * 4,
                             positions * F * 4, positions * F * 4, positions * H * 4,
@@ -498,8 +565,17 @@ int moe_gguf(const kdq_moe_gguf_layer* layer, const kdq_moe_gguf_packed_stacks* 
         if ((rc = indexed_gemv_batch(first, pair_shared ? 2 : 3, st)))
             return rc;
     } else {
-        if ((rc = run_rows(first[0], st)))
+        if (L.router.encoding == KDQ_F32 && L.router.row_bytes % 16 == 0 &&
+            !misaligned(L.router.weights, 16)) {
+            hipLaunchKernelGGL(router_kernel,
+                               dim3(unsigned((E + 15) / 16), unsigned((rows + 15) / 16)),
+                               dim3(512), 0, st, x, unsigned(rows), unsigned(H),
+                               static_cast<const uint8_t*>(L.router.weights), L.router.row_bytes,
+                               unsigned(E), logits, status);
+            KDQ_HIP(hipGetLastError());
+        } else if ((rc = run_rows(first[0], st))) {
             return rc;
+        }
         if (!gemm_sh && (rc = shared_rows()))
             return rc;
     }
@@ -531,8 +607,7 @@ int moe_gguf(const kdq_moe_gguf_layer* layer, const kdq_moe_gguf_packed_stacks* 
                  (rc = kdq_gguf_pack(L.down_shexp.encoding, L.down_shexp.weights,
                                      L.down_shexp.row_bytes, S, H, part[23], st))))
                 return rc;
-            if (same_layout(L.gate_shexp, L.up_shexp) &&
-                grouped_gemm_pairs(L.gate_shexp.encoding)) {
+            if (same_layout(L.gate_shexp, L.up_shexp)) {
                 // one paired launch writing silu(gate) * up
                 if ((rc = dense_gemm_pair(L.gate_shexp.encoding, sh_gate, sh_up, S, H, x, rows,
                                           sg, gemm_status, sh_work, st)))
@@ -588,19 +663,19 @@ int moe_gguf(const kdq_moe_gguf_layer* layer, const kdq_moe_gguf_packed_stacks* 
                  (rc = kdq_gguf_pack(L.up_exps.encoding, L.up_exps.weights, L.up_exps.row_bytes,
                                      H, E * F, packed_up, st))))
                 return rc;
-            if (same_layout(L.gate_exps, L.up_exps) &&
-                grouped_gemm_pairs(L.gate_exps.encoding)) {
+            if (same_layout(L.gate_exps, L.up_exps)) {
                 // one paired launch: x staged once, h = silu(gate) * up in its epilogue
                 if ((rc = grouped_gemm(L.gate_exps.encoding, packed_gate, gu_bytes, tile_expert,
-                                       F, H, x, inv, unsigned(K), used, positions, g,
+                                       F, H, x, rows, inv, unsigned(K), used, positions, g,
                                        gemm_status, xs, sigma, st, packed_up)))
                     return rc;
             } else {
                 if ((rc = grouped_gemm(L.gate_exps.encoding, packed_gate, gu_bytes, tile_expert,
-                                       F, H, x, inv, unsigned(K), used, positions, g,
+                                       F, H, x, rows, inv, unsigned(K), used, positions, g,
                                        gemm_status, xs, sigma, st)) ||
                     (rc = grouped_gemm(L.up_exps.encoding, packed_up, up_bytes, tile_expert, F,
-                                       H, x, inv, unsigned(K), used, positions, u, gemm_status,
+                                       H, x, rows, inv, unsigned(K), used, positions, u,
+                                       gemm_status,
                                        xs, sigma, st)))
                     return rc;
                 hipLaunchKernelGGL(swiglu_kernel, dim3(unsigned((positions * F + 255) / 256)),
@@ -617,8 +692,8 @@ int moe_gguf(const kdq_moe_gguf_layer* layer, const kdq_moe_gguf_packed_stacks* 
                  (rc = kdq_gguf_pack(L.down_exps.encoding, L.down_exps.weights,
                                      L.down_exps.row_bytes, F, E * H, packed_down, st))) ||
                 (rc = grouped_gemm(L.down_exps.encoding, packed_down, dn_bytes, tile_expert, H,
-                                   F, g, nullptr, 1u, used, positions, d, gemm_status, xs,
-                                   sigma, st)))
+                                   F, g, positions, inv, 0u, used, positions, d,
+                                   gemm_status, xs, sigma, st)))
                 return rc;
         } else if ((rc = items_down())) {
             return rc;

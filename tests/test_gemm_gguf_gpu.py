@@ -60,6 +60,16 @@ def test_gemm_small_shapes(device, oracle, enc, m, k, n):
 
 
 @pytest.mark.parametrize("enc", ENCODINGS)
+@pytest.mark.parametrize("m,k,n", [(31, 512, 144), (32, 768, 130), (33, 1024, 270),
+                                   (63, 1280, 33), (64, 256, 128), (65, 512, 257),
+                                   (5, 2816, 1000)])
+def test_gemm_short_chunks(device, oracle, enc, m, k, n):
+    """Chunks of one 64-token tile, and just past it: one or two 32-token blocks, odd and
+    even group counts, partial weight tiles, and K slices (the deeper k)."""
+    run(device, oracle, enc, m, k, n, seed=0x5E + m + n)
+
+
+@pytest.mark.parametrize("enc", ENCODINGS)
 @pytest.mark.parametrize("k,n", [(4096, 14336), (14336, 4096)])
 def test_gemm_prefill_chunk(device, oracle, enc, k, n):
     """A 512-token prefill chunk (IW/src/models/text/gguf_engine.cpp:16) at Llama-3-8B's

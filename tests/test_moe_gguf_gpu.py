@@ -101,6 +101,24 @@ def test_moe_gguf_more_rows(device, oracle, rows, top_k, encs):
     assert_close(y.cpu().numpy(), want, what=f"moe_gguf rows={rows} top_k={top_k}")
 
 
+@pytest.mark.parametrize("rows", [17, 32, 97])
+def test_moe_gguf_router_and_token_tile_edges(device, oracle, rows):
+    """An expert count that is no multiple of the router's 16-expert tile, rows past its
+    16-token tile, a hidden size whose pieces do not divide evenly over its wavefronts, and
+    experts on both sides of 32 and 64 rows; Q6_K gate and up run paired."""
+    import torch
+    H, E, K, F, S = 768, 10, 4, 256, 256
+    encs = dict(MIXED, gate_exps=Q6_K, up_exps=Q6_K, down_exps=Q8_0)
+    spec = make_layer(60 + rows, H, E, K, F, S, encs)
+    x = synth.normal(61 + rows, 1, rows * H).reshape(rows, H)
+    want, idx, w = oracle.moe_gguf_forward(spec, x)
+    from kadan_amd import ops
+    y, sel, ws = ops.moe_gguf(to_device(torch, device, spec), torch.from_numpy(x).to(device))
+    assert np.array_equal(sel.cpu().numpy(), idx)
+    assert np.abs(ws.cpu().numpy() - w).max() < 1e-6
+    assert_close(y.cpu().numpy(), want, what=f"moe_gguf rows={rows}")
+
+
 def test_moe_gguf_qwen3_shape(device, oracle):
     """Qwen3-30B-A3B's expert geometry (hidden 2048, 128 experts, top-8, expert ff 768)
     with a 768-wide shared expert, one decode token and a batch of four."""
