@@ -9,20 +9,20 @@
 // Kernels:
 //   quantize_kernel  one wavefront per 64 values: the int8 codes and scales, and the
 //                    dequantised activation fp16(code * d) that the GEMM consumes
-//   gemm_kernel      128x128 output tile per 256-thread workgroup (4 wavefronts of
-//                    64x64), k in steps of 64 staged through double-buffered LDS:
-//                    fp16 activations copied, Q4_0 weights dequantised once per tile
-//                    to fp16 ((q-8)*d rounded once, packed-fp16 arithmetic), products on
-//                    v_mfma_f32_32x32x16_f16 with fp32 accumulation; workgroups are
-//                    ordered so the four M tiles of one weight tile share an XCD (L2).
-//   packed_gemm_kernel  the same product over the tile-packed Q4_0 layout that the
-//                    decode GEMV reads (kdq_gguf_pack): 128x256 output tile per
+//   packed_gemm_kernel  the product over the tile-packed Q4_0 layout that the decode GEMV
+//                    reads (kdq_gguf_pack): up to 128 tokens x 256 weight rows per
 //                    workgroup; weights go from HBM straight into 32x32x16 MFMA operand
 //                    registers (16-byte loads of the packed lane images) and are
-//                    dequantised there; activations are staged into swizzled LDS by
-//                    global->LDS DMA in the order the weight lanes consume them, so no
-//                    LDS traffic is spent on weights.
+//                    dequantised there ((q - 8) * d rounded once); activations are staged
+//                    into swizzled LDS by buffer->LDS DMA in the order the weight lanes
+//                    consume them, so no LDS traffic is spent on weights.
+//   sum_kernel       the K slices of outputs too narrow for the compute units, summed in
+//                    slice order
+// Row-major weights are packed into the workspace first: the pass (33 MB at 4096 -> 14336)
+// costs less than multiplying them from rows did (weights through LDS, 128 x 128 tiles).
 #include "kdq_common.hpp"
+
+#include <algorithm>
 
 namespace kdq {
 namespace {
@@ -100,168 +100,6 @@ __global__ __launch_bounds__(256) void quantize_kernel(const uint16_t* __restric
         d[e / 32] = scale;
 }
 
-// ------------------------------------------------------------------- GEMM
-
-constexpr int BM = 128, BN = 128, BK = 64;
-constexpr int kPitch = BK + 8;  // fp16 per LDS row (144 bytes: conflict-free fragment reads)
-
-// 32 Q4_0 values (one block) -> 16 fp16x2 words of round((q - 8) * d).
-// `codes` are the 16 code bytes as four dwords; values j and j+16 share byte j.
-__device__ __forceinline__ void dequant_q4_0(const unsigned codes[4], unsigned d_bits,
-                                             unsigned out[16]) {
-    const f16x2 scale = __builtin_bit_cast(f16x2, d_bits | (d_bits << 16));
-    const f16x2 bias = __builtin_bit_cast(f16x2, 0x64086408u);  // (1032, 1032)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const unsigned w = codes[i];
-        // bytes (b0, b1) -> positions (0, 16) and (b2, b3) -> (0, 16)
-        const unsigned lo01 = __builtin_amdgcn_perm(0u, w, 0x0c010c00u);
-        const unsigned lo23 = __builtin_amdgcn_perm(0u, w, 0x0c030c02u);
-        const unsigned q[4] = {(lo01 & 0x000f000fu) | 0x64006400u,
-                               (lo23 & 0x000f000fu) | 0x64006400u,
-                               ((lo01 >> 4) & 0x000f000fu) | 0x64006400u,
-                               ((lo23 >> 4) & 0x000f000fu) | 0x64006400u};
-        f16x2 r[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            r[k] = (__builtin_bit_cast(f16x2, q[k]) - bias) * scale;  // exact (q-8), one rounding
-        // values: 4i, 4i+1 (lo01), 4i+2, 4i+3 (lo23), 16+4i.. (high nibbles)
-        out[2 * i] = __builtin_bit_cast(unsigned, r[0]);
-        out[2 * i + 1] = __builtin_bit_cast(unsigned, r[1]);
-        out[8 + 2 * i] = __builtin_bit_cast(unsigned, r[2]);
-        out[8 + 2 * i + 1] = __builtin_bit_cast(unsigned, r[3]);
-    }
-}
-
-struct Stage {
-    u32x4 a[4];     // 32 activation values (fp16)
-    unsigned w[5];  // 20 bytes covering one Q4_0 block
-};
-
-__global__ __launch_bounds__(256) void gemm_kernel(const uint16_t* __restrict__ a,
-                                                   const uint8_t* __restrict__ w, unsigned m,
-                                                   unsigned n, unsigned k,
-                                                   uint16_t* __restrict__ y) {
-    __shared__ __align__(16) uint16_t lds_a[2][BM * kPitch];
-    __shared__ __align__(16) uint16_t lds_b[2][BN * kPitch];
-
-    // XCD-aware tile order: the M tiles of one N tile run back to back on one XCD.
-    const unsigned m_tiles = (m + BM - 1) / BM, n_tiles = (n + BN - 1) / BN;
-    const unsigned id = blockIdx.x, xcd = id % 8, local = id / 8;
-    const unsigned per_xcd = (n_tiles * m_tiles + 7) / 8;
-    const unsigned linear = xcd * per_xcd + local;  // contiguous chunk per XCD
-    if (local >= per_xcd || linear >= n_tiles * m_tiles)
-        return;
-    const unsigned n_tile = linear / m_tiles, m_tile = linear % m_tiles;
-    const unsigned m0 = m_tile * BM, n0 = n_tile * BN;
-
-    const unsigned tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-    const size_t row_bytes = size_t(k / 32) * 18;
-
-    // global -> register staging: thread t copies activation row t/2, values
-    // 32*(t%2) .. +31 of the 64-value step, and dequantises block t%2 of weight row t/2.
-    const unsigned ar = tid / 2, ah = tid % 2;
-    const bool a_ok = m0 + ar < m, b_ok = n0 + ar < n;
-    const uint16_t* a_src = a + size_t(m0 + (a_ok ? ar : 0)) * k + 32 * ah;
-    const uint8_t* b_src = w + size_t(n0 + (b_ok ? ar : 0)) * row_bytes + (ah ? 16 : 0);
-
-    auto load = [&](unsigned step, Stage& s) {
-        const uint16_t* pa = a_src + size_t(step) * BK;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            s.a[i] = a_ok ? *reinterpret_cast<const u32x4*>(pa + 8 * i) : u32x4{0, 0, 0, 0};
-        const uint8_t* p = b_src + size_t(step) * 36;
-        if (b_ok) {
-            const u32x4 v = load16(p);
-            s.w[0] = v.x, s.w[1] = v.y, s.w[2] = v.z, s.w[3] = v.w;
-            s.w[4] = load4(p + 16);
-        } else {
-            s.w[0] = s.w[1] = s.w[2] = s.w[3] = s.w[4] = 0;
-        }
-    };
-    auto store = [&](unsigned buf, const Stage& s) {
-        uint16_t* da = lds_a[buf] + ar * kPitch + 32 * ah;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<u32x4*>(da + 8 * i) = s.a[i];
-        unsigned codes[4], d_bits;
-        if (ah == 0) {  // block at byte 0: d in bytes 0-1, codes at bytes 2..17
-            d_bits = s.w[0] & 0xffffu;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                codes[i] = __builtin_amdgcn_alignbyte(s.w[i + 1], s.w[i], 2);
-        } else {  // loaded from byte 16: d in bytes 18-19, codes at bytes 20..35
-            d_bits = s.w[0] >> 16;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                codes[i] = s.w[i + 1];
-        }
-        unsigned vals[16];
-        dequant_q4_0(codes, d_bits, vals);
-        uint16_t* db = lds_b[buf] + ar * kPitch + 32 * ah;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<u32x4*>(db + 8 * i) =
-                u32x4{vals[4 * i], vals[4 * i + 1], vals[4 * i + 2], vals[4 * i + 3]};
-    };
-
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-            acc[i][j] = f32x16{};
-
-    const unsigned wm = (wave / 2) * 64, wn = (wave % 2) * 64;
-    const unsigned frag_row = lane % 32, frag_k = 8 * (lane / 32);
-    const unsigned steps = k / BK;
-
-    Stage s;
-    load(0, s);
-    store(0, s);
-    __syncthreads();
-
-    for (unsigned step = 0; step < steps; ++step) {
-        const unsigned buf = step & 1;
-        const bool more = step + 1 < steps;
-        if (more)
-            load(step + 1, s);
-#pragma unroll
-        for (unsigned ks = 0; ks < BK; ks += 16) {
-            f16x8 af[2], bf[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                af[i] = *reinterpret_cast<const f16x8*>(
-                    lds_a[buf] + (wm + 32 * i + frag_row) * kPitch + ks + frag_k);
-                bf[i] = *reinterpret_cast<const f16x8*>(
-                    lds_b[buf] + (wn + 32 * i + frag_row) * kPitch + ks + frag_k);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
-        }
-        if (more)
-            store(buf ^ 1, s);
-        __syncthreads();
-    }
-
-    // C fragment: lane holds column lane%32, rows 8*(v/4) + 4*(lane/32) + v%4.
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const unsigned col = n0 + wn + 32 * j + lane % 32;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const unsigned row = m0 + wm + 32 * i + 8 * (v / 4) + 4 * (lane / 32) + v % 4;
-                if (row < m && col < n)
-                    y[size_t(row) * n + col] = __builtin_bit_cast(uint16_t, _Float16(acc[i][j][v]));
-            }
-        }
-}
-
 // ------------------------------------------------- GEMM over tile-packed weights
 
 // Tile-packed Q4_0 (kdq_gguf_pack): one 2304-byte unit per (16 weight rows, 256 values);
@@ -273,9 +111,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const uint16_t* __restrict__ 
 // tile r / 16, i.e. values 4u..4u+3 and 16+4u..16+4u+3 of block 4j + 2h + p.  Those
 // 16-byte loads cover whole 512-byte runs of each tile's pieces.
 constexpr int kUnitBytes = 2304;
-constexpr int PM = 128;                      // tokens per workgroup tile (4 blocks of 32)
 constexpr int kStageRow = 512;               // LDS bytes per token of one staged group
-constexpr int kStageBytes = PM * kStageRow;  // 64 KB
 constexpr int kDmaRows = 1024 / kStageRow;   // token rows per 64-lane 16-byte DMA
 
 typedef __attribute__((address_space(3))) void lds_void;
@@ -302,6 +138,9 @@ __device__ __forceinline__ f16x8 dequant_dword(unsigned w, f16x2 d, unsigned mag
     return f16x8{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
 }
 
+// fp32 output row of a sliced tile in LDS (+16: banks)
+template <int NB> constexpr int sliced_pitch = 8 * NB * 16 * 4 + 16;
+
 // One group of a 32-row weight operand in a lane's registers: code pieces [j][p] and the
 // scale dwords [j] (d of blocks 4j + 2h and 4j + 2h + 1).
 struct RowGroup {
@@ -309,33 +148,41 @@ struct RowGroup {
     unsigned scale[2];
 };
 
-// Workgroup tile: 128 tokens x 64*NB weight rows; each of the 4 wavefronts owns NB
-// 32-row weight operands and all 128 tokens, so every weight byte is loaded and
+// Workgroup tile: 32 TB tokens x 64*NB weight rows; each of the 4 wavefronts owns NB
+// 32-row weight operands and all the tokens, so every weight byte is loaded and
 // dequantised once per workgroup, straight into operand registers.  The K loop runs
-// over 256-value groups: per group the workgroup stages its 128 tokens x 512 bytes of
+// over 256-value groups: per group the workgroup stages its tokens x 512 bytes of
 // permuted activations into LDS with 16-byte DMA (double-buffered, one group ahead)
 // and each wavefront loads its operands' next group into registers.  LDS chunk q (16
 // bytes, 4 per block: q = 4 * block + u) of token t sits at t*512 + 16*(q ^ (t % 16)):
 // the 16 tokens a quarter-wavefront reads fall in 16 distinct bank groups.  `xs` has
-// rows up to the next multiple of 128 tokens (rows past m are computed, never stored).
-template <int NB>
-__global__ __launch_bounds__(256, 1) void packed_gemm_kernel(const uint16_t* __restrict__ xs,
-                                                             const uint8_t* __restrict__ w,
-                                                             unsigned m, unsigned n, unsigned k,
-                                                             uint16_t* __restrict__ y) {
+// rows up to the next whole tile (rows past m are computed, never stored).  TB = 4 runs one
+// workgroup per compute unit, smaller tiles two.
+// K slices: slice `ks` runs groups [ks * per, (ks + 1) * per) and writes its fp32 tile to
+// part + ks * part_stride, rows `pitch` apart.
+template <int NB, int TB>
+__global__ __launch_bounds__(256, TB == 4 ? 1 : 2) void packed_gemm_kernel(
+    const uint16_t* __restrict__ xs, const uint8_t* __restrict__ w, unsigned m, unsigned n,
+    unsigned k, unsigned slices, unsigned per, uint16_t* __restrict__ y,
+    float* __restrict__ part, size_t part_stride, unsigned pitch) {
     extern __shared__ __align__(16) uint8_t lds[];
-    constexpr int TILES = 8 * NB;               // 16-row weight tiles per workgroup
-    constexpr int DMAS = PM / kDmaRows / 4;     // DMA instructions per wavefront per group
+    constexpr int PM = 32 * TB;                  // tokens per workgroup
+    constexpr int kStageBytes = PM * kStageRow;  // one activation stage
+    constexpr int TILES = 8 * NB;                // 16-row weight tiles per workgroup
+    constexpr int DMAS = PM / kDmaRows / 4;      // DMA instructions per wavefront per group
 
     const unsigned groups = k / 256, wtiles = (n + 15) / 16;
     const unsigned m_tiles = (m + PM - 1) / PM, n_tiles = (wtiles + TILES - 1) / TILES;
-    // XCD-aware order: the M tiles of one weight tile run together on one XCD (L2).
+    // XCD-aware order: the M tiles of one weight tile (and K slice) run together on one XCD
     const unsigned id = blockIdx.x, xcd = id % 8, local = id / 8;
-    const unsigned per_xcd = (m_tiles * n_tiles + 7) / 8;
+    const unsigned per_xcd = (m_tiles * n_tiles * slices + 7) / 8;
     const unsigned linear = xcd * per_xcd + local;
-    if (local >= per_xcd || linear >= m_tiles * n_tiles)
+    if (local >= per_xcd || linear >= m_tiles * n_tiles * slices)
         return;
-    const unsigned n_tile = linear / m_tiles, m0 = (linear % m_tiles) * PM;
+    const unsigned n_tile = linear / (m_tiles * slices);
+    const unsigned slice = (linear / m_tiles) % slices, m0 = (linear % m_tiles) * PM;
+    // slices = ceil(groups / per), so every slice has at least one group
+    const unsigned g_begin = slice * per, g_end = min(groups, g_begin + per);
 
     const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const unsigned lane = threadIdx.x % 64;
@@ -379,12 +226,23 @@ __global__ __launch_bounds__(256, 1) void packed_gemm_kernel(const uint16_t* __r
         const unsigned tok = kDmaRows * jm + lane / 32;
         xlane[jm] = unsigned(tok * row_pitch) + 16 * ((lane % 32) ^ tok);
     }
+    // Buffer loads for the small tiles: the compiler takes a global load to LDS for a flat
+    // access, whose return order it does not trust, and waits for everything in flight
+    // wherever it needs a load or an LDS read.  The 128-token tile, whose loop waits for
+    // little else, measured 2 % faster with global loads (512 x 4096 -> 14336).
     const uint8_t* xtile = reinterpret_cast<const uint8_t*>(xs) + size_t(m0) * row_pitch;
+    const auto x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(xtile), 0,
+                                                          int(0xffffffffu), 0x00027000);
     auto stage_one = [&](unsigned g, unsigned buf, int j) {
         const unsigned J = wave * DMAS + j;
-        __builtin_amdgcn_global_load_lds(
-            (global_void*)(xtile + size_t(g) * 512 + (J / 8) * (16 * row_pitch) + xlane[J % 8]),
-            (lds_void*)(lds + buf * kStageBytes + J * 1024), 16, 0, 0);
+        auto* to = (lds_void*)(lds + buf * kStageBytes + J * 1024);
+        const size_t at = size_t(g) * 512 + (J / 8) * (16 * row_pitch);
+        if constexpr (TB == 4)
+            __builtin_amdgcn_global_load_lds((global_void*)(xtile + at + xlane[J % 8]), to, 16, 0,
+                                             0);
+        else
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, to, 16, int(xlane[J % 8]), int(at),
+                                                     0, 0);
     };
     auto stage = [&](unsigned g, unsigned buf) {
 #pragma unroll
@@ -405,11 +263,11 @@ __global__ __launch_bounds__(256, 1) void packed_gemm_kernel(const uint16_t* __r
         }
     };
 
-    f32x16 acc[NB][4];
+    f32x16 acc[NB][TB];
 #pragma unroll
     for (int c = 0; c < NB; ++c)
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+        for (int b = 0; b < TB; ++b)
             acc[c][b] = f32x16{};
 
     unsigned magic = 0x64006400u;  // kept in a VGPR: the mask-and-or takes one SGPR only
@@ -425,7 +283,7 @@ __global__ __launch_bounds__(256, 1) void packed_gemm_kernel(const uint16_t* __r
         auto read_x = [&](int s, f16x8* xf) {
             const unsigned q = 16 * (s / 8) + 8 * h + 4 * ((s / 4) % 2) + s % 4;
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
+            for (int b = 0; b < TB; ++b)
                 xf[b] = *reinterpret_cast<const f16x8*>(a + b * 32 * kStageRow +
                                                          16 * (q ^ (r % 16)));
         };
@@ -445,7 +303,7 @@ __global__ __launch_bounds__(256, 1) void packed_gemm_kernel(const uint16_t* __r
             for (int c = 0; c < NB; ++c)
                 wf[c] = dequant_dword(rg[c].code[j][p][u], d[c][j][p], magic);
         };
-        f16x8 xf[2][4], wf[2][NB];
+        f16x8 xf[2][TB], wf[2][NB];
         read_x(0, xf[0]);
         weights(0, wf[0]);
 #pragma unroll
@@ -459,14 +317,14 @@ __global__ __launch_bounds__(256, 1) void packed_gemm_kernel(const uint16_t* __r
 #pragma unroll
             for (int c = 0; c < NB; ++c)
 #pragma unroll
-                for (int b = 0; b < 4; ++b)
+                for (int b = 0; b < TB; ++b)
                     acc[c][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[s % 2][c], xf[s % 2][b],
                                                                        acc[c][b], 0, 0, 0);
 #pragma unroll
-            for (int q = 0; q < 4 * NB; ++q) {
+            for (int q = 0; q < TB * NB; ++q) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // up to four VALU
-                if (q < 4)
+                __builtin_amdgcn_sched_group_barrier(0x002, 16 / TB, 0);  // VALU
+                if (q < TB)
                     __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
                 if (q < kPerStep)
                     __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // one global load
@@ -479,11 +337,11 @@ __global__ __launch_bounds__(256, 1) void packed_gemm_kernel(const uint16_t* __r
     // reloads the last group (consumed only when the group count is odd); the
     // accumulators never change registers between paths.
     RowGroup ra[NB], rb[NB];
-    const unsigned last = groups - 1;
-    stage(0, 0);
-    load_weights(0, ra);
-    unsigned g = 0;
-    for (; g + 1 < groups; g += 2) {
+    const unsigned last = g_end - 1;
+    stage(g_begin, 0);
+    load_weights(g_begin, ra);
+    unsigned g = g_begin;
+    for (; g + 1 < g_end; g += 2) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         compute(0, ra, g + 1, 1, rb);
@@ -492,7 +350,7 @@ __global__ __launch_bounds__(256, 1) void packed_gemm_kernel(const uint16_t* __r
         compute(1, rb, min(g + 2, last), 0, ra);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no DMA outlives the workgroup
-    if (g < groups) {  // odd group count: the last group sits in buffer 0 / ra
+    if (g < g_end) {  // odd group count: the last group sits in buffer 0 / ra
         __syncthreads();
         compute(0, ra, last, 1, rb);  // its prefetch reloads the last group (never used)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -500,14 +358,37 @@ __global__ __launch_bounds__(256, 1) void packed_gemm_kernel(const uint16_t* __r
 
     // Output tile through LDS (free after the K loop): D of operand c, token block b holds
     // token 32b + r and weight rows 8(v / 4) + 4h + v % 4 of the operand's 32 in each lane;
-    // each wavefront writes its 128 x 64NB fp16 slice as [token][row] (pitch kOutPitch), then
-    // the workgroup stores whole token rows with 16-byte writes.
-    constexpr int kOutPitch = TILES * 32 + 16;  // bytes; the 16 spreads tokens over banks
+    // each wavefront writes its slice as [token][row], then the workgroup stores whole
+    // token rows with 16-byte writes.
     __syncthreads();  // every wavefront is done reading the activation stages
+    const unsigned f0 = n_tile * TILES * 16;  // first weight row of the tile
+    if (slices > 1) {                         // fp32 partials
+        constexpr int kPitch = sliced_pitch<NB>, kChunks = TILES * 16 * 4 / 16;
+#pragma unroll
+        for (int c = 0; c < NB; ++c)
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<float4*>(lds + (32 * b + r) * kPitch +
+                                               4 * ((wave * NB + c) * 32 + 8 * q + 4 * h)) =
+                        make_float4(acc[c][b][4 * q], acc[c][b][4 * q + 1], acc[c][b][4 * q + 2],
+                                    acc[c][b][4 * q + 3]);
+        __syncthreads();
+        float* out = part + slice * part_stride;
+        for (unsigned e = threadIdx.x; e < PM * kChunks; e += 256) {
+            const unsigned t = e / kChunks, ch = e % kChunks, tok = m0 + t, f = f0 + 4 * ch;
+            if (tok < m && f < n)  // (the row's padding too: pitch is n rounded up to 4)
+                *reinterpret_cast<u32x4*>(out + size_t(tok) * pitch + f) =
+                    *reinterpret_cast<const u32x4*>(lds + t * kPitch + 16 * ch);
+        }
+        return;
+    }
+    constexpr int kOutPitch = TILES * 32 + 16;  // bytes; the 16 spreads tokens over banks
 #pragma unroll
     for (int c = 0; c < NB; ++c)
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+        for (int b = 0; b < TB; ++b)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 unsigned hv[4];
@@ -519,8 +400,7 @@ __global__ __launch_bounds__(256, 1) void packed_gemm_kernel(const uint16_t* __r
                     make_uint2(hv[0] | hv[1] << 16, hv[2] | hv[3] << 16);
             }
     __syncthreads();
-    const unsigned f0 = n_tile * TILES * 16;              // first weight row of the tile
-    constexpr int kChunks = TILES * 16 * 2 / 16;          // 16-byte chunks per token row
+    constexpr int kChunks = TILES * 16 * 2 / 16;  // 16-byte chunks per token row
     for (unsigned e = threadIdx.x; e < PM * kChunks; e += 256) {
         const unsigned t = e / kChunks, ch = e % kChunks, tok = m0 + t, f = f0 + 8 * ch;
         if (tok >= m || f >= n)
@@ -537,17 +417,76 @@ __global__ __launch_bounds__(256, 1) void packed_gemm_kernel(const uint16_t* __r
     }
 }
 
-template <int NB>
-int launch_packed_gemm(const uint16_t* xs, const uint8_t* w, unsigned m, unsigned n,
-                       unsigned k, uint16_t* y, hipStream_t stream) {
+// y[t, f] = fp16 of the slices' partials summed in slice order; one thread per 4 columns.
+__global__ __launch_bounds__(256) void sum_kernel(const float* __restrict__ part, unsigned m,
+                                                  unsigned n, unsigned pitch, size_t stride,
+                                                  unsigned slices, uint16_t* __restrict__ y) {
+    const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
+    const unsigned quads = pitch / 4, t = unsigned(i / quads), f = unsigned(i % quads) * 4;
+    if (t >= m)
+        return;
+    float4 acc = reinterpret_cast<const float4*>(part)[i];
+    for (unsigned s = 1; s < slices; ++s) {
+        const float4 v = reinterpret_cast<const float4*>(part + s * stride)[i];
+        acc = make_float4(acc.x + v.x, acc.y + v.y, acc.z + v.z, acc.w + v.w);
+    }
+    const float vals[4] = {acc.x, acc.y, acc.z, acc.w};
+    uint16_t* out = y + size_t(t) * n + f;
+    for (unsigned j = 0; j < 4 && f + j < n; ++j)
+        out[j] = __builtin_bit_cast(uint16_t, _Float16(vals[j]));
+}
+
+constexpr int kOperands = 2;  // 32-row weight operands per wavefront
+
+// The token tile (TB blocks of 32), the K slices and the scratch of one call.
+struct Plan {
+    unsigned blocks, per, slices, pitch;
+    size_t rows, xs, part_stride, total;
+};
+
+// Token tile: 128 tokens (each dequantised weight multiplies four 32-token blocks) where
+// such tiles fill more than half of the compute units, else 64, two workgroups per unit; 32
+// when they hold every token.  100 x 4096 -> 14336: 44.2 us on 56 tiles of 128, 33.3 on 112
+// of 64.
+// K slices: where the output tiles are fewer than an eighth of the workgroups that fit, as
+// many slices as fit, at least two groups deep (64 x 4096 -> 14336: 43.6 -> 31.4 us;
+// 9 x 11776 -> 3387: 106 -> 21.6).  Above that line they gain less (100 x 4096 -> 14336:
+// 32.4) and would sum a row in another order than a longer chunk does.
+Plan plan_of(size_t m, size_t n, size_t k) {
+    Plan p;
+    const size_t units = compute_units(), groups = k / 256;
+    const size_t wtiles = ((n + 15) / 16 + 8 * kOperands - 1) / (8 * kOperands);
+    p.blocks = m <= 32 ? 1 : (m + 127) / 128 * wtiles * 2 > units ? 4 : 2;
+    const size_t tokens = 32 * size_t(p.blocks), tiles = (m + tokens - 1) / tokens * wtiles;
+    const size_t slots = units * (p.blocks == 4 ? 1 : 2);
+    const size_t want = tiles * 8 > slots ? 1 : slots / tiles;
+    p.per = unsigned(std::min(groups, std::max<size_t>(2, (groups + want - 1) / want)));
+    p.slices = unsigned((groups + p.per - 1) / p.per);
+    p.pitch = unsigned((n + 3) / 4 * 4);
+    p.rows = (m + tokens - 1) / tokens * tokens;
+    p.xs = (p.rows * k * 2 + 255) & ~size_t(255);
+    p.part_stride = m * p.pitch;
+    p.total = p.xs + (p.slices > 1 ? p.slices * p.part_stride * 4 : 0);
+    return p;
+}
+
+template <int TB>
+int launch_tiles(const Plan& p, const uint16_t* xs, const uint8_t* w, unsigned m, unsigned n,
+                 unsigned k, uint16_t* y, float* part, hipStream_t stream) {
     const unsigned wtiles = (n + 15) / 16;
-    const unsigned tiles = ((m + PM - 1) / PM) * ((wtiles + 8 * NB - 1) / (8 * NB));
-    const unsigned grid = (tiles + 7) / 8 * 8;
-    const size_t lds = 2 * kStageBytes;
-    KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&packed_gemm_kernel<NB>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    hipLaunchKernelGGL((packed_gemm_kernel<NB>), dim3(grid), dim3(256), lds, stream, xs, w, m, n,
-                       k, y);
+    const unsigned tiles =
+        unsigned(p.rows / (32 * TB)) * ((wtiles + 8 * kOperands - 1) / (8 * kOperands)) * p.slices;
+    constexpr size_t lds = std::max(size_t(2) * 32 * TB * kStageRow,
+                                    size_t(32) * TB * sliced_pitch<kOperands>);
+    auto kernel = packed_gemm_kernel<kOperands, TB>;
+    static bool configured = false;  // one attribute call per instantiation
+    if (!configured) {
+        KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+        configured = true;
+    }
+    hipLaunchKernelGGL(kernel, dim3((tiles + 7) / 8 * 8), dim3(256), lds, stream, xs, w, m, n, k,
+                       p.slices, p.per, y, part, p.part_stride, p.pitch);
     KDQ_HIP(hipGetLastError());
     return KDQ_OK;
 }
@@ -558,6 +497,29 @@ int launch_quantize(const uint16_t* x, size_t m, size_t k, int8_t* q, float* d,
     const size_t threads = m * k / 8;
     hipLaunchKernelGGL(quantize_kernel<PERMUTED>, dim3(unsigned((threads + 255) / 256)),
                        dim3(256), 0, stream, x, m * k, q, d, dequant);
+    KDQ_HIP(hipGetLastError());
+    return KDQ_OK;
+}
+
+// The product over tile-packed weights: permuted activations (rows padded to whole tiles,
+// the padding never stored), the tiles, and the slices' sum.
+int run_packed(const Plan& p, const uint16_t* x, const uint8_t* packed, size_t m, size_t n,
+               size_t k, uint16_t* y, uint8_t* scratch, hipStream_t st) {
+    auto* xs = reinterpret_cast<uint16_t*>(scratch);
+    auto* part = reinterpret_cast<float*>(scratch + p.xs);
+    int rc = launch_quantize<true>(x, m, k, nullptr, nullptr, xs, st);
+    if (rc)
+        return rc;
+    auto run = [&](auto launch) {
+        return launch(p, xs, packed, unsigned(m), unsigned(n), unsigned(k), y, part, st);
+    };
+    rc = p.blocks == 1   ? run(launch_tiles<1>)
+         : p.blocks == 2 ? run(launch_tiles<2>)
+                         : run(launch_tiles<4>);
+    if (rc || p.slices == 1)
+        return rc;
+    hipLaunchKernelGGL(sum_kernel, dim3(unsigned((p.part_stride / 4 + 255) / 256)), dim3(256), 0,
+                       st, part, unsigned(m), unsigned(n), p.pitch, p.part_stride, p.slices, y);
     KDQ_HIP(hipGetLastError());
     return KDQ_OK;
 }
@@ -589,26 +551,17 @@ extern "C" int kdq_gemm_q4_0(const void* weights, size_t n, size_t k, const uint
     if (overlaps(y_f16, m * n * 2, x_f16, m * k * 2) ||
         overlaps(y_f16, m * n * 2, weights, n * (k / 32) * 18))
         return KDQ_ERR_ALIAS;
-    // workspace: int8 codes, fp32 scales, fp16 dequantised activations
     int rc;
-    const size_t codes = (m * k + 255) & ~size_t(255), scales = (m * k / 32 * 4 + 255) & ~size_t(255);
-    auto* base = static_cast<uint8_t*>(workspace(codes + scales + m * k * 2, &rc));
+    const Plan p = plan_of(m, n, k);
+    const size_t packed_bytes = kdq_gguf_packed_bytes(KDQ_Q4_0, k, n);
+    const size_t at = (p.total + 255) & ~size_t(255);
+    auto* base = static_cast<uint8_t*>(workspace(at + packed_bytes, &rc));
     if (rc)
         return rc;
-    auto st = static_cast<hipStream_t>(stream);
-    rc = launch_quantize(x_f16, m, k, reinterpret_cast<int8_t*>(base),
-                         reinterpret_cast<float*>(base + codes),
-                         reinterpret_cast<uint16_t*>(base + codes + scales), st);
-    if (rc)
+    uint8_t* packed = base + at;
+    if ((rc = kdq_gguf_pack(KDQ_Q4_0, weights, (k / 32) * 18, k, n, packed, stream)))
         return rc;
-    const unsigned tiles = unsigned(((m + BM - 1) / BM) * ((n + BN - 1) / BN));
-    const unsigned grid = (tiles + 7) / 8 * 8;
-    hipLaunchKernelGGL(gemm_kernel, dim3(grid), dim3(256), 0, st,
-                       reinterpret_cast<const uint16_t*>(base + codes + scales),
-                       static_cast<const uint8_t*>(weights), unsigned(m), unsigned(n),
-                       unsigned(k), y_f16);
-    KDQ_HIP(hipGetLastError());
-    return KDQ_OK;
+    return run_packed(p, x_f16, packed, m, n, k, y_f16, base, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int kdq_gemm_q4_0_packed(const void* packed, size_t n, size_t k, const uint16_t* x_f16,
@@ -624,16 +577,11 @@ extern "C" int kdq_gemm_q4_0_packed(const void* packed, size_t n, size_t k, cons
     if (overlaps(y_f16, m * n * 2, x_f16, m * k * 2) ||
         overlaps(y_f16, m * n * 2, packed, packed_bytes))
         return KDQ_ERR_ALIAS;
-    // permuted activations, rows padded to the 128-token tile (padding never stored)
     int rc;
-    const size_t m_pad = (m + PM - 1) / PM * PM;
-    auto* xs = static_cast<uint16_t*>(workspace(m_pad * k * 2, &rc));
+    const Plan p = plan_of(m, n, k);
+    auto* scratch = static_cast<uint8_t*>(workspace(p.total, &rc));
     if (rc)
         return rc;
-    auto st = static_cast<hipStream_t>(stream);
-    rc = launch_quantize<true>(x_f16, m, k, nullptr, nullptr, xs, st);
-    if (rc)
-        return rc;
-    return launch_packed_gemm<2>(xs, static_cast<const uint8_t*>(packed), unsigned(m),
-                                 unsigned(n), unsigned(k), y_f16, st);
+    return run_packed(p, x_f16, static_cast<const uint8_t*>(packed), m, n, k, y_f16, scratch,
+                      static_cast<hipStream_t>(stream));
 }

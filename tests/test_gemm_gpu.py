@@ -41,6 +41,9 @@ def test_quantize_bit_exact(device, oracle, m, k):
 
 SHAPES = [(1, 256, 1), (5, 256, 130), (128, 512, 128), (130, 1024, 300), (33, 4096, 256),
           (256, 4096, 1024), (512, 4096, 640)]
+# token tiles of 32, 64 and 128 at their edges, K slices (odd m * n, partial weight tiles)
+SHAPES += [(2, 2560, 770), (31, 1280, 33), (32, 2304, 512), (63, 1536, 257), (65, 5632, 131),
+           (129, 2048, 1001)]
 
 
 @pytest.mark.parametrize("m,k,n", SHAPES)
