@@ -721,7 +721,14 @@ __global__ __launch_bounds__(1024) void prologue_kernel(
 }
 
 // ------------------------------------------------------------- grouped GEMMs
-//
+
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        (f.template operator()<I>(), ...);
+    }(std::make_integer_sequence<int, N>{});
+}
+
 // A workgroup of kGemmWaves wavefronts takes one work item (expert e, up to kItemRows
 // consecutive rows of its segment: one or two activation tiles of 32 rows) and one K
 // slice; every wavefront owns two 32-row weight groups (gate and up of the same 32
@@ -745,8 +752,8 @@ __device__ __forceinline__ v8i32 b_operand(const u32x4& c) {
     return __builtin_shufflevector(v, v, 0, 1, 2, 3, -1, -1, -1, -1);
 }
 
-// One wavefront's two packed weight groups (codes at + step * 1 KB, scales at + group * 64
-// dwords, both already offset by the lane).
+// One wavefront's two packed weight groups: codes at + step * 1 KB, the lane's scales at +
+// group * 64 dwords.
 struct WavePair {
     const uint8_t* codes[2];
     const unsigned* scales[2];
@@ -758,7 +765,7 @@ __device__ __forceinline__ WavePair wave_pair(const uint8_t* packed, const Packe
     const size_t g[2] = {group0, group1};
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
-        w.codes[m] = packed + g[m] * shape.steps * 1024 + lane * 16;
+        w.codes[m] = packed + g[m] * shape.steps * 1024;
         w.scales[m] = reinterpret_cast<const unsigned*>(packed + shape.code_bytes +
                                                         g[m] * shape.scale_groups * 256) +
                       lane;
@@ -766,10 +773,22 @@ __device__ __forceinline__ WavePair wave_pair(const uint8_t* packed, const Packe
     return w;
 }
 
-// K slice `slice` of `slices`: [begin, end) in steps, begin a multiple of 8.
+// Steps per turn of the products' loop (staged_pair).
+constexpr unsigned kTurnSteps = 12;
+
+// Steps of a K slice when `steps` are cut into about `slices`: whole turns of the products'
+// loop, unless that leaves the last slice less than half a slice; then whole sets of scales.
+__host__ __device__ inline unsigned steps_per_slice(unsigned steps, unsigned slices) {
+    const unsigned even = (steps + slices - 1) / slices;
+    const unsigned turns = (even + kTurnSteps - 1) / kTurnSteps * kTurnSteps;
+    const unsigned last = steps - (steps - 1) / turns * turns;
+    return turns == kTurnSteps || last * 2 >= turns ? turns : (even + 3) / 4 * 4;
+}
+
+// K slice `slice` of `slices`: [begin, end) in steps, begin a multiple of 4.
 __device__ __forceinline__ void slice_steps(unsigned steps, unsigned slices, unsigned slice,
                                             unsigned& begin, unsigned& end) {
-    const unsigned per = ((steps + slices - 1) / slices + 7) / 8 * 8;
+    const unsigned per = steps_per_slice(steps, slices);
     begin = min(steps, slice * per);
     end = min(steps, begin + per);
 }
@@ -781,151 +800,169 @@ __device__ __forceinline__ void issue_order() {
 
 // The item's activation tiles pass through LDS: per chunk of kChunk steps the workgroup
 // copies the chunk of every tile it multiplies (contiguous in the tile layout: kChunk *
-// TERMS * 2 KB per tile) into one of two LDS buffers, 16 bytes per thread per piece, and
+// TERMS * 2 KB per tile) into one of kStages LDS buffers by DMA, 1 KB per instruction, and
 // every wavefront reads its MFMA A operands from there at lane * 16 (conflict free): one
-// activation load per thread and piece instead of one per wavefront.  A chunk is loaded
-// while the one before it is multiplied and stored behind it, with one workgroup barrier
-// per chunk; weights stream per wavefront BRING - 1 steps ahead.  (Measured at T = 256,
-// 32 experts: activations loaded by every wavefront from L2 kept the address unit 60 %
-// busy and the MFMAs 18 %; staging two chunks ahead or weights seven steps ahead were
-// slower; so was a register cap for three workgroups per compute unit, which spills.)
-constexpr int kChunk = 2;
+// activation load per workgroup instead of one per wavefront.
+// A wavefront's loads return in the order they were issued, so waiting for a chunk waits for
+// every weight load before it.  Chunks therefore go out two ahead (three buffers) and
+// weights four steps ahead, a chunk's registers reloaded as its products are issued: at
+// the wait for a chunk the weights of the last two chunks may still be in flight (the count
+// in `arrive`).  With the chunk loaded into registers one ahead, all but one chunk's weights
+// had to be there.  The DMAs are buffer loads: the compiler takes a global load to LDS for a
+// flat access, whose return order it does not trust, and waits for everything wherever it
+// needs a load (so written, this pipeline measured slower than the one it replaces).
+constexpr int kChunk = 2, kStages = 3, kAheadSteps = 4;
 
-template <int TERMS, int TILES, int WAVES = kGemmWaves> struct StageCopy {
-    static constexpr int chunk_bytes = TILES * kChunk * TERMS * 2048;  // one LDS buffer
-    static constexpr int threads = WAVES * 64;
-    // per thread; when the chunk's 16-byte pieces are not a multiple of the threads, the
-    // last piece of the threads past the end is clamped on load and not stored
-    static constexpr int pieces = (chunk_bytes / 16 + threads - 1) / threads;
-    static constexpr bool ragged = chunk_bytes / 16 % threads != 0;
-    const uint8_t* src[pieces];  // piece j of this thread at step 0 (tile base + offset)
-    unsigned step[pieces];       // step of the piece within the chunk
-};
+template <int TERMS, int TILES> constexpr int chunk_bytes = TILES * kChunk * TERMS * 2048;
 
-template <int TERMS, int TILES, int WAVES>
-__device__ __forceinline__ StageCopy<TERMS, TILES, WAVES> stage_copy(const Tiles& l,
-                                                                     unsigned item) {
-    using C = StageCopy<TERMS, TILES, WAVES>;
-    C c;
-    constexpr int per_tile = kChunk * TERMS * 2048;
-#pragma unroll
-    for (int j = 0; j < C::pieces; ++j) {
-        const unsigned o = min(unsigned(threadIdx.x + j * WAVES * 64) * 16,
-                               unsigned(C::chunk_bytes - 16));  // byte in the chunk
-        const unsigned t = o / per_tile, within = o % per_tile;
-        c.step[j] = within / (TERMS * 2048);
-        c.src[j] = l.codes + (2 * size_t(item) + t) * l.code_stride + within % (TERMS * 2048);
-    }
-    return c;
-}
-
-
-// acc[m][t] += A(tile t, steps [q0, q1)) * B(group m), q0 % 8 == 0; A through LDS, weights
-// BRING - 1 steps ahead (BRING = 4 or 8 steps: whole scale groups and LDS buffer pairs),
-// with the non-temporal policy when NT (weights read once per layer call).
-template <int TERMS, int TILES, bool NT, int BRING = 4, int WAVES = kGemmWaves>
-__device__ __forceinline__ void staged_pair(const Tiles& l, unsigned item, unsigned lane,
-                                            const WavePair& w, unsigned q0, unsigned q1,
-                                            bool active, uint8_t* stage,
+// acc[m][t] += A(tile t, steps [q0, q1)) * B(group m), q0 % 4 == 0; weights with the
+// non-temporal policy when NT (weights read once per layer call).  Ends with no DMA in
+// flight and `stage` free.
+template <int TERMS, int TILES, bool NT, int WAVES>
+__device__ __forceinline__ void staged_pair(const Tiles& l, unsigned item, unsigned wave,
+                                            unsigned lane, const WavePair& w, unsigned q0,
+                                            unsigned q1, bool active,
+                                            uint8_t* const (&stage)[kStages],
                                             f32x16 (&acc)[2][TILES]) {
-    using C = StageCopy<TERMS, TILES, WAVES>;
-    const C cp = stage_copy<TERMS, TILES, WAVES>(l, item);
+    constexpr int kBytes = chunk_bytes<TERMS, TILES>, kPieces = kBytes / 1024;
+    constexpr int kDmas = (kPieces + WAVES - 1) / WAVES;  // per wavefront and chunk
+    constexpr int kPerTile = kChunk * TERMS * 2;          // pieces of one tile
+    // (rsrc: raw buffer over the item's tiles)
+    const auto x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        l.codes + 2 * size_t(item) * l.code_stride, 0, int(0xffffffffu), 0x00027000);
+    auto stage_x = [&](unsigned qc, uint8_t* to) {  // chunk of steps qc .. into `to`
+#pragma unroll
+        for (int j = 0; j < kDmas; ++j) {
+            // (where the last round has fewer pieces than wavefronts, the others repeat them:
+            // the same bytes to the same place)
+            constexpr int kLast = kPieces - (kDmas - 1) * WAVES;
+            static_assert((kLast & (kLast - 1)) == 0, "a power of two");
+            const unsigned piece = j * WAVES + (j + 1 < kDmas ? wave : wave & (kLast - 1));
+            const unsigned t = piece / kPerTile, within = piece % kPerTile;
+            const unsigned q = min(qc + within / (TERMS * 2), q1 - 1);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                x_rsrc, (__attribute__((address_space(3))) void*)(to + piece * 1024), 16,
+                int(lane * 16),
+                int(t * unsigned(l.code_stride) + q * (TERMS * 2048) +
+                    within % (TERMS * 2) * 1024),
+                0, 0);
+        }
+        issue_order();
+    };
     const unsigned* ascale[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t)
         ascale[t] = reinterpret_cast<const unsigned*>(l.scales + (2 * size_t(item) + t) * l.scale_stride) +
                     lane;
-    struct BSlot {
-        u32x4 c[2];
-        unsigned s[2];
-        unsigned as[TILES];
+    struct Scales {  // of four steps
+        unsigned w[2], a[TILES];
     };
-    auto load_b = [&](unsigned q, BSlot& B) {
-        q = min(q, q1 - 1);
+    auto load_scales = [&](unsigned q, Scales& s) {
+        const size_t at = size_t(min(q, q1 - 1) / 4) * 64;
 #pragma unroll
         for (int m = 0; m < 2; ++m)
-            B.c[m] = NT ? stream16(w.codes[m] + size_t(q) * 1024)
-                        : load16(w.codes[m] + size_t(q) * 1024);
-#pragma unroll
-        for (int m = 0; m < 2; ++m)
-            B.s[m] = w.scales[m][size_t(q / 4) * 64];
+            s.w[m] = w.scales[m][at];
 #pragma unroll
         for (int t = 0; t < TILES; ++t)
-            B.as[t] = ascale[t][size_t(q / 4) * 64];
+            s.a[t] = ascale[t][at];
+        issue_order();
     };
-    struct Pieces {
-        u32x4 v[C::pieces];
-    };
-    auto stage_load = [&](unsigned qc, Pieces& P) {  // chunk starting at step qc
+    // the wavefront's codes as buffers that end with step q1 (empty for an inactive one): loads
+    // past the end return zeros, so those products add nothing
+    const int code_bytes = active ? int(q1 * 1024) : 0;
+    const __amdgpu_buffer_rsrc_t code_rsrc[2] = {
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w.codes[0]), 0, code_bytes,
+                                          0x00027000),
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w.codes[1]), 0, code_bytes,
+                                          0x00027000)};
+    auto load_codes = [&](unsigned q, u32x4 (&c)[2]) {
+        typedef unsigned u4 __attribute__((ext_vector_type(4)));
 #pragma unroll
-        for (int j = 0; j < C::pieces; ++j)
-            P.v[j] = load16(cp.src[j] + size_t(min(qc + cp.step[j], q1 - 1)) * TERMS * 2048);
-    };
-    auto stage_store = [&](const Pieces& P, int buffer) {
-#pragma unroll
-        for (int j = 0; j < C::pieces; ++j) {
-            const unsigned o = (threadIdx.x + j * WAVES * 64) * 16;
-            if (!C::ragged || j + 1 < C::pieces || o < unsigned(C::chunk_bytes))
-                *reinterpret_cast<u32x4*>(stage + buffer * C::chunk_bytes + o) = P.v[j];
+        for (int m = 0; m < 2; ++m) {
+            const u4 v = __builtin_amdgcn_raw_buffer_load_b128(
+                code_rsrc[m], int(q * 1024 + lane * 16), 0, NT ? 2 : 0);
+            c[m] = u32x4{v.x, v.y, v.z, v.w};
         }
+        issue_order();
+    };
+    // The chunk that the next products read has arrived, for every wavefront: behind its DMAs
+    // at least the loads of two chunks (four steps' codes, one set of scales) and the DMAs of
+    // the chunk after were issued.
+    constexpr int kBehind = 2 * kAheadSteps + 2 + TILES + kDmas;
+    static_assert(kBehind < 64, "vmcnt holds six bits");
+    auto arrive = [&]() {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kBehind) : "memory");
+        __builtin_amdgcn_s_barrier();
+        issue_order();
     };
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
         for (int t = 0; t < TILES; ++t)
             acc[m][t] = f32x16{};
-    BSlot bs[BRING];
-    Pieces xr;
-    stage_load(q0, xr);
+    u32x4 codes[kAheadSteps][2];
+    Scales scales[3];
     issue_order();
+    stage_x(q0, stage[0]);
+    stage_x(q0 + kChunk, stage[1]);
+    load_scales(q0, scales[0]);
 #pragma unroll
-    for (int d = 0; d + 1 < BRING; ++d)
-        load_b(q0 + d, bs[d]);
-    issue_order();
-    stage_store(xr, 0);
-    __syncthreads();
-    // one chunk (kChunk = 2 steps) per call; CI = chunk index within the BRING-step period
-    auto chunk = [&]<int CI>(unsigned qc) {
-        constexpr int C2 = CI % 2;  // LDS buffer
-        stage_load(qc + kChunk, xr);
-        issue_order();
-        auto step = [&]<int S>() {
-            constexpr int U = CI * kChunk + S;  // step within the period
-            const unsigned q = qc + S;
-            load_b(q + BRING - 1, bs[(U + BRING - 1) % BRING]);
-            if (active && q < q1) {
-                const BSlot& B = bs[U];
-                const uint8_t* buf = stage + C2 * C::chunk_bytes + 16 * lane;
+    for (int d = 0; d < kAheadSteps; ++d)
+        load_codes(q0 + d, codes[d]);
+    // Twelve steps per turn (six chunks: whole rounds of the buffers, the code registers and
+    // three sets of scales), every load issued whether or not its step exists: a branch
+    // around them would let the compiler move them away from where `arrive` counts them.
+    // Chunks past q1 multiply nothing; within a chunk the A operands are read two ahead of
+    // their products.
+    for (unsigned qt = q0; qt < q1; qt += kTurnSteps) {
+        static_for<kTurnSteps / kChunk>([&]<int C>() {
+            constexpr int kOperands = kChunk * TILES * TERMS, kReadAhead = 2;
+            const unsigned qc = qt + C * kChunk;
+            arrive();
+            // two chunks ahead, into the buffer that the previous chunk's products have left
+            stage_x(qc + 2 * kChunk, stage[(C + 2) % kStages]);
+            if constexpr (C % 2 == 0)
+                load_scales(qc + 4, scales[(C / 2 + 1) % 3]);
+            if (qc < q1) {
+                v8i32 av[kReadAhead + 1];
+                auto read = [&](int i) {  // operand i: step S, tile t, term k
+                    const int S = i / (TILES * TERMS), t = i / TERMS % TILES, k = i % TERMS;
+                    const uint8_t* p =
+                        stage[C % kStages] + 16 * lane + ((t * kChunk + S) * TERMS + k) * 2048;
+                    av[i % (kReadAhead + 1)] =
+                        a_operand(*reinterpret_cast<const u32x4*>(p),
+                                  *reinterpret_cast<const u32x4*>(p + 1024));
+                };
 #pragma unroll
-                for (int t = 0; t < TILES; ++t)
+                for (int i = 0; i < kReadAhead; ++i)
+                    read(i);
+                static_for<kOperands>([&]<int I>() {
+                    constexpr int S = I / (TILES * TERMS), t = I / TERMS % TILES,
+                                  U = C * kChunk + S;
+                    const Scales& sc = scales[U / 4];
+                    // (past q1 the activations' scale bytes may never have been written: 1,
+                    // so that the zero codes' products are zero)
+                    const unsigned as = S == 0 || qc + S < q1 ? sc.a[t] : 0x7f7f7f7fu;
+                    if constexpr (I + kReadAhead < kOperands)
+                        read(I + kReadAhead);
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int k = 0; k < TERMS; ++k) {
-                        const uint8_t* p = buf + ((t * kChunk + S) * TERMS + k) * 2048;
-                        const v8i32 av = a_operand(*reinterpret_cast<const u32x4*>(p),
-                                                   *reinterpret_cast<const u32x4*>(p + 1024));
-#pragma unroll
-                        for (int m = 0; m < 2; ++m)
-                            acc[m][t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                                av, b_operand(B.c[m]), acc[m][t], 0 /* A: fp8 e4m3 */,
-                                4 /* B: fp4 e2m1 */, U % 4, int(B.as[t]), U % 4, int(B.s[m]));
-                    }
+                    for (int m = 0; m < 2; ++m)
+                        acc[m][t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                            av[I % (kReadAhead + 1)], b_operand(codes[U % kAheadSteps][m]),
+                            acc[m][t], 0 /* A: fp8 e4m3 */, 4 /* B: fp4 e2m1 */, U % 4, int(as),
+                            U % 4, int(sc.w[m]));
+                    __builtin_amdgcn_sched_barrier(0);
+                });
             }
-        };
-        step.template operator()<0>();
-        step.template operator()<1>();
-        stage_store(xr, (C2 + 1) % 2);  // also past the end (never read)
-        __syncthreads();
-    };
-    const unsigned periods = (q1 - q0 + BRING - 1) / BRING;
-    for (unsigned p = 0; p < periods; ++p) {
-        const unsigned qc = q0 + p * BRING;
-        chunk.template operator()<0>(qc);
-        chunk.template operator()<1>(qc + kChunk);
-        if constexpr (BRING == 8) {
-            chunk.template operator()<2>(qc + 2 * kChunk);
-            chunk.template operator()<3>(qc + 3 * kChunk);
-        }
+            issue_order();
+#pragma unroll
+            for (int S = 0; S < kChunk; ++S)
+                load_codes(qc + S + kAheadSteps, codes[(C * kChunk + S) % kAheadSteps]);
+        });
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no DMA outlives the call
+    __syncthreads();
 }
 
 // Output row of accumulator element v in lane half h of tile t (32x32 MFMA layout).
@@ -1050,12 +1087,15 @@ __global__ __launch_bounds__(kGemmWaves * 64, 3) void gate_up_kernel(
     const int32_t* __restrict__ item_count, uint8_t* __restrict__ ha,
     float* __restrict__ part_g, float* __restrict__ part_u, size_t part_stride,
     unsigned cols) {
-    __shared__ __align__(16) uint8_t stage[2 * StageCopy<kXTerms, 2>::chunk_bytes];
+    __shared__ __align__(16) uint8_t stage0[chunk_bytes<kXTerms, 2>],
+        stage1[chunk_bytes<kXTerms, 2>], stage2[chunk_bytes<kXTerms, 2>];
+    uint8_t* const stage[kStages] = {stage0, stage1, stage2};
     const ItemCell cell = item_cell(cols);
     if (int(cell.item) >= *item_count)
         return;
     const Item it = load_item(items, offsets, cell.item);
-    const unsigned wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64),
+                   lane = threadIdx.x % 64;
     const unsigned i32 = lane % 32, h = lane / 32;
     const Packed shape = packed_shape(1, inter, hidden);  // per expert
     const unsigned fg = cell.col * kGemmWaves + wave;     // feature group of 32
@@ -1076,7 +1116,8 @@ __global__ __launch_bounds__(kGemmWaves * 64, 3) void gate_up_kernel(
 
     auto run = [&]<int TILES>() {
         f32x16 acc[2][TILES];
-        staged_pair<kXTerms, TILES, NT>(xl, cell.item, lane, wp, q0, q1, active, stage, acc);
+        staged_pair<kXTerms, TILES, NT, kGemmWaves>(xl, cell.item, wave, lane, wp, q0, q1, active,
+                                                    stage, acc);
         if (!active)
             return;
         if (gridDim.z > 1) {
@@ -1096,7 +1137,7 @@ __global__ __launch_bounds__(kGemmWaves * 64, 3) void gate_up_kernel(
         }
         // the LDS stage is free once staged_pair has returned (it ends on a barrier
         // after the last MFMA read); each wavefront takes its own 1 KB of it
-        store_h_tiles<TILES>(acc, fg, lane, cell.item, hl, stage + wave * 1024);
+        store_h_tiles<TILES>(acc, fg, lane, cell.item, hl, stage0 + wave * 1024);
     };
     if (it.count <= kTileRows)
         run.template operator()<1>();
@@ -1139,12 +1180,15 @@ __global__ __launch_bounds__(kDownWaves * 64) void down_kernel(
     unsigned experts, const uint8_t* __restrict__ down, const int32_t* __restrict__ offsets,
     const int32_t* __restrict__ items, const int32_t* __restrict__ item_count,
     float* __restrict__ part_d, size_t part_stride, unsigned cols) {
-    __shared__ __align__(16) uint8_t stage[2 * StageCopy<kHTerms, 2, kDownWaves>::chunk_bytes];
+    __shared__ __align__(16) uint8_t stage0[chunk_bytes<kHTerms, 2>],
+        stage1[chunk_bytes<kHTerms, 2>], stage2[chunk_bytes<kHTerms, 2>];
+    uint8_t* const stage[kStages] = {stage0, stage1, stage2};
     const ItemCell cell = item_cell(cols);
     if (int(cell.item) >= *item_count)
         return;
     const Item it = load_item(items, offsets, cell.item);
-    const unsigned wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64),
+                   lane = threadIdx.x % 64;
     const unsigned i32 = lane % 32, h = lane / 32;
     const Packed shape = packed_shape(1, hidden, inter);  // per expert
     const unsigned pair = cell.col * kDownWaves + wave;
@@ -1160,8 +1204,8 @@ __global__ __launch_bounds__(kDownWaves * 64) void down_kernel(
     const Tiles hl = tile_layout(const_cast<uint8_t*>(ha), tiles, inter / 64, kHTerms);
     auto run = [&]<int TILES>() {
         f32x16 acc[2][TILES];
-        staged_pair<kHTerms, TILES, NT, 4, kDownWaves>(hl, cell.item, lane, w, q0, q1, active,
-                                                       stage, acc);
+        staged_pair<kHTerms, TILES, NT, kDownWaves>(hl, cell.item, wave, lane, w, q0, q1, active,
+                                                    stage, acc);
         if (!active)
             return;
 #pragma unroll
@@ -1259,13 +1303,6 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
 
 constexpr int kDecodeWaves = 16;
 constexpr unsigned kDecodeMaxSteps = 256;  // hidden / 64 of the single-token path (x in LDS)
-
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    [&]<int... I>(std::integer_sequence<int, I...>) {
-        (f.template operator()<I>(), ...);
-    }(std::make_integer_sequence<int, N>{});
-}
 
 // One packed 32-row group of an expert as buffer resources (wave-uniform): its codes
 // (steps KB) and its scale dwords (per 4 steps, 256 bytes).  Loads address a lane's bytes
@@ -1668,15 +1705,17 @@ unsigned down_columns(size_t hidden) {
 }
 
 // K slices of the grouped GEMMs: enough workgroups for about two per compute unit (two
-// fit at once) when the items are few (decode), one slice otherwise; slices are whole
-// multiples of 8 steps and none is empty.
+// fit at once) when the items are few (decode), one slice otherwise; none is empty.
 struct MoeSlices {
     unsigned gate_up, down;
 };
 
 MoeSlices moe_slices(size_t tokens, size_t hidden, size_t inter, size_t experts,
                      size_t top_k) {
-    const size_t items = std::min(tokens * top_k, experts);  // at least this many
+    // about this many work items: an expert each, or whole items when experts have several
+    // (4096 slots over 8 experts, counted as 8 items, ran gate / up in three slices: 420 us)
+    const size_t slots = tokens * top_k;
+    const size_t items = std::max(std::min(slots, experts), slots / kItemRows);
     // workgroups for about two gate/up (four waves) or one down (eight waves) per compute
     // unit
     auto slices = [&](size_t columns, size_t steps, size_t per_cu, bool round_up) {
@@ -1684,7 +1723,7 @@ MoeSlices moe_slices(size_t tokens, size_t hidden, size_t inter, size_t experts,
         size_t ks = round_up ? (target + columns * items - 1) / (columns * items)
                              : target / (columns * items);
         ks = std::min(std::max<size_t>(ks, 1), steps);
-        const size_t per = ((steps + ks - 1) / ks + 7) / 8 * 8;
+        const size_t per = steps_per_slice(unsigned(steps), unsigned(ks));
         return unsigned((steps + per - 1) / per);
     };
     // down rounds down: its workgroups (one per compute unit at its register count) then
@@ -2016,16 +2055,12 @@ int launch_layer(const uint16_t* x_bf16, const float* logits, size_t tokens, siz
     const unsigned items8 = (items + 7) / 8 * 8;
     const unsigned gu_cols = gate_up_columns(inter), d_cols = down_columns(hidden);
     const dim3 gu_grid(gu_cols * items8, 1, ks.gate_up);
-    if (nt)
-        hipLaunchKernelGGL(gate_up_kernel<true>, gu_grid, dim3(kGemmWaves * 64), 0, st, s.xa,
-                           unsigned(hidden), unsigned(inter), unsigned(experts), tiles, gate, up,
-                           s.offsets, s.items, s.item_count, s.ha, s.part_g, s.part_u, part_gu,
-                           gu_cols);
-    else
-        hipLaunchKernelGGL(gate_up_kernel<false>, gu_grid, dim3(kGemmWaves * 64), 0, st, s.xa,
-                           unsigned(hidden), unsigned(inter), unsigned(experts), tiles, gate, up,
-                           s.offsets, s.items, s.item_count, s.ha, s.part_g, s.part_u, part_gu,
-                           gu_cols);
+    const auto gate_up = nt ? gate_up_kernel<true> : gate_up_kernel<false>;
+    const auto down_product = nt ? down_kernel<true> : down_kernel<false>;
+    hipLaunchKernelGGL(gate_up, gu_grid, dim3(kGemmWaves * 64), 0, st, s.xa,
+                       unsigned(hidden), unsigned(inter), unsigned(experts), tiles, gate, up,
+                       s.offsets, s.items, s.item_count, s.ha, s.part_g, s.part_u, part_gu,
+                       gu_cols);
     KDQ_HIP(hipGetLastError());
     if (ks.gate_up > 1) {
         hipLaunchKernelGGL(finalize_kernel, dim3(unsigned((inter + 255) / 256), unsigned(slots)),
@@ -2035,14 +2070,9 @@ int launch_layer(const uint16_t* x_bf16, const float* logits, size_t tokens, siz
     }
     const size_t stride = slots * hidden;
     const dim3 d_grid(d_cols * items8, 1, ks.down);
-    if (nt)
-        hipLaunchKernelGGL(down_kernel<true>, d_grid, dim3(kDownWaves * 64), 0, st, s.ha, tiles,
-                           unsigned(hidden), unsigned(inter), unsigned(experts), down, s.offsets,
-                           s.items, s.item_count, s.part_d, stride, d_cols);
-    else
-        hipLaunchKernelGGL(down_kernel<false>, d_grid, dim3(kDownWaves * 64), 0, st, s.ha, tiles,
-                           unsigned(hidden), unsigned(inter), unsigned(experts), down, s.offsets,
-                           s.items, s.item_count, s.part_d, stride, d_cols);
+    hipLaunchKernelGGL(down_product, d_grid, dim3(kDownWaves * 64), 0, st,
+                       s.ha, tiles, unsigned(hidden), unsigned(inter), unsigned(experts), down,
+                       s.offsets, s.items, s.item_count, s.part_d, stride, d_cols);
     KDQ_HIP(hipGetLastError());
     const size_t n = tokens * hidden / 4;
     const dim3 grid(unsigned((n + 255) / 256));

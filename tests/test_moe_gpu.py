@@ -189,6 +189,9 @@ def run_layer(device, oracle, tokens, hidden, inter, experts, top_k, seed, hot=0
 
 @pytest.mark.parametrize("tokens,hidden,inter,experts,top_k", [
     (1, 64, 64, 4, 2), (3, 128, 192, 8, 2), (37, 256, 128, 8, 4), (130, 128, 128, 4, 4),
+    # K of 23, 13, 25 and 7 steps (part turns of the products' 12-step loop, in one slice and
+    # in several), few experts with many rows each
+    (70, 1472, 832, 8, 3), (20, 832, 1600, 4, 1), (700, 448, 320, 4, 2),
     (16, 2880, 2880, 32, 4),
     # more than 4096 slots (the chunked permutation): heavy items first, and experts of
     # several work items each
