@@ -151,9 +151,11 @@ struct XUnit {
     float4 a, b;
 };
 
-__device__ __forceinline__ void load_unit(const float* x, unsigned in, unsigned u, XUnit& v) {
+// (rows of x `pitch` values apart)
+__device__ __forceinline__ void load_unit(const float* x, unsigned in, unsigned u, XUnit& v,
+                                          size_t pitch) {
     const unsigned r = u / (in / 8), e = (u % (in / 8)) * 8;
-    const float4* src = reinterpret_cast<const float4*>(x + size_t(r) * in + e);
+    const float4* src = reinterpret_cast<const float4*>(x + r * pitch + e);
     v.a = src[0];
     v.b = src[1];
 }
@@ -517,7 +519,7 @@ __global__ __launch_bounds__(kThreads) void fast_gemv(const uint8_t* __restrict_
     // for them.
     const unsigned units = R * in / 8;
     XUnit first_unit;
-    load_unit(x, in, min(unsigned(threadIdx.x), units - 1), first_unit);
+    load_unit(x, in, min(unsigned(threadIdx.x), units - 1), first_unit, in);
     asm volatile("" ::: "memory");  // x is not restrict: its loads stay before this point
     __builtin_amdgcn_sched_barrier(0);
     Lane L[kRowsInFlight];
@@ -532,7 +534,7 @@ __global__ __launch_bounds__(kThreads) void fast_gemv(const uint8_t* __restrict_
         stage_unit<ENC>(in, threadIdx.x, first_unit, xq, xs);
     for (unsigned u = threadIdx.x + kThreads; u < units; u += kThreads) {
         XUnit more;
-        load_unit(x, in, u, more);
+        load_unit(x, in, u, more, in);
         stage_unit<ENC>(in, u, more, xq, xs);
     }
     __syncthreads();
@@ -1193,7 +1195,9 @@ struct MfmaJobs {
 // workgroups of several row tiles: every wavefront's activation request is issued before
 // any wavefront's weight requests (one barrier between them), so the staging's data does
 // not return behind other wavefronts' weights (C2 4096 -> 14336: 7.95 -> 7.77 us; with
-// one tile a workgroup, C1, it measured 0.35 us slower).
+// one tile a workgroup, C1, it measured 0.35 us slower).  FORM 4 is one K slice of a plain
+// product (job 0, `in` the slice's values): its x rows are x_step values apart and its
+// packed tiles y_step groups; with x_every set it adds to y (the slices after the first).
 //
 // mfma_gemv_body is the workgroup (bx, by) of that grid; `routed` >= 0 stands in for the
 // job's device index (the fused MoE decode, which selects the experts itself).  COHERENT
@@ -1207,7 +1211,8 @@ template <int ENC, int R, int W, bool PACKED, int FORM, bool COHERENT = false,
 __device__ __forceinline__ void mfma_gemv_body(const MfmaJobs& jobs, unsigned bx,
                                                unsigned by, int routed,
                                                const LateRoute& late = LateRoute{}) {
-    constexpr bool PLAIN = FORM > 0, X2 = FORM == 2, XFIRST = FORM == 3;
+    constexpr bool PLAIN = FORM > 0, SLICED = FORM == 4, X2 = FORM == 2 || SLICED,
+                   XFIRST = FORM == 3;
     constexpr bool LATE = !std::is_same_v<LateRoute, EarlyRoute>;
     const bool affine = !PLAIN && jobs.affine;
     const unsigned jid = affine ? 0 : by, step = affine ? by : 0;
@@ -1283,7 +1288,8 @@ __device__ __forceinline__ void mfma_gemv_body(const MfmaJobs& jobs, unsigned bx
             const uint8_t* w = second ? up : weights;
             const unsigned n = min(p0 + 16 * (second ? t - tiles : t) + j, r1 - 1);
             if constexpr (PACKED)
-                load_packed<ENC>(w + (size_t(n / 16) * groups + g) * PackedFormat<ENC>::unit,
+                load_packed<ENC>(w + (size_t(n / 16) * (SLICED ? jobs.y_step : groups) + g) *
+                                         PackedFormat<ENC>::unit,
                                  G, n % 16, L[k]);
             else if constexpr (ENC == KDQ_Q6_K)
                 load_lane_q6k(w + size_t(n) * row_bytes, g, G, L[k]);
@@ -1307,9 +1313,11 @@ __device__ __forceinline__ void mfma_gemv_body(const MfmaJobs& jobs, unsigned bx
 
     const unsigned units_x = R * in / 8;
     XUnit first_unit, second_unit;
-    load_unit(x, in, min(unsigned(threadIdx.x), units_x - 1), first_unit);
+    const size_t x_pitch = SLICED ? jobs.x_step : in;
+    load_unit(x, in, min(unsigned(threadIdx.x), units_x - 1), first_unit, x_pitch);
     if constexpr (X2)
-        load_unit(x, in, min(unsigned(threadIdx.x) + kThreads, units_x - 1), second_unit);
+        load_unit(x, in, min(unsigned(threadIdx.x) + kThreads, units_x - 1), second_unit,
+                  x_pitch);
     // the lattice grid entries this thread converts, requested before the weights (the
     // staging waits for them)
     unsigned entry[lattice(ENC) ? lattice_per_thread<ENC, kThreads> : 1];
@@ -1338,7 +1346,7 @@ __device__ __forceinline__ void mfma_gemv_body(const MfmaJobs& jobs, unsigned bx
         mstage_unit<ENC>(in, threadIdx.x + kThreads, second_unit, atab, blocks);
     for (unsigned u = threadIdx.x + (X2 ? 2 : 1) * kThreads; u < units_x; u += kThreads) {
         XUnit more;
-        load_unit(x, in, u, more);
+        load_unit(x, in, u, more, x_pitch);
         mstage_unit<ENC>(in, u, more, atab, blocks);
     }
     __syncthreads();
@@ -1412,6 +1420,8 @@ __device__ __forceinline__ void mfma_gemv_body(const MfmaJobs& jobs, unsigned bx
                 if constexpr (COHERENT)
                     __hip_atomic_store(&y[size_t(r) * stride + n], v, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
+                else if (SLICED && jobs.x_every)
+                    y[size_t(r) * stride + n] += v;
                 else
                     y[size_t(r) * stride + n] = v;
             }
@@ -1553,6 +1563,8 @@ size_t mfma_lds(size_t batch, size_t in, unsigned mats = 1, size_t table = 0) {
     return mfma_layout(unsigned(batch), unsigned(in), mats, table).total;
 }
 
+constexpr size_t kMfmaLdsLimit = 160 * 1024;
+
 struct MfmaPlan {
     unsigned rows_per_wg, grid, batch, waves;
 };
@@ -1564,7 +1576,7 @@ struct MfmaPlan {
 // (8 row slots of one chunk) belongs to one workgroup.
 bool plan_mfma(size_t rows, size_t in, size_t total_out, MfmaPlan& p, bool packed = false,
                unsigned mats = 1, size_t table = 0) {
-    constexpr size_t limit = 160 * 1024;
+    constexpr size_t limit = kMfmaLdsLimit;
     if (in % 256 || mfma_lds(1, in, mats, table) > limit)
         return false;
     unsigned batch = 1;
@@ -1669,19 +1681,78 @@ int launch_mfma_rows(unsigned r, unsigned waves, const MfmaJobs& jobs, hipStream
     }
 }
 
+// One pass of R activation rows whose staged form does not fit the LDS over all of K: K
+// slices of equal groups, the fewest that fit, launched in order, each adding to y.
+template <int ENC, int R, bool PACKED>
+int launch_sliced(const uint8_t* w, size_t row_bytes, const float* x, size_t in, size_t out,
+                  float* y, size_t stride, unsigned* status, hipStream_t stream) {
+    const size_t groups = in / 256, table = mfma_table_bytes(ENC);
+    size_t slices = 2;
+    while (mfma_lds(R, (groups + slices - 1) / slices * 256, 1, table) > kMfmaLdsLimit)
+        ++slices;
+    const size_t per = (groups + slices - 1) / slices;
+    size_t group_bytes = 256 / block_values(ENC) * block_bytes(ENC);
+    if constexpr (PACKED)
+        group_bytes = PackedFormat<ENC>::unit;
+    for (size_t g = 0; g < groups; g += per) {
+        const size_t n = std::min(per, groups - g);
+        MfmaPlan p;
+        if (!plan_mfma(R, n * 256, out, p, PACKED, 1, table) || p.batch < unsigned(R))
+            return KDQ_ERR_UNSUPPORTED;  // (never: R rows of `per` groups fit)
+        MfmaJobs jobs{};
+        jobs.count = 1;
+        jobs.in = unsigned(n * 256);
+        jobs.job[0] = MfmaJob{w + g * group_bytes, x + g * 256, y, status, row_bytes, stride,
+                              unsigned(out), 0};
+        jobs.x_step = in;
+        jobs.y_step = groups;
+        jobs.x_every = g ? 1u : 0u;
+        // whole compute units' shares of rows: the launch runs 16 wavefronts a workgroup
+        const size_t share = (out + compute_units() - 1) / compute_units();
+        number_workgroups(jobs, unsigned(PACKED ? (share + 7) & ~size_t(7) : share));
+        const int rc = launch_mfma_form<ENC, R, 16, PACKED, 4>(jobs, stream);
+        if (rc)
+            return rc;
+    }
+    return KDQ_OK;
+}
+
 // `rows` activation rows in passes of the plan's batch (the largest power of two that
-// fits what is left).  `row_bytes` is unused over packed weights.
+// fits what is left).  `row_bytes` is unused over packed weights.  Where several rows do
+// not fit the LDS together over all of K (a long input), a pass still takes up to 4 of them
+// and runs in K slices, so that the weights are read once a pass: 4 rows of Q3_K
+// 14336 -> 4096 42.7 us in two passes of 2 rows, 26.8 in two slices of 4.  Passes of 8 rows
+// gain nothing over two of 4 (Q8_0 7168 -> 16384: 54.7 us, in two slices of 8 57.2): the
+// products then outweigh the weights.  Nor do 4 rows of a shorter input (Q4_K 9216 -> 6562,
+// packed: 21.7 us in two passes of 2, 22.6 in slices; 14336 -> 4096 24.8 and 21.1).
+constexpr size_t kSlicedInputs = 12288;
+
 template <int ENC, bool PACKED>
 int launch_mfma(const void* w, size_t row_bytes, const float* x, size_t rows, size_t in,
                 size_t out, float* y, size_t stride, unsigned* status, hipStream_t stream) {
     MfmaPlan p;
     if (!plan_mfma(rows, in, out, p, PACKED, 1, mfma_table_bytes(ENC)))
         return KDQ_ERR_UNSUPPORTED;
+    const unsigned most = unsigned(std::min<size_t>(rows, 4));
+    // (a larger pass than fits would be filled)
+    const bool sliced = in >= kSlicedInputs && p.batch * 2 <= most;
     for (size_t first = 0; first < rows;) {
         const size_t left = rows - first;
-        unsigned r = p.batch;
+        unsigned r = sliced ? 4 : p.batch;
         while (r > left)
             r /= 2;
+        if (r > p.batch) {
+            auto run = [&](auto launch) {
+                return launch(static_cast<const uint8_t*>(w), row_bytes, x + first * in, in, out,
+                              y + first * stride, stride, status, stream);
+            };
+            const int rc = r == 2 ? run(launch_sliced<ENC, 2, PACKED>)
+                                  : run(launch_sliced<ENC, 4, PACKED>);
+            if (rc)
+                return rc;
+            first += r;
+            continue;
+        }
         MfmaJobs jobs{};
         jobs.count = 1;
         jobs.in = unsigned(in);

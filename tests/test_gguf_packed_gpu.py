@@ -202,3 +202,30 @@ def test_packed_rejections(device):
     with pytest.raises(kadan_amd.KdqError):
         kadan_amd.call("kdq_gemv_packed", Q4_K, buf.data_ptr() + 4, x.data_ptr(), 1, 256, 16,
                        y.data_ptr(), 16, None, ops._stream())
+
+
+@pytest.mark.parametrize("enc", [2, 8, 12, 14, 11, 23, 20, 22])
+@pytest.mark.parametrize("rows", [4, 5, 8, 15])
+def test_gemv_long_rows_in_k_slices(device, oracle, enc, rows):
+    """Several rows of a long input (14336 and 14336 + 256 values: equal and unequal K
+    slices) do not fit the LDS together and run in K slices that add to y: y starts as
+    garbage, and 5, 8 and 15 rows take several passes."""
+    import torch
+    from kadan_amd import ops
+    for n_in in (14336, 14592):
+        n_out = 40
+        w = synth.gguf_weights(enc, 0x51 + rows, n_out, n_in)
+        x = synth.normal(0x51 + rows, 5, rows * n_in).reshape(rows, n_in)
+        want = oracle.gemv(enc, w, x, n_in, n_out)
+        wd, xd = torch.from_numpy(w).to(device), torch.from_numpy(x).to(device)
+        forms = [lambda y: ops.gemv(enc, wd, xd, n_out, out=y)]
+        if enc in (2, 8, 12, 14):
+            packed = ops.gguf_pack(enc, wd, n_in)
+            forms.append(lambda y: ops.gemv_packed(enc, packed, xd, n_out, out=y))
+        got = []
+        for product in forms:
+            y = torch.full((rows, n_out), float("nan"), device=device)
+            product(y)
+            assert_close(y.cpu().numpy(), want, what=f"sliced gemv enc={enc} rows={rows}")
+            got.append(y.cpu().numpy())
+        assert all(np.array_equal(got[0], g) for g in got)
