@@ -147,8 +147,16 @@ def check(function: str, status: int) -> None:
     raise KdqError(function, status, hip)
 
 
+_functions: dict[str, C._CFuncPtr] = {}  # the entry points called so far
+
+
 def call(function: str, *args) -> None:
-    check(function, getattr(lib(), function)(*args))
+    fn = _functions.get(function)
+    if fn is None:
+        fn = _functions[function] = getattr(lib(), function)
+    status = fn(*args)
+    if status:
+        check(function, status)
 
 
 def row_bytes(encoding: int, n_in: int) -> int:

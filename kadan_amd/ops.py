@@ -7,6 +7,7 @@ current HIP stream to the corresponding ``kdq_*`` entry point, and raises
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -14,11 +15,21 @@ from . import BLOCK_BYTES, BLOCK_VALUES, MatvecJob, call, lib
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current HIP stream.  A decode product takes 6-8 us on the device, so its wrapper must
+    not take longer: the raw handle, without the Stream object torch.cuda.current_stream()
+    builds."""
+    if not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
+
+
+def _rows(x: torch.Tensor) -> torch.Tensor:
+    """x as [rows, n_in]."""
+    return x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
 
 
 def _need(t: torch.Tensor, dtype, name: str) -> None:
@@ -44,7 +55,7 @@ def gemv(encoding: int, weights: torch.Tensor, x: torch.Tensor, n_out: int,
     x fp32 [rows, n_in] -> y fp32 [rows, n_out] (kdq_gemv / kdq_gemv_exact)."""
     _need(weights, torch.uint8, "weights")
     _need(x, torch.float32, "x")
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = _rows(x)
     rows, n_in = x2.shape
     if weights.shape[0] != n_out:
         raise ValueError("weights rows != n_out")
@@ -64,7 +75,7 @@ def gemv_batch(jobs: list[dict]) -> None:
     table = (MatvecJob * len(jobs))()
     for i, j in enumerate(jobs):
         w, x, y = j["weights"], j["input"], j["output"]
-        x2 = x.reshape(-1, x.shape[-1])
+        x2 = _rows(x)
         table[i] = MatvecJob(w.data_ptr(), x2.data_ptr(), y.data_ptr(),
                              _ptr(j.get("status")) or 0, w.shape[1],
                              y.stride(0) if y.dim() == 2 else w.shape[0],
@@ -72,6 +83,7 @@ def gemv_batch(jobs: list[dict]) -> None:
     call("kdq_gemv_batch", C.addressof(table) if jobs else None, len(jobs), _stream())
 
 
+@functools.lru_cache(maxsize=4096)
 def gguf_packed_bytes(encoding: int, n_in: int, n_out: int) -> int:
     return int(lib().kdq_gguf_packed_bytes(encoding, n_in, n_out))
 
@@ -96,7 +108,7 @@ def gemv_packed(encoding: int, packed: torch.Tensor, x: torch.Tensor, n_out: int
     """gemv over tile-packed weights (kdq_gemv_packed)."""
     _need(packed, torch.uint8, "packed")
     _need(x, torch.float32, "x")
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = _rows(x)
     rows, n_in = x2.shape
     if packed.numel() != gguf_packed_bytes(encoding, n_in, n_out):
         raise ValueError("packed size does not match (encoding, n_in, n_out)")
@@ -115,7 +127,7 @@ def gemv_packed_batch(jobs: list[dict]) -> None:
     table = (MatvecJob * len(jobs))()
     for i, j in enumerate(jobs):
         w, x, y = j["weights"], j["input"], j["output"]
-        x2 = x.reshape(-1, x.shape[-1])
+        x2 = _rows(x)
         table[i] = MatvecJob(w.data_ptr(), x2.data_ptr(), y.data_ptr(),
                              _ptr(j.get("status")) or 0, 0,
                              y.stride(0) if y.dim() == 2 else j["columns"],
