@@ -339,23 +339,23 @@ __global__ __launch_bounds__(256) void check_kernel(const uint8_t* __restrict__ 
 // Row t of x (fp32, k values): its scale sigma = 2^e with max|x| / sigma in [2^14, 2^15)
 // (1 for an all-zero row), and fp16(x / sigma) permuted per 256-value group: logical
 // 16-byte chunk q = 16j + 8h + 4p + u of a group holds operand elements 0..7 of sub-step
-// s = 8j + 4p + u for lane half h.  One 256-thread workgroup per row; the row passes
+// s = 8j + 4p + u for lane half h.  One workgroup per row; the row passes
 // through LDS.  With `slot_of` (rows are positions of a grouped layer), rows from *used on
 // and rows with slot_of[t] < 0 are not staged.
-template <int ENC>
-__global__ __launch_bounds__(256) void stage_kernel(const float* __restrict__ x, unsigned k,
+template <int ENC, int THREADS>
+__global__ __launch_bounds__(THREADS) void stage_kernel(const float* __restrict__ x, unsigned k,
                                                     uint16_t* __restrict__ xs,
                                                     float* __restrict__ sigma,
                                                     const int32_t* __restrict__ slot_of,
                                                     const unsigned* __restrict__ used) {
     extern __shared__ __align__(16) float row[];
-    __shared__ float wave_max[4];
+    __shared__ float wave_max[THREADS / 64];
     const unsigned t = blockIdx.x;
     if (slot_of && (t >= *used || slot_of[t] < 0))
         return;
     const float* src = x + size_t(t) * k;
     float amax = 0.f;
-    for (unsigned i = threadIdx.x; i < k / 4; i += 256) {
+    for (unsigned i = threadIdx.x; i < k / 4; i += THREADS) {
         const float4 v = reinterpret_cast<const float4*>(src)[i];
         reinterpret_cast<float4*>(row)[i] = v;
         amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
@@ -366,7 +366,10 @@ __global__ __launch_bounds__(256) void stage_kernel(const float* __restrict__ x,
     if (threadIdx.x % 64 == 0)
         wave_max[threadIdx.x / 64] = amax;
     __syncthreads();
-    amax = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
+    amax = wave_max[0];
+#pragma unroll
+    for (int v = 1; v < THREADS / 64; ++v)
+        amax = fmaxf(amax, wave_max[v]);
     // exponent of amax (normal or subnormal), scale 2^(e - 14)
     int e = 0;
     float scale = 1.f, inv = 1.f;
@@ -380,7 +383,7 @@ __global__ __launch_bounds__(256) void stage_kernel(const float* __restrict__ x,
     if (threadIdx.x == 0)
         sigma[t] = scale;
     uint16_t* dst = xs + size_t(t) * k;
-    for (unsigned c = threadIdx.x; c < k / 8; c += 256) {
+    for (unsigned c = threadIdx.x; c < k / 8; c += THREADS) {
         const unsigned g = c / 32, q = c % 32;
         const unsigned h = (q / 8) % 2, s = 8 * (q / 16) + 4 * ((q / 4) % 2) + q % 4;
         unsigned words[4];
@@ -1002,8 +1005,12 @@ int configure() {
     static bool configured = false;  // one attribute call per instantiation
     if (!configured) {
         constexpr int W = gemm_waves<ENC>;
-        KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&stage_kernel<ENC>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024));
+        const auto few = stage_kernel<ENC, 256>;
+        const auto many = stage_kernel<ENC, 1024>;
+        for (const void* f : {reinterpret_cast<const void*>(few),
+                              reinterpret_cast<const void*>(many)})
+            KDQ_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        128 * 1024));
         KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<ENC, W>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds)));
         for (const void* f : {reinterpret_cast<const void*>(&stream_gemm_kernel<ENC, false>),
@@ -1012,6 +1019,20 @@ int configure() {
                                         int(kStreamLds<ENC>)));
         configured = true;
     }
+    return KDQ_OK;
+}
+
+// Stages `rows` rows of k values: 1024 threads a row where each has a whole 16-byte load or
+// more (4096 values), else 256, which would loop: 77 rows of 14336 8.0 -> 4.3 us, 512 of 4096
+// 7.2 -> 6.2.
+template <int ENC>
+int launch_stage(const float* x, size_t rows, size_t k, uint16_t* xs, float* sigma,
+                 const int32_t* slot_of, const unsigned* used, hipStream_t st) {
+    const bool wide = k >= 4096;
+    auto kernel = wide ? stage_kernel<ENC, 1024> : stage_kernel<ENC, 256>;
+    hipLaunchKernelGGL(kernel, dim3(unsigned(rows)), dim3(wide ? 1024 : 256), k * 4, st, x,
+                       unsigned(k), xs, sigma, slot_of, used);
+    KDQ_HIP(hipGetLastError());
     return KDQ_OK;
 }
 
@@ -1045,9 +1066,8 @@ int launch_grouped(const void* packed, const void* up, size_t expert_bytes,
     int rc;
     if ((rc = configure<ENC>()))
         return rc;
-    hipLaunchKernelGGL(stage_kernel<ENC>, dim3(unsigned(x_rows)), dim3(256), k * 4, st, x,
-                       unsigned(k), xs, sigma, topk ? nullptr : inv, used);
-    KDQ_HIP(hipGetLastError());
+    if ((rc = launch_stage<ENC>(x, x_rows, k, xs, sigma, topk ? nullptr : inv, used, st)))
+        return rc;
     return launch_stream<ENC>(xs, sigma, packed, up, positions, n, k, 1u, unsigned(k / 256), y,
                               nullptr, status, tile_expert, expert_bytes, inv, topk, used, st);
 }
@@ -1106,9 +1126,8 @@ int launch_gemm(const float* x, const uint8_t* packed, size_t m, size_t n, size_
     auto* part = slices > 1 ? reinterpret_cast<float*>(scratch + g.xs + g.sigma) : nullptr;
     if ((rc = configure<ENC>()))
         return rc;
-    hipLaunchKernelGGL(stage_kernel<ENC>, dim3(unsigned(m)), dim3(256), k * 4, st, x,
-                       unsigned(k), xs, sigma, nullptr, nullptr);
-    KDQ_HIP(hipGetLastError());
+    if ((rc = launch_stage<ENC>(x, m, k, xs, sigma, nullptr, nullptr, st)))
+        return rc;
     if (plan.stream) {
         if ((rc = launch_stream<ENC>(xs, sigma, packed, nullptr, m, n, k, slices, per, y, part,
                                      status, nullptr, 0, nullptr, 0u, nullptr, st)))
@@ -1191,9 +1210,8 @@ int dense_gemm_pair(int encoding, const void* gate, const void* up, size_t n, si
             return rc;
         auto* xs = reinterpret_cast<uint16_t*>(sc);
         auto* sigma = reinterpret_cast<float*>(sc + g.xs);
-        hipLaunchKernelGGL(stage_kernel<ENC>, dim3(unsigned(m)), dim3(256), k * 4, st, x,
-                           unsigned(k), xs, sigma, nullptr, nullptr);
-        KDQ_HIP(hipGetLastError());
+        if ((rc = launch_stage<ENC>(x, m, k, xs, sigma, nullptr, nullptr, st)))
+            return rc;
         return launch_stream<ENC>(xs, sigma, gate, up, m, n, k, 1u, unsigned(k / 256), y, nullptr,
                                   status, nullptr, 0, nullptr, 0u, nullptr, st);
     };
