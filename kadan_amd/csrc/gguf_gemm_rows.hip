@@ -555,8 +555,9 @@ __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
 
     // Software pipeline, one barrier per step.  The top of step s refills the LDS buffers
     // that step s - 1 finished reading: activations of step s + 1 (from a register ring,
-    // loaded kAhead steps earlier) and, on a group's last step, the raw bytes of the next
-    // group (loaded a whole group earlier).  Each refill is followed at once by the load
+    // loaded kAhead steps earlier) and, on a group's last step but one, the raw bytes of the next
+    // group (loaded a whole group earlier; stored a step early, as the weights are decoded one
+    // step ahead).  Each refill is followed at once by the load
     // that reuses its registers, so a store only ever waits on loads issued at least
     // kAhead steps (or one group) before.  The loop is unrolled by one turn of the ring, so
     // its register indices are constants; loads past the end re-read the last step or
@@ -585,32 +586,50 @@ __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     const uint8_t* my_row0 = raw + (wave * 32 + r) * G::pitch;
+    // this lane's weights of step s: per 16-value sub-step values 8 h .. +7
+    auto decode = [&](unsigned s, f16x8 (&a)[2]) {
+        const unsigned g = s / PG, within = s % PG;
+        const uint8_t* row = my_row0 + (g % 2) * RN * G::pitch;
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub)
+            a[sub] = RowsDecode<ENC>::run(row, within * RK + 16 * sub + 8 * h, flags, table);
+    };
+    // The weights are decoded one step ahead, so that the decode's VALU work and LDS reads run
+    // beside the products instead of before them (512 x 4096 -> 14336: IQ4_XS 111 -> 106 us,
+    // IQ4_NL 129 -> 124).
+    f16x8 a[2];
+    decode(0, a);
     auto step = [&]<int U>(unsigned s) {  // U = s % kUnroll
         constexpr int slot = (U + 1) % kAhead;
         const unsigned g = s / PG, within = s % PG;
         store_x((s + 1) % 2, xv[slot]);
         load_x(min(s + 1 + kAhead, steps - 1), xv[slot]);
-        if (within == PG - 1) {
+        if (within == PG - 2) {  // the last step decodes the next group's first weights
             store_raw((g + 1) % 2, rv);
             load_raw(min(g + 2, groups - 1), rv);
         }
-        const uint8_t* row = my_row0 + (g % 2) * RN * G::pitch;
         const uint8_t* xb = xt + (s % 2) * RM * RK * 2;
+        f16x8 xf[2][TB];
 #pragma unroll
         for (int sub = 0; sub < 2; ++sub) {
-            // this lane's 8 weights: values 16 sub + 8 h .. +7 of the step
-            const unsigned kk = within * RK + 16 * sub + 8 * h;
-            const f16x8 a = RowsDecode<ENC>::run(row, kk, flags, table);
             const unsigned c = 2 * sub + h;  // 16-byte chunk of the token's 64 bytes
 #pragma unroll
             for (int b = 0; b < TB; ++b) {
                 const unsigned t = 32 * b + r;
-                const f16x8 xf =
-                    *reinterpret_cast<const f16x8*>(xb + t * 64 +
-                                                    16 * (c ^ (((t >> 1) ^ (t >> 3)) & 3u)));
-                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, xf, acc[b], 0, 0, 0);
+                xf[sub][b] = *reinterpret_cast<const f16x8*>(
+                    xb + t * 64 + 16 * (c ^ (((t >> 1) ^ (t >> 3)) & 3u)));
             }
         }
+        // (BF16, which has little to decode meanwhile: every read ahead of the products, 119 ->
+        // 114 us at 512 x 4096 -> 14336; 2-4 % slower for the others)
+        if constexpr (ENC == KDQ_BF16)
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[sub], xf[sub][b], acc[b], 0, 0, 0);
+        decode(min(s + 1, steps - 1), a);  // beside the products
         __syncthreads();
     };
     unsigned s = 0;
