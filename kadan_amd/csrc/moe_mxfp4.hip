@@ -1723,8 +1723,15 @@ MoeSlices moe_slices(size_t tokens, size_t hidden, size_t inter, size_t experts,
         size_t ks = round_up ? (target + columns * items - 1) / (columns * items)
                              : target / (columns * items);
         ks = std::min(std::max<size_t>(ks, 1), steps);
-        const size_t per = steps_per_slice(unsigned(steps), unsigned(ks));
-        return unsigned((steps + per - 1) / per);
+        const auto count = [&](size_t per) { return (steps + per - 1) / per; };
+        // no more than slices of whole eights would give: the partials of more took layers
+        // past the static scratch below (64 -> 2496, 64 experts, 4096 slots: 4 for 3)
+        ks = std::min(count(steps_per_slice(unsigned(steps), unsigned(ks))),
+                      count(((steps + ks - 1) / ks + 7) / 8 * 8));
+        // and none empty: fewer slices may be longer ones, so until the count stands
+        for (size_t n; (n = count(steps_per_slice(unsigned(steps), unsigned(ks)))) < ks;)
+            ks = n;
+        return unsigned(ks);
     };
     // down rounds down: its workgroups (one per compute unit at its register count) then
     // run in one round rather than one and a part (C4 T=256: 1 slice, 192 workgroups)

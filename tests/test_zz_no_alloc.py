@@ -64,3 +64,22 @@ def test_noalloc_refuses_what_does_not_fit(device):
     logits = torch.zeros(tokens, experts, dtype=torch.float32, device=device)
     with pytest.raises(kadan_amd.KdqError, match="kdq_projection_scratch"):
         _call_noalloc(torch, x, logits, top_k, inter, packed)
+
+
+def test_noalloc_takes_what_eights_of_steps_fit(device):
+    """4096 slots of 64 -> 2496 over 64 experts: 64 MiB less 0.3 with the down product in three K
+    slices (as slices of whole eights of steps give), 0.7 MiB too many with four."""
+    import torch
+    hidden, inter, experts, top_k, tokens = 64, 2496, 64, 8, 512
+    weights = synth.moe_weights_torch(0x7C, experts, hidden, inter, device)
+    packed = [ops.moe_mxfp4_pack(*weights[0], experts, inter, hidden),
+              ops.moe_mxfp4_pack(*weights[1], experts, inter, hidden),
+              ops.moe_mxfp4_pack(*weights[2], experts, hidden, inter)]
+    x, logits = synth.moe_inputs(0x7D, tokens, hidden, experts)
+    xb = torch.from_numpy(x).to(device).view(torch.bfloat16)
+    lg = torch.from_numpy(logits).to(device)
+    got = _call_noalloc(torch, xb, lg, top_k, inter, packed)
+    want = ops.moe_mxfp4_packed(xb, lg, top_k, inter, *packed, routing=True)
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert np.array_equal(a.cpu().numpy().view(np.uint8), b.cpu().numpy().view(np.uint8))
