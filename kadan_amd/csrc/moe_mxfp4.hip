@@ -776,10 +776,13 @@ __device__ __forceinline__ WavePair wave_pair(const uint8_t* packed, const Packe
 // Steps per turn of the products' loop (staged_pair).
 constexpr unsigned kTurnSteps = 12;
 
-// Steps of a K slice when `steps` are cut into about `slices`: whole turns of the products'
-// loop, unless that leaves the last slice less than half a slice; then whole sets of scales.
+// Steps of a K slice when `steps` are cut into about `slices`: eight (two sets of scales) when
+// they are short, else whole turns of the products' loop, unless that leaves the last slice
+// less than half a slice; then whole sets of scales.
 __host__ __device__ inline unsigned steps_per_slice(unsigned steps, unsigned slices) {
     const unsigned even = (steps + slices - 1) / slices;
+    if (even <= 8)
+        return 8;
     const unsigned turns = (even + kTurnSteps - 1) / kTurnSteps * kTurnSteps;
     const unsigned last = steps - (steps - 1) / turns * turns;
     return turns == kTurnSteps || last * 2 >= turns ? turns : (even + 3) / 4 * 4;
@@ -1726,8 +1729,15 @@ MoeSlices moe_slices(size_t tokens, size_t hidden, size_t inter, size_t experts,
         const auto count = [&](size_t per) { return (steps + per - 1) / per; };
         // no more than slices of whole eights would give: the partials of more took layers
         // past the static scratch below (64 -> 2496, 64 experts, 4096 slots: 4 for 3)
-        ks = std::min(count(steps_per_slice(unsigned(steps), unsigned(ks))),
-                      count(((steps + ks - 1) / ks + 7) / 8 * 8));
+        const size_t even = (steps + ks - 1) / ks, eights = count((even + 7) / 8 * 8);
+        // short slices: a whole turn each where that still gives three compute units in four
+        // a workgroup (264 tokens, top 2 of 8, 1536 -> 1856: 62.9 us, with eights 65.2), else
+        // eights (2 tokens, 64 experts, 1024 -> 2048: 25.1 us, with turns 27.7)
+        if (even > 8)
+            ks = eights;
+        else
+            ks = columns * items * count(kTurnSteps) * 4 >= 3 * size_t(compute_units())
+                     ? count(kTurnSteps) : eights;
         // and none empty: fewer slices may be longer ones, so until the count stands
         for (size_t n; (n = count(steps_per_slice(unsigned(steps), unsigned(ks)))) < ks;)
             ks = n;
