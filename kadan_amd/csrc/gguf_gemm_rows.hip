@@ -6,8 +6,8 @@
 // services/hikari/inference_worker), whatever the encoding.  The packed GEMM
 // (gguf_gemm.hip) covers Q4_K, Q8_0 and Q6_K over the bank's tile-packed copy with
 // dequantisation specialised per format; this kernel takes every other encoding (Q3_K,
-// IQ4_XS, IQ4_NL, IQ3_XXS, IQ3_S, IQ2_S, BF16, Q4_0) through the one exact decoder the
-// decode-time products use (decode_run, kdq_decode.hpp), so each weight byte is read once
+// IQ4_XS, IQ4_NL, IQ3_XXS, IQ3_S, IQ2_S, BF16, Q4_0) with the values of the exact decoder
+// that the decode-time products use (decode_run, kdq_decode.hpp), so each weight byte is read once
 // per workgroup tile instead of once per 8 activation rows.
 //
 //   stage_rows_kernel  one workgroup per token row (rows up to the next whole token tile,
@@ -22,7 +22,7 @@
 //                      through LDS (double-buffered, swizzled; loaded up to four steps
 //                      ahead into a ring of registers); each lane decodes the 8
 //                      values of its MFMA A operand (its row, its half of the 16-value
-//                      sub-step) with decode_run from the LDS bytes, rounds them to fp16 and
+//                      sub-step) from the LDS bytes a step ahead (RowsDecode), as fp16, and
 //                      multiplies on v_mfma_f32_32x32x16_f16 with fp32 accumulation.  The
 //                      epilogue undoes sigma and stores fp32 rows.  Outputs too narrow to
 //                      give every compute unit two workgroups split K into slices whose

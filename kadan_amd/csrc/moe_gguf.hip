@@ -24,6 +24,7 @@
 // on them with per-expert batch jobs of gathered rows, IW/include/kadan/dense_compute.hpp:
 // 197-201) take stages 4-6 grouped by expert instead of per slot, so each expert's
 // weights are read once per 8 of its rows rather than once per slot:
+//   1'. router_kernel for an F32 router (MFMA, full fp32), the shared gate and up as in 1
 //   4'. group_kernel: a counting sort of the slots by expert into segments padded to whole
 //       items of kItemRows rows (slot -> position, position -> slot, the expert of every
 //       item, -1 past the used ones); gather_kernel: x rows into position order (padding
