@@ -83,7 +83,7 @@ def gemv_batch(jobs: list[dict]) -> None:
     call("kdq_gemv_batch", C.addressof(table) if jobs else None, len(jobs), _stream())
 
 
-@functools.lru_cache(maxsize=4096)
+@functools.lru_cache(maxsize=4096, typed=True)  # (256.0 is refused, also after 256)
 def gguf_packed_bytes(encoding: int, n_in: int, n_out: int) -> int:
     return int(lib().kdq_gguf_packed_bytes(encoding, n_in, n_out))
 

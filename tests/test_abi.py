@@ -126,6 +126,14 @@ def test_product_path_has_no_cpu_fallback(monkeypatch, tmp_path):
         kadan_amd.lib()
 
 
+def test_packed_sizes_looked_up_once_still_refuse_a_float():
+    import ctypes
+    from kadan_amd import ops
+    assert ops.gguf_packed_bytes(12, 256, 16) == 2304
+    with pytest.raises(ctypes.ArgumentError):
+        ops.gguf_packed_bytes(12, 256.0, 16)  # equal to 256, and hashed like it
+
+
 def test_gguf_packed_geometry_and_argument_errors():
     import kadan_amd
     lib = kadan_amd.lib()
