@@ -43,8 +43,9 @@ constexpr int kStageRow = 512;               // LDS bytes per token of one stage
 constexpr int kDmaRows = 1024 / kStageRow;   // token rows per 64-lane 16-byte DMA
 constexpr int kOutPitch = kTiles * 16 * 4 + 16;  // fp32 output row in LDS (+16: banks)
 constexpr int kStreamTM = int(kGroupedTileRows);  // tokens per tile of the streaming kernel
-// LDS of a workgroup: two activation stages, reused for the output
-constexpr size_t kLds = std::max(size_t(PM) * kOutPitch, 2 * size_t(PM) * kStageRow);
+// LDS of a workgroup of TB 32-token blocks: two activation stages, reused for the output
+template <int TB> constexpr size_t kLds =
+    32 * TB * std::max(size_t(kOutPitch), 2 * size_t(kStageRow));
 
 typedef __attribute__((address_space(3))) void lds_void;
 
@@ -409,9 +410,9 @@ __device__ __forceinline__ auto activation_resource(const uint16_t* xs) {
                                              0x00027000);
 }
 
-// Workgroup tile: 128 tokens x 256 weight rows (16 packed tiles); wavefront w owns tiles
-// 4w .. 4w + 3 as two 32-row operands.  K runs over 256-value groups; each group's 128
-// tokens x 512 bytes of permuted activations are staged into LDS by 16-byte DMA
+// Workgroup tile: 32 TB tokens (128; 96 where they hold every token) x 256 weight rows (16
+// packed tiles); wavefront w owns tiles 4w .. 4w + 3 as two 32-row operands.  K runs over
+// 256-value groups; each group's tokens x 512 bytes of permuted activations are staged into LDS by 16-byte DMA
 // (double-buffered, one group ahead), chunk q of token t at t*512 + 16*(q ^ (t % 16)),
 // and the next group's weight registers load during the current group's sub-steps.
 // `xs` has rows up to the next multiple of 128 tokens (rows past m are computed, never
@@ -422,7 +423,7 @@ __device__ __forceinline__ auto activation_resource(const uint16_t* xs) {
 // runs groups [ks * per, (ks + 1) * per) and writes its fp32 tile to part[ks] (m x n);
 // reduce_kernel then sums the slices in order.
 //
-template <int ENC, int W>
+template <int ENC, int W, int TB>
 __global__ __launch_bounds__(W * 64, 1) void gemm_kernel(
     const uint16_t* __restrict__ xs, const float* __restrict__ sigma,
     const uint8_t* __restrict__ w, unsigned m, unsigned n, unsigned k, unsigned slices,
@@ -433,7 +434,7 @@ __global__ __launch_bounds__(W * 64, 1) void gemm_kernel(
     extern __shared__ __align__(16) uint8_t lds[];
     // W wavefronts of NBW 32-row operands each (8 operands, 256 rows, per workgroup), TB
     // token blocks of 32
-    constexpr int TM = PM, NBW = 8 / W, TB = TM / 32;
+    constexpr int TM = 32 * TB, NBW = 8 / W;
     constexpr int DMAS = TM / kDmaRows / W;  // DMA instructions per wavefront per group
     constexpr int SB = TM * kStageRow;       // bytes of one activation stage
     constexpr int TILES = kTiles;            // 16-row output tiles per workgroup
@@ -471,20 +472,23 @@ __global__ __launch_bounds__(W * 64, 1) void gemm_kernel(
                        i % F::loads);
     };
 
-    // DMA: instruction J = wave * DMAS + j covers tokens 2J, 2J + 1 of the tile; lane L
-    // fills LDS chunk L % 32 of token 2J + L / 32 from logical chunk (L % 32) ^ (token % 16)
-    unsigned xlane[8];  // per J % 8 (the swizzle repeats every 16 tokens)
+    // DMA: instruction J = W j + wave covers tokens 2J, 2J + 1 of the tile; lane L fills LDS
+    // chunk L % 32 of token 2J + L / 32 from logical chunk (L % 32) ^ (token % 16).  The
+    // wavefronts take turns, so that a wavefront's tokens repeat every 8 / W of its
+    // instructions, 16 tokens on, and so does the swizzle.
+    constexpr int kTurn = 8 / W;
+    unsigned xlane[kTurn];
 #pragma unroll
-    for (int jm = 0; jm < 8; ++jm) {
-        const unsigned tok = kDmaRows * jm + lane / 32;
+    for (int jm = 0; jm < kTurn; ++jm) {
+        const unsigned tok = kDmaRows * (W * jm + wave) + lane / 32;
         xlane[jm] = unsigned(tok * row_pitch) + 16 * ((lane % 32) ^ tok);
     }
     const auto x_rsrc = activation_resource(xs + size_t(m0) * k);
     auto stage_one = [&](unsigned g, unsigned buf, int j) {
-        const unsigned J = wave * DMAS + j;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            x_rsrc, (lds_void*)(lds + buf * SB + J * 1024), 16, int(xlane[J % 8]),
-            int(g * 512 + (J / 8) * (16 * unsigned(row_pitch))), 0, 0);
+            x_rsrc, (lds_void*)(lds + buf * SB + (W * j + wave) * 1024), 16,
+            int(xlane[j % kTurn]),
+            int(g * 512 + unsigned(j / kTurn) * (16 * unsigned(row_pitch))), 0, 0);
     };
     constexpr int kLoads = DMAS + F::loads * NBW, kPerStep = 4;
     static_assert(kLoads <= 16 * kPerStep, "the loads must fit the group's sub-steps");
@@ -1011,8 +1015,10 @@ int configure() {
                               reinterpret_cast<const void*>(many)})
             KDQ_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
                                         128 * 1024));
-        KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<ENC, W>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds)));
+        KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<ENC, W, 3>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds<3>)));
+        KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<ENC, W, 4>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds<4>)));
         for (const void* f : {reinterpret_cast<const void*>(&stream_gemm_kernel<ENC, false>),
                               reinterpret_cast<const void*>(&stream_gemm_kernel<ENC, true>)})
             KDQ_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1135,8 +1141,14 @@ int launch_gemm(const float* x, const uint8_t* packed, size_t m, size_t n, size_
     } else {
         constexpr int W = gemm_waves<ENC>;
         const size_t tiles = (m + PM - 1) / PM * (((n + 15) / 16 + kTiles - 1) / kTiles) * slices;
-        auto kernel = gemm_kernel<ENC, W>;
-        hipLaunchKernelGGL(kernel, dim3(unsigned((tiles + 7) / 8 * 8)), dim3(W * 64), kLds, st,
+        // 65 to 96 rows leave a fourth 32-token block empty: without its products 77 x 14336 ->
+        // 4096 takes 32.8 us in place of 34.2 (Q6_K), 30.5 of 33.5 (Q4_K) and 34.1 of 37.4
+        // (Q8_0).  Longer chunks keep 128-token tiles, which read the weights once per four
+        // blocks.
+        const bool three = m <= 96;
+        auto kernel = three ? gemm_kernel<ENC, W, 3> : gemm_kernel<ENC, W, 4>;
+        hipLaunchKernelGGL(kernel, dim3(unsigned((tiles + 7) / 8 * 8)), dim3(W * 64),
+                           three ? kLds<3> : kLds<4>, st,
                            xs, sigma, packed, unsigned(m), unsigned(n), unsigned(k), slices, per,
                            y, part, status);
         KDQ_HIP(hipGetLastError());

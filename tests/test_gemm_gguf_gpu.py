@@ -70,6 +70,15 @@ def test_gemm_short_chunks(device, oracle, enc, m, k, n):
 
 
 @pytest.mark.parametrize("enc", ENCODINGS)
+@pytest.mark.parametrize("m,k,n", [(66, 256, 16), (80, 4608, 272), (95, 768, 513),
+                                   (96, 1024, 256), (97, 1280, 130), (128, 768, 300)])
+def test_gemm_three_block_tile(device, oracle, enc, m, k, n):
+    """The 96-token tile and its edges to the 128-token one: one group and several, an odd
+    count, K slices (the deeper k), partial weight tiles."""
+    run(device, oracle, enc, m, k, n, seed=0x3B + m + n)
+
+
+@pytest.mark.parametrize("enc", ENCODINGS)
 @pytest.mark.parametrize("k,n", [(4096, 14336), (14336, 4096)])
 def test_gemm_prefill_chunk(device, oracle, enc, k, n):
     """A 512-token prefill chunk (IW/src/models/text/gguf_engine.cpp:16) at Llama-3-8B's
