@@ -410,10 +410,10 @@ __device__ __forceinline__ auto activation_resource(const uint16_t* xs) {
                                              0x00027000);
 }
 
-// Workgroup tile: 32 TB tokens (128; 96 where they hold every token) x 256 weight rows (16
-// packed tiles); wavefront w owns tiles 4w .. 4w + 3 as two 32-row operands.  K runs over
-// 256-value groups; each group's tokens x 512 bytes of permuted activations are staged into LDS by 16-byte DMA
-// (double-buffered, one group ahead), chunk q of token t at t*512 + 16*(q ^ (t % 16)),
+// Workgroup tile: 32 TB tokens (96 or 128, launch_gemm) x 256 weight rows (16 packed
+// tiles); wavefront w owns tiles 4w .. 4w + 3 as two 32-row operands.  K runs over
+// 256-value groups; each group's tokens x 512 bytes of permuted activations are staged into
+// LDS by 16-byte DMA (double-buffered, one group ahead), chunk q of token t at t*512 + 16*(q ^ (t % 16)),
 // and the next group's weight registers load during the current group's sub-steps.
 // `xs` has rows up to the next multiple of 128 tokens (rows past m are computed, never
 // stored).  *status |= 1 for a non-finite weight scale, |= 2 when a dequantised weight
@@ -1141,11 +1141,12 @@ int launch_gemm(const float* x, const uint8_t* packed, size_t m, size_t n, size_
     } else {
         constexpr int W = gemm_waves<ENC>;
         const size_t tiles = (m + PM - 1) / PM * (((n + 15) / 16 + kTiles - 1) / kTiles) * slices;
-        // 65 to 96 rows leave a fourth 32-token block empty: without its products 77 x 14336 ->
-        // 4096 takes 32.8 us in place of 34.2 (Q6_K), 30.5 of 33.5 (Q4_K) and 34.1 of 37.4
-        // (Q8_0).  Longer chunks keep 128-token tiles, which read the weights once per four
-        // blocks.
-        const bool three = m <= 96;
+        // Tiles of three 32-token blocks where no more of them are needed than of four (up to 96
+        // rows, 129 to 192, 257 to 288): they multiply less padding for the same reads of the
+        // weights.  Four blocks and three, Q6_K / Q4_K / Q8_0: 77 x 14336 -> 4096 34.2 -> 32.8,
+        // 33.5 -> 30.5, 37.4 -> 34.1 us; 150 x 4096 -> 14336 47 -> 44.5, 42.0 -> 37.9, 46.2 ->
+        // 41.2; 288 (Q8_0 270) x 4096 -> 14336 64.6 -> 61.9, 55.3 -> 47.3, 59.6 -> 53.5.
+        const bool three = (m + 95) / 96 == (m + PM - 1) / PM;
         auto kernel = three ? gemm_kernel<ENC, W, 3> : gemm_kernel<ENC, W, 4>;
         hipLaunchKernelGGL(kernel, dim3(unsigned((tiles + 7) / 8 * 8)), dim3(W * 64),
                            three ? kLds<3> : kLds<4>, st,

@@ -71,10 +71,12 @@ def test_gemm_short_chunks(device, oracle, enc, m, k, n):
 
 @pytest.mark.parametrize("enc", ENCODINGS)
 @pytest.mark.parametrize("m,k,n", [(66, 256, 16), (80, 4608, 272), (95, 768, 513),
-                                   (96, 1024, 256), (97, 1280, 130), (128, 768, 300)])
+                                   (96, 1024, 256), (97, 1280, 130), (128, 768, 300),
+                                   (192, 512, 130), (193, 768, 272), (257, 1280, 96),
+                                   (288, 512, 257), (289, 768, 130)])
 def test_gemm_three_block_tile(device, oracle, enc, m, k, n):
-    """The 96-token tile and its edges to the 128-token one: one group and several, an odd
-    count, K slices (the deeper k), partial weight tiles."""
+    """The 96-token tile, one to three of them, and its edges to the 128-token one: one group
+    and several, an odd count, K slices (the deeper k), partial weight tiles."""
     run(device, oracle, enc, m, k, n, seed=0x3B + m + n)
 
 
