@@ -168,7 +168,8 @@ int kdq_gemv_packed_supported(int encoding, size_t in);
  * Activations: fp16 [m x k] quantized per 32 to int8 with an fp32 scale
  * (amax/127, codes round-half-even(x*127/amax), G/src/ggml-cpu/arch/x86/quants.c:302-398).
  * y[m x n] fp16 = sum_b float(sumi_b) * d_w * d_x, fp32 accumulation.
- * k % 256 == 0; any m, n >= 1. */
+ * k % 256 == 0; any m, n >= 1.  Weights of up to 256 MiB are packed into the library's
+ * workspace first, on each call, where that is faster (and its memory can be had). */
 int kdq_gemm_q4_0(const void* weights, size_t n, size_t k, const uint16_t* x_f16, size_t m,
                   uint16_t* y_f16, void* stream);
 
@@ -176,8 +177,9 @@ int kdq_gemm_q4_0(const void* weights, size_t n, size_t k, const uint16_t* x_f16
  * the decode product kdq_gemv_packed reads, so one resident copy serves decode and
  * prefill): `packed` holds kdq_gguf_packed_bytes(KDQ_Q4_0, k, n) bytes, 16-byte
  * aligned.  Same semantics as kdq_gemm_q4_0 (same activation quantisation, fp16
- * products of fp16(code * d_x) and fp16((q - 8) * d_w), fp32 accumulation); results
- * may differ from kdq_gemm_q4_0 in the last fp32 bits (summation order). */
+ * products of fp16(code * d_x) and fp16((q - 8) * d_w), fp32 accumulation); where
+ * kdq_gemm_q4_0 multiplies its rows as they lie, results may differ from it in the last
+ * fp32 bits (summation order). */
 int kdq_gemm_q4_0_packed(const void* packed, size_t n, size_t k, const uint16_t* x_f16,
                          size_t m, uint16_t* y_f16, void* stream);
 

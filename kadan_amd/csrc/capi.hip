@@ -45,6 +45,7 @@ void* workspace(size_t bytes, int* status) {
         }
         size_t grown = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
         if (hipMalloc(&w.ptr, grown) != hipSuccess) {
+            (void)hipGetLastError();  // reported here: not the next launch's error
             w.ptr = nullptr;
             *status = KDQ_ERR_SCRATCH;
             return nullptr;

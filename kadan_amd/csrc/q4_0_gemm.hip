@@ -18,8 +18,8 @@
 //                    consume them, so no LDS traffic is spent on weights.
 //   sum_kernel       the K slices of outputs too narrow for the compute units, summed in
 //                    slice order
-// Row-major weights are packed into the workspace first: the pass (33 MB at 4096 -> 14336)
-// costs less than multiplying them from rows did (weights through LDS, 128 x 128 tiles).
+//   rows_kernel      the product over row-major weights as they lie (weights through LDS,
+//                    128 x 128 tiles), where packing them first costs more (pack_first)
 #include "kdq_common.hpp"
 
 #include <algorithm>
@@ -98,6 +98,173 @@ __global__ __launch_bounds__(256) void quantize_kernel(const uint16_t* __restric
     }
     if (d && (t & 3) == 0)
         d[e / 32] = scale;
+}
+
+// ---------------------------------------------------- GEMM over rows as they lie
+
+constexpr int BM = 128, BN = 128, BK = 64;
+constexpr int kRowPitch = BK + 8;  // fp16 per LDS row (144 bytes: conflict-free fragment reads)
+
+// 32 Q4_0 values (one block) -> 16 fp16x2 words of round((q - 8) * d).
+// `codes` are the 16 code bytes as four dwords; values j and j+16 share byte j.
+__device__ __forceinline__ void dequant_q4_0(const unsigned codes[4], unsigned d_bits,
+                                             unsigned out[16]) {
+    const f16x2 scale = __builtin_bit_cast(f16x2, d_bits | (d_bits << 16));
+    const f16x2 bias = __builtin_bit_cast(f16x2, 0x64086408u);  // (1032, 1032)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const unsigned w = codes[i];
+        // bytes (b0, b1) -> positions (0, 16) and (b2, b3) -> (0, 16)
+        const unsigned lo01 = __builtin_amdgcn_perm(0u, w, 0x0c010c00u);
+        const unsigned lo23 = __builtin_amdgcn_perm(0u, w, 0x0c030c02u);
+        const unsigned q[4] = {(lo01 & 0x000f000fu) | 0x64006400u,
+                               (lo23 & 0x000f000fu) | 0x64006400u,
+                               ((lo01 >> 4) & 0x000f000fu) | 0x64006400u,
+                               ((lo23 >> 4) & 0x000f000fu) | 0x64006400u};
+        f16x2 r[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            r[k] = (__builtin_bit_cast(f16x2, q[k]) - bias) * scale;  // exact (q-8), one rounding
+        // values: 4i, 4i+1 (lo01), 4i+2, 4i+3 (lo23), 16+4i.. (high nibbles)
+        out[2 * i] = __builtin_bit_cast(unsigned, r[0]);
+        out[2 * i + 1] = __builtin_bit_cast(unsigned, r[1]);
+        out[8 + 2 * i] = __builtin_bit_cast(unsigned, r[2]);
+        out[8 + 2 * i + 1] = __builtin_bit_cast(unsigned, r[3]);
+    }
+}
+
+struct Stage {
+    u32x4 a[4];     // 32 activation values (fp16)
+    unsigned w[5];  // 20 bytes covering one Q4_0 block
+};
+
+// 128 x 128 output tile per 256-thread workgroup (4 wavefronts of 64 x 64), k in steps of
+// 64 through double-buffered LDS: activations copied, weights dequantised once per tile.  A
+// workgroup's chain over k bounds it (14 us per 1024 values until the tiles are more than
+// about 1.3 per compute unit), then the LDS passage of the weights: 64 x 4096 -> 131072
+// 191 us, 1.6 TB/s of weights.
+__global__ __launch_bounds__(256) void rows_kernel(const uint16_t* __restrict__ a,
+                                                   const uint8_t* __restrict__ w, unsigned m,
+                                                   unsigned n, unsigned k,
+                                                   uint16_t* __restrict__ y) {
+    __shared__ __align__(16) uint16_t lds_a[2][BM * kRowPitch];
+    __shared__ __align__(16) uint16_t lds_b[2][BN * kRowPitch];
+
+    // XCD-aware tile order: the M tiles of one N tile run back to back on one XCD.
+    const unsigned m_tiles = (m + BM - 1) / BM, n_tiles = (n + BN - 1) / BN;
+    const unsigned id = blockIdx.x, xcd = id % 8, local = id / 8;
+    const unsigned per_xcd = (n_tiles * m_tiles + 7) / 8;
+    const unsigned linear = xcd * per_xcd + local;  // contiguous chunk per XCD
+    if (local >= per_xcd || linear >= n_tiles * m_tiles)
+        return;
+    const unsigned n_tile = linear / m_tiles, m_tile = linear % m_tiles;
+    const unsigned m0 = m_tile * BM, n0 = n_tile * BN;
+
+    const unsigned tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+    const size_t row_bytes = size_t(k / 32) * 18;
+
+    // global -> register staging: thread t copies activation row t/2, values
+    // 32*(t%2) .. +31 of the 64-value step, and dequantises block t%2 of weight row t/2.
+    const unsigned ar = tid / 2, ah = tid % 2;
+    const bool a_ok = m0 + ar < m, b_ok = n0 + ar < n;
+    const uint16_t* a_src = a + size_t(m0 + (a_ok ? ar : 0)) * k + 32 * ah;
+    const uint8_t* b_src = w + size_t(n0 + (b_ok ? ar : 0)) * row_bytes + (ah ? 16 : 0);
+
+    auto load = [&](unsigned step, Stage& s) {
+        const uint16_t* pa = a_src + size_t(step) * BK;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            s.a[i] = a_ok ? *reinterpret_cast<const u32x4*>(pa + 8 * i) : u32x4{0, 0, 0, 0};
+        const uint8_t* p = b_src + size_t(step) * 36;
+        if (b_ok) {
+            const u32x4 v = load16(p);
+            s.w[0] = v.x, s.w[1] = v.y, s.w[2] = v.z, s.w[3] = v.w;
+            s.w[4] = load4(p + 16);
+        } else {
+            s.w[0] = s.w[1] = s.w[2] = s.w[3] = s.w[4] = 0;
+        }
+    };
+    auto store = [&](unsigned buf, const Stage& s) {
+        uint16_t* da = lds_a[buf] + ar * kRowPitch + 32 * ah;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<u32x4*>(da + 8 * i) = s.a[i];
+        unsigned codes[4], d_bits;
+        if (ah == 0) {  // block at byte 0: d in bytes 0-1, codes at bytes 2..17
+            d_bits = s.w[0] & 0xffffu;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                codes[i] = __builtin_amdgcn_alignbyte(s.w[i + 1], s.w[i], 2);
+        } else {  // loaded from byte 16: d in bytes 18-19, codes at bytes 20..35
+            d_bits = s.w[0] >> 16;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                codes[i] = s.w[i + 1];
+        }
+        unsigned vals[16];
+        dequant_q4_0(codes, d_bits, vals);
+        uint16_t* db = lds_b[buf] + ar * kRowPitch + 32 * ah;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<u32x4*>(db + 8 * i) =
+                u32x4{vals[4 * i], vals[4 * i + 1], vals[4 * i + 2], vals[4 * i + 3]};
+    };
+
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            acc[i][j] = f32x16{};
+
+    const unsigned wm = (wave / 2) * 64, wn = (wave % 2) * 64;
+    const unsigned frag_row = lane % 32, frag_k = 8 * (lane / 32);
+    const unsigned steps = k / BK;
+
+    Stage s;
+    load(0, s);
+    store(0, s);
+    __syncthreads();
+
+    for (unsigned step = 0; step < steps; ++step) {
+        const unsigned buf = step & 1;
+        const bool more = step + 1 < steps;
+        if (more)
+            load(step + 1, s);
+#pragma unroll
+        for (unsigned ks = 0; ks < BK; ks += 16) {
+            f16x8 af[2], bf[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                af[i] = *reinterpret_cast<const f16x8*>(
+                    lds_a[buf] + (wm + 32 * i + frag_row) * kRowPitch + ks + frag_k);
+                bf[i] = *reinterpret_cast<const f16x8*>(
+                    lds_b[buf] + (wn + 32 * i + frag_row) * kRowPitch + ks + frag_k);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
+        }
+        if (more)
+            store(buf ^ 1, s);
+        __syncthreads();
+    }
+
+    // C fragment: lane holds column lane%32, rows 8*(v/4) + 4*(lane/32) + v%4.
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const unsigned col = n0 + wn + 32 * j + lane % 32;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const unsigned row = m0 + wm + 32 * i + 8 * (v / 4) + 4 * (lane / 32) + v % 4;
+                if (row < m && col < n)
+                    y[size_t(row) * n + col] = __builtin_bit_cast(uint16_t, _Float16(acc[i][j][v]));
+            }
+        }
 }
 
 // ------------------------------------------------- GEMM over tile-packed weights
@@ -491,6 +658,28 @@ int launch_tiles(const Plan& p, const uint16_t* xs, const uint8_t* w, unsigned m
     return KDQ_OK;
 }
 
+// Whether row-major weights are packed into the workspace and multiplied from there.  That
+// costs a launch and the weights' bytes twice more; rows_kernel costs a chain over k and,
+// beyond about one tile a compute unit, the weights' passage through LDS.  So it is
+// rows_kernel for
+// - short k: 64 x 256 -> 14336 10.3 us, packed 16.0;
+// - outputs so wide that every compute unit has a tile (every second or third one where k,
+//   and with it the chain, is short), and few enough tokens that the weights are not
+//   dequantised often: 64 x 4096 -> 131072 191 us, packed 264; 64 x 768 -> 32768 18 and 22;
+//   129 x 4096 -> 28672 81 and 93.  But 384 x 4096 -> 65536 281 and 262, 64 x 4096 -> 14336
+//   66 and 43, 129 x 1024 -> 8192 (128 tiles, 64 of them side by side) 22 and 17;
+// - matrices whose copy would pass kPackLimit: a call holds no second copy of a large one.
+constexpr size_t kPackLimit = size_t(256) << 20;
+
+bool pack_first(size_t m, size_t n, size_t k) {
+    const size_t m_tiles = (m + BM - 1) / BM, n_tiles = (n + BN - 1) / BN;
+    const size_t filled = compute_units() * std::min<size_t>(k, 2048);  // in 2048ths
+    const bool wide = m_tiles * n_tiles * 2048 >= filled && n_tiles * 2048 * 4 >= filled * 3;
+    if (k <= 512 || (wide && m <= (k <= 1024 ? 512 : 256)))
+        return false;
+    return kdq_gguf_packed_bytes(KDQ_Q4_0, k, n) <= kPackLimit;
+}
+
 template <bool PERMUTED = false>
 int launch_quantize(const uint16_t* x, size_t m, size_t k, int8_t* q, float* d,
                     uint16_t* dequant, hipStream_t stream) {
@@ -552,16 +741,27 @@ extern "C" int kdq_gemm_q4_0(const void* weights, size_t n, size_t k, const uint
         overlaps(y_f16, m * n * 2, weights, n * (k / 32) * 18))
         return KDQ_ERR_ALIAS;
     int rc;
-    const Plan p = plan_of(m, n, k);
-    const size_t packed_bytes = kdq_gguf_packed_bytes(KDQ_Q4_0, k, n);
-    const size_t at = (p.total + 255) & ~size_t(255);
-    auto* base = static_cast<uint8_t*>(workspace(at + packed_bytes, &rc));
-    if (rc)
+    auto st = static_cast<hipStream_t>(stream);
+    if (pack_first(m, n, k)) {
+        const Plan p = plan_of(m, n, k);
+        const size_t at = (p.total + 255) & ~size_t(255);
+        auto* base = static_cast<uint8_t*>(
+            workspace(at + kdq_gguf_packed_bytes(KDQ_Q4_0, k, n), &rc));
+        if (rc != KDQ_ERR_SCRATCH) {  // (no memory for the copy: from the rows)
+            if (rc || (rc = kdq_gguf_pack(KDQ_Q4_0, weights, (k / 32) * 18, k, n, base + at, st)))
+                return rc;
+            return run_packed(p, x_f16, base + at, m, n, k, y_f16, base, st);
+        }
+    }
+    auto* xs = static_cast<uint16_t*>(workspace(m * k * 2, &rc));
+    if (rc || (rc = launch_quantize(x_f16, m, k, nullptr, nullptr, xs, st)))
         return rc;
-    uint8_t* packed = base + at;
-    if ((rc = kdq_gguf_pack(KDQ_Q4_0, weights, (k / 32) * 18, k, n, packed, stream)))
-        return rc;
-    return run_packed(p, x_f16, packed, m, n, k, y_f16, base, static_cast<hipStream_t>(stream));
+    const unsigned tiles = unsigned(((m + BM - 1) / BM) * ((n + BN - 1) / BN));
+    hipLaunchKernelGGL(rows_kernel, dim3((tiles + 7) / 8 * 8), dim3(256), 0, st, xs,
+                       static_cast<const uint8_t*>(weights), unsigned(m), unsigned(n),
+                       unsigned(k), y_f16);
+    KDQ_HIP(hipGetLastError());
+    return KDQ_OK;
 }
 
 extern "C" int kdq_gemm_q4_0_packed(const void* packed, size_t n, size_t k, const uint16_t* x_f16,

@@ -134,3 +134,53 @@ def test_gemm_q4_0_packed_baseline_shape_property(device, oracle):
     got = out.float().cpu().numpy()
     assert_close(got[:100], y[:100], rel=1e-6, mabs=1e-5, what="first 100 tokens")
     assert (got[100:] == 7.0).all()
+
+
+def _rows_case(device, m, k, n):
+    torch = _torch()
+    w = synth.q4_0_weights(m + k + n, n, k)
+    x = synth.normal(m + k + n, 9, m * k).reshape(m, k).astype(np.float16)
+    return w, x, torch.from_numpy(w).to(device), torch.from_numpy(x).to(device)
+
+
+@pytest.mark.parametrize("m,k,n,packs", [
+    (1, 512, 300, False), (64, 512, 12288, False), (513, 256, 640, False),   # short rows
+    (1, 768, 12161, False), (64, 1024, 16384, False), (300, 768, 9217, False),  # wide outputs
+    (200, 2048, 24449, False), (5, 2304, 32641, False),
+    (9, 768, 1000, True), (64, 768, 12160, True), (300, 768, 9088, True),    # packed first:
+    (200, 2048, 24448, True), (70, 2304, 300, True)])                        # K slices or none
+def test_gemm_q4_0_rows_packed_first_or_not(device, oracle, m, k, n, packs):
+    """Both ways that row-major weights take, at the edges of the rule between them: against
+    the oracle on a sample of columns, and, packed first, the bits of kdq_gemm_q4_0_packed."""
+    torch = _torch()
+    from kadan_amd import ops
+    w, x, wd, xd = _rows_case(device, m, k, n)
+    y = torch.full((m, n), float("nan"), dtype=torch.float16, device=device)
+    ops.gemm_q4_0(wd, xd, n, out=y)
+    assert torch.isfinite(y).all(), "an output element was not written"
+    cols = np.unique(np.concatenate([np.arange(0, n, max(1, n // 150)), [n - 1]]))
+    xq, xs = oracle.quantize_q8_f16(x.view(np.uint16))
+    want = oracle.gemm_q4_0_q8(np.ascontiguousarray(w[cols]), cols.size, k, xq, xs)
+    assert_close(y.float().cpu().numpy()[:, cols], want, what=f"rows gemm m={m} k={k} n={n}")
+    if packs:
+        packed = ops.gemm_q4_0_packed(ops.gguf_pack(2, wd, k), xd, n)
+        assert torch.equal(y.view(torch.int16), packed.view(torch.int16))
+
+
+@pytest.mark.parametrize("m,k,n", [(4, 4096, 131072), (300, 8192, 65536)])
+def test_gemm_q4_0_rows_holds_no_copy_of_large_weights(device, m, k, n):
+    """302 MB of row-major weights: the workspace holds the activations, no second copy."""
+    torch = _torch()
+    import kadan_amd
+    from kadan_amd import ops
+    w = torch.zeros(n, k // 32 * 18, dtype=torch.uint8, device=device)
+    x = torch.ones(m, k, dtype=torch.float16, device=device)
+    y = torch.full((m, n), 1.0, dtype=torch.float16, device=device)
+    ops.gemm_q4_0(w[:16], x[:1].contiguous(), 16)  # the kernels are loaded
+    kadan_amd.call("kdq_release_scratch")
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    ops.gemm_q4_0(w, x, n, out=y)
+    torch.cuda.synchronize()
+    assert before - torch.cuda.mem_get_info()[0] < 64 << 20
+    assert not y.any()  # d = 0
