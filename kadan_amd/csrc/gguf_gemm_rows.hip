@@ -459,7 +459,8 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(const float* __restrict
 // narrow to fill the compute units): slice `ks` runs groups [ks * per, (ks + 1) * per) and
 // writes its fp32 tile to part + ks * part_stride (m x n, already scaled back by sigma, a
 // power of two: exact), summed in slice order by slice_sum_kernel.
-template <int ENC, int TB>
+// AHEAD: a step decodes the weights of the next one (decodes_ahead).
+template <int ENC, int TB, bool AHEAD>
 __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
     const uint16_t* __restrict__ xs, const float* __restrict__ sigma,
     const uint8_t* __restrict__ w, size_t row_bytes, const uint8_t* __restrict__ tail,
@@ -555,9 +556,8 @@ __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
 
     // Software pipeline, one barrier per step.  The top of step s refills the LDS buffers
     // that step s - 1 finished reading: activations of step s + 1 (from a register ring,
-    // loaded kAhead steps earlier) and, on a group's last step but one, the raw bytes of the next
-    // group (loaded a whole group earlier; stored a step early, as the weights are decoded one
-    // step ahead).  Each refill is followed at once by the load
+    // loaded kAhead steps earlier) and, on a group's last step (AHEAD: the last but one), the raw
+    // bytes of the next group (loaded a whole group earlier).  Each refill is followed at once by the load
     // that reuses its registers, so a store only ever waits on loads issued at least
     // kAhead steps (or one group) before.  The loop is unrolled by one turn of the ring, so
     // its register indices are constants; loads past the end re-read the last step or
@@ -586,50 +586,60 @@ __global__ __launch_bounds__(kThreads, 2) void rows_gemm_kernel(
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     const uint8_t* my_row0 = raw + (wave * 32 + r) * G::pitch;
-    // this lane's weights of step s: per 16-value sub-step values 8 h .. +7
-    auto decode = [&](unsigned s, f16x8 (&a)[2]) {
-        const unsigned g = s / PG, within = s % PG;
-        const uint8_t* row = my_row0 + (g % 2) * RN * G::pitch;
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-            a[sub] = RowsDecode<ENC>::run(row, within * RK + 16 * sub + 8 * h, flags, table);
+    // this lane's weights of sub-step `sub` of step s: values 16 sub + 8 h .. +7
+    auto decode = [&](unsigned s, int sub) {
+        const uint8_t* row = my_row0 + (s / PG % 2) * RN * G::pitch;
+        return RowsDecode<ENC>::run(row, s % PG * RK + 16 * sub + 8 * h, flags, table);
     };
-    // The weights are decoded one step ahead, so that the decode's VALU work and LDS reads run
-    // beside the products instead of before them (512 x 4096 -> 14336: IQ4_XS 111 -> 106 us,
-    // IQ4_NL 129 -> 124).
+    auto activations = [&](unsigned s, int sub, int b) {
+        const unsigned t = 32 * b + r, c = 2 * sub + h;  // 16-byte chunk of the token's 64 bytes
+        return *reinterpret_cast<const f16x8*>(xt + (s % 2) * RM * RK * 2 + t * 64 +
+                                               16 * (c ^ (((t >> 1) ^ (t >> 3)) & 3u)));
+    };
     f16x8 a[2];
-    decode(0, a);
+    if constexpr (AHEAD) {
+        a[0] = decode(0, 0);
+        a[1] = decode(0, 1);
+    }
     auto step = [&]<int U>(unsigned s) {  // U = s % kUnroll
         constexpr int slot = (U + 1) % kAhead;
         const unsigned g = s / PG, within = s % PG;
         store_x((s + 1) % 2, xv[slot]);
         load_x(min(s + 1 + kAhead, steps - 1), xv[slot]);
-        if (within == PG - 2) {  // the last step decodes the next group's first weights
+        if (within == PG - (AHEAD ? 2 : 1)) {  // before the next group's first decode
             store_raw((g + 1) % 2, rv);
             load_raw(min(g + 2, groups - 1), rv);
         }
-        const uint8_t* xb = xt + (s % 2) * RM * RK * 2;
-        f16x8 xf[2][TB];
+        if constexpr (AHEAD) {
+            f16x8 xf[2][TB];
 #pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-            const unsigned c = 2 * sub + h;  // 16-byte chunk of the token's 64 bytes
+            for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
-            for (int b = 0; b < TB; ++b) {
-                const unsigned t = 32 * b + r;
-                xf[sub][b] = *reinterpret_cast<const f16x8*>(
-                    xb + t * 64 + 16 * (c ^ (((t >> 1) ^ (t >> 3)) & 3u)));
+                for (int b = 0; b < TB; ++b)
+                    xf[sub][b] = activations(s, sub, b);
+            // (BF16, which has little to decode meanwhile: every read ahead of the products, 119
+            // -> 114 us at 512 x 4096 -> 14336; 2-4 % slower for the others)
+            if constexpr (ENC == KDQ_BF16)
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+                for (int b = 0; b < TB; ++b)
+                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[sub], xf[sub][b], acc[b], 0,
+                                                                    0, 0);
+#pragma unroll
+            for (int sub = 0; sub < 2; ++sub)  // beside the products
+                a[sub] = decode(min(s + 1, steps - 1), sub);
+        } else {
+#pragma unroll
+            for (int sub = 0; sub < 2; ++sub) {
+                const f16x8 w8 = decode(s, sub);
+#pragma unroll
+                for (int b = 0; b < TB; ++b)
+                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w8, activations(s, sub, b),
+                                                                    acc[b], 0, 0, 0);
             }
         }
-        // (BF16, which has little to decode meanwhile: every read ahead of the products, 119 ->
-        // 114 us at 512 x 4096 -> 14336; 2-4 % slower for the others)
-        if constexpr (ENC == KDQ_BF16)
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-            for (int b = 0; b < TB; ++b)
-                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[sub], xf[sub][b], acc[b], 0, 0, 0);
-        decode(min(s + 1, steps - 1), a);  // beside the products
         __syncthreads();
     };
     unsigned s = 0;
@@ -752,20 +762,48 @@ RowsScratch rows_scratch(size_t m, size_t n, size_t k, const RowsPlan& plan) {
     return s;
 }
 
+// Decoding a step ahead runs the decode's VALU work and LDS reads beside the products instead
+// of before them (512 x 4096 -> 14336: IQ4_XS 111 -> 106 us, IQ4_NL 129 -> 124, IQ3_XXS 130 ->
+// 115, BF16 127 -> 106).  Its registers cost some encodings, at 128 tokens, the third
+// workgroup of a compute unit.  Q3_K, which gains nothing in return (127 us both ways; 640
+// tokens 157, ahead 198), decodes in front.  A lattice encoding does where fewer rounds of
+// three to a unit outweigh it (a round of three takes 4/3 as long: IQ2_S 4096 -> 32768,
+// 300 tokens 170, ahead 183; 512 tokens 242, ahead 224); BF16 only in one such round over
+// short rows (300 tokens 768 -> 32768 40, ahead 46; 4096 -> 32768 191 and 190).
+template <int ENC, int TB> constexpr bool third_workgroup =
+    TB == 4 && (ENC == KDQ_Q3_K || ENC == KDQ_BF16 || lattice_rows_entries<ENC> != 0);
+
+template <int ENC, int TB> bool decodes_ahead(size_t workgroups, size_t k) {
+    if (!third_workgroup<ENC, TB>)
+        return true;
+    if (ENC == KDQ_Q3_K)
+        return false;
+    const size_t units = compute_units();
+    const size_t two = (workgroups + 2 * units - 1) / (2 * units);
+    const size_t three = (workgroups + 3 * units - 1) / (3 * units);
+    if (ENC == KDQ_BF16)
+        return k > 1024 || two == 1 || three > 1;
+    return 3 * two < 4 * three;
+}
+
 template <int ENC, int TB>
 int launch_rows_gemm(const uint8_t* w, size_t row_bytes, size_t n, size_t k, size_t m,
                      const RowsPlan& plan, const RowsScratch& s, const uint16_t* xs,
                      const float* sigma, const uint8_t* tail, float* part, float* y,
                      unsigned* status, hipStream_t st) {
-    static bool configured = false;  // one attribute call per instantiation
     constexpr size_t lds = rows_lds<ENC, TB>;
+    const auto front = rows_gemm_kernel<ENC, TB, !third_workgroup<ENC, TB>>;
+    const auto ahead = rows_gemm_kernel<ENC, TB, ENC != KDQ_Q3_K || TB != 4>;
+    static bool configured = false;  // attribute calls once per instantiation
     if (!configured) {
-        KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&rows_gemm_kernel<ENC, TB>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+        for (const void* f : {reinterpret_cast<const void*>(front),
+                              reinterpret_cast<const void*>(ahead)})
+            KDQ_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
         configured = true;
     }
     const size_t tiles = s.m_pad / (32 * TB) * ((n + RN - 1) / RN) * plan.slices;
-    hipLaunchKernelGGL((rows_gemm_kernel<ENC, TB>), dim3(unsigned((tiles + 7) / 8 * 8)),
+    hipLaunchKernelGGL((decodes_ahead<ENC, TB>(tiles, k) ? ahead : front),
+                       dim3(unsigned((tiles + 7) / 8 * 8)),
                        dim3(kThreads), lds, st, xs, sigma, w, row_bytes, tail,
                        unsigned(m), unsigned(n), unsigned(k), plan.slices, plan.per, y, part,
                        s.part_stride, status);

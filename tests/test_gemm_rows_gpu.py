@@ -58,6 +58,22 @@ def test_gemm_rows_token_tiles_and_odd_slices(device, oracle, enc, m, n):
     run(device, oracle, enc, m, 1280, n, seed=0x1A0 + enc + m)
 
 
+@pytest.mark.parametrize("enc", [Q3_K, IQ3_XXS, IQ3_S, IQ2_S, BF16])
+def test_gemm_rows_decode_in_front(device, oracle, enc):
+    """768 workgroups, one round of three to a compute unit: the lattice encodings and BF16
+    decode in front of the products there and a step ahead elsewhere, Q3_K always in front.  The
+    first columns of the one against a product of theirs alone, which has K slices (fp32 sums
+    of 512 values in parts: a few eps, 1e-6 allowed)."""
+    import torch
+    from kadan_amd import ops
+    m, k, n = 300, 512, 32768
+    y = run(device, oracle, enc, m, k, n, seed=0xB0 + enc, cols=64)
+    w = torch.from_numpy(synth.gguf_weights(enc, 0xB0 + enc, n, k)[:2048]).to(device)
+    x = torch.from_numpy(synth.normal(0xB0 + enc, 7, m * k).reshape(m, k)).to(device)
+    few = ops.gemm_rows(enc, w, x, 2048).cpu().numpy()  # 48 workgroups in K slices
+    assert_close(y[:, :2048], few, rel=1e-6, mabs=1e-5, what="one slice against several")
+
+
 def test_gemm_rows_bf16_k64(device, oracle):
     """BF16 stages 64-value groups: a k that is a multiple of 64 but not of 256."""
     run(device, oracle, BF16, 40, 192, 96, seed=0xA7)
