@@ -1093,7 +1093,14 @@ GemmPlan gemm_plan(int encoding, size_t m, size_t n, size_t k) {
         const size_t wt = encoding == KDQ_Q4_K ? stream_tiles<KDQ_Q4_K, false>
                                                : stream_tiles<KDQ_Q8_0, false>;
         const size_t tiles = (m + kStreamTM - 1) / kStreamTM * (((n + 15) / 16 + wt - 1) / wt);
-        const size_t ks = std::max<size_t>(1, 2 * compute_units() / tiles);
+        // K slices of two groups or more, as many as there are places for; none where their
+        // partials, written and read back, cost more than the idle places: a tile has two
+        // places and K is not very deep (64 x 1280 -> 65536 Q4_K 34.4 us in two slices, 23.2
+        // in one; 9 x 14336 -> 28672 Q6_K 82.0 and 92.7), or fewer than eight and K is short
+        // (64 x 768 -> 28672 Q6_K 22.3 and 13.0)
+        const size_t places = std::max<size_t>(1, 2 * compute_units() / tiles);
+        const bool whole = (places < 3 && groups < 32) || (places < 8 && groups <= 4);
+        const size_t ks = whole ? 1 : places;
         p.per = unsigned((groups + ks - 1) / ks);
         p.per = unsigned(std::min<size_t>(groups, std::max<size_t>(p.per, 2)));
     } else {

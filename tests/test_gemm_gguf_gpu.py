@@ -62,10 +62,11 @@ def test_gemm_small_shapes(device, oracle, enc, m, k, n):
 @pytest.mark.parametrize("enc", ENCODINGS)
 @pytest.mark.parametrize("m,k,n", [(31, 512, 144), (32, 768, 130), (33, 1024, 270),
                                    (63, 1280, 33), (64, 256, 128), (65, 512, 257),
-                                   (5, 2816, 1000)])
+                                   (5, 2816, 1000), (41, 768, 24590)])
 def test_gemm_short_chunks(device, oracle, enc, m, k, n):
     """Chunks of one 64-token tile, and just past it: one or two 32-token blocks, odd and
-    even group counts, partial weight tiles, and K slices (the deeper k)."""
+    even group counts, partial weight tiles, K slices (the deeper k), and a wide output of
+    short k without them."""
     run(device, oracle, enc, m, k, n, seed=0x5E + m + n)
 
 
