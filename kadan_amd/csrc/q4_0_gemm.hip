@@ -618,7 +618,9 @@ struct Plan {
 // K slices: where the output tiles are fewer than an eighth of the workgroups that fit, as
 // many slices as fit, at least two groups deep (64 x 4096 -> 14336: 43.6 -> 31.4 us;
 // 9 x 11776 -> 3387: 106 -> 21.6).  Above that line they gain less (100 x 4096 -> 14336:
-// 32.4) and would sum a row in another order than a longer chunk does.
+// 32.4) and would sum a row in another order than a longer chunk does; and up to 1024 values of
+// k their partials cost more than the idle units (64 x 768 -> 14336: 16.0 us in two slices, 11.4
+// in one).
 Plan plan_of(size_t m, size_t n, size_t k) {
     Plan p;
     const size_t units = compute_units(), groups = k / 256;
@@ -626,7 +628,7 @@ Plan plan_of(size_t m, size_t n, size_t k) {
     p.blocks = m <= 32 ? 1 : (m + 127) / 128 * wtiles * 2 > units ? 4 : 2;
     const size_t tokens = 32 * size_t(p.blocks), tiles = (m + tokens - 1) / tokens * wtiles;
     const size_t slots = units * (p.blocks == 4 ? 1 : 2);
-    const size_t want = tiles * 8 > slots ? 1 : slots / tiles;
+    const size_t want = tiles * 8 > slots || groups <= 4 ? 1 : slots / tiles;
     p.per = unsigned(std::min(groups, std::max<size_t>(2, (groups + want - 1) / want)));
     p.slices = unsigned((groups + p.per - 1) / p.per);
     p.pitch = unsigned((n + 3) / 4 * 4);

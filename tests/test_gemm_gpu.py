@@ -147,8 +147,8 @@ def _rows_case(device, m, k, n):
     (1, 512, 300, False), (64, 512, 12288, False), (513, 256, 640, False),   # short rows
     (1, 768, 12161, False), (64, 1024, 16384, False), (300, 768, 9217, False),  # wide outputs
     (200, 2048, 24449, False), (5, 2304, 32641, False),
-    (9, 768, 1000, True), (64, 768, 12160, True), (300, 768, 9088, True),    # packed first:
-    (200, 2048, 24448, True), (70, 2304, 300, True)])                        # K slices or none
+    (9, 768, 1000, True), (64, 768, 12160, True), (300, 768, 9088, True),    # packed first,
+    (200, 2048, 24448, True), (70, 2304, 300, True)])                        # K whole or sliced
 def test_gemm_q4_0_rows_packed_first_or_not(device, oracle, m, k, n, packs):
     """Both ways that row-major weights take, at the edges of the rule between them: against
     the oracle on a sample of columns, and, packed first, the bits of kdq_gemm_q4_0_packed."""
