@@ -147,14 +147,9 @@ def check(function: str, status: int) -> None:
     raise KdqError(function, status, hip)
 
 
-_functions: dict[str, C._CFuncPtr] = {}  # the entry points called so far
-
-
 def call(function: str, *args) -> None:
-    fn = _functions.get(function)
-    if fn is None:
-        fn = _functions[function] = getattr(lib(), function)
-    status = fn(*args)
+    # (the handle keeps its entry points as attributes: nothing is kept beside it)
+    status = getattr(_lib or lib(), function)(*args)
     if status:
         check(function, status)
 

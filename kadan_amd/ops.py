@@ -84,8 +84,13 @@ def gemv_batch(jobs: list[dict]) -> None:
 
 
 @functools.lru_cache(maxsize=4096, typed=True)  # (256.0 is refused, also after 256)
-def gguf_packed_bytes(encoding: int, n_in: int, n_out: int) -> int:
+def _packed_bytes(encoding: int, n_in: int, n_out: int) -> int:
     return int(lib().kdq_gguf_packed_bytes(encoding, n_in, n_out))
+
+
+def gguf_packed_bytes(encoding: int, n_in: int, n_out: int) -> int:
+    lib()  # (raises where the library is missing, also for a size asked before)
+    return _packed_bytes(encoding, n_in, n_out)
 
 
 def gguf_pack(encoding: int, weights: torch.Tensor, n_in: int) -> torch.Tensor:
@@ -110,7 +115,7 @@ def gemv_packed(encoding: int, packed: torch.Tensor, x: torch.Tensor, n_out: int
     _need(x, torch.float32, "x")
     x2 = _rows(x)
     rows, n_in = x2.shape
-    if packed.numel() != gguf_packed_bytes(encoding, n_in, n_out):
+    if packed.numel() != _packed_bytes(encoding, n_in, n_out):
         raise ValueError("packed size does not match (encoding, n_in, n_out)")
     if out is None:
         out = torch.empty(rows, n_out, dtype=torch.float32, device=x.device)
@@ -165,7 +170,7 @@ def gemm_q4_0_packed(packed: torch.Tensor, x_f16: torch.Tensor, n_out: int,
     _need(packed, torch.uint8, "packed")
     _need(x_f16, torch.float16, "x")
     m, k = x_f16.shape
-    if packed.numel() != gguf_packed_bytes(2, k, n_out):  # KDQ_Q4_0
+    if packed.numel() != _packed_bytes(2, k, n_out):  # KDQ_Q4_0
         raise ValueError("packed size does not match (k, n_out)")
     if out is None:
         out = torch.empty(m, n_out, dtype=torch.float16, device=x_f16.device)
@@ -182,7 +187,7 @@ def gemm_packed(encoding: int, packed: torch.Tensor, x: torch.Tensor, n_out: int
     _need(packed, torch.uint8, "packed")
     _need(x, torch.float32, "x")
     m, k = x.shape
-    if packed.numel() != gguf_packed_bytes(encoding, k, n_out):
+    if packed.numel() != _packed_bytes(encoding, k, n_out):
         raise ValueError("packed size does not match (k, n_out)")
     if out is None:
         out = torch.empty(m, n_out, dtype=torch.float32, device=x.device)

@@ -126,6 +126,22 @@ def test_product_path_has_no_cpu_fallback(monkeypatch, tmp_path):
         kadan_amd.lib()
 
 
+def test_missing_library_is_noticed_after_earlier_calls(monkeypatch, tmp_path):
+    """Entry points and sizes used before do not stand in for a library that is gone."""
+    import kadan_amd
+    from kadan_amd import ops
+    assert kadan_amd.row_bytes(12, 256) == 144
+    assert ops.gguf_packed_bytes(12, 512, 16) == 4608
+    with pytest.raises(kadan_amd.KdqError):
+        kadan_amd.call("kdq_dequantize", 12, None, 144, 1, 256, None, None, None)
+    monkeypatch.setattr(kadan_amd, "LIBRARY", str(tmp_path / "missing.so"))
+    monkeypatch.setattr(kadan_amd, "_lib", None)
+    for use in (lambda: kadan_amd.call("kdq_dequantize", 12, None, 144, 1, 256, None, None, None),
+                lambda: ops.gguf_packed_bytes(12, 512, 16)):
+        with pytest.raises(RuntimeError, match="no CPU fallback"):
+            use()
+
+
 def test_packed_sizes_looked_up_once_still_refuse_a_float():
     import ctypes
     from kadan_amd import ops
