@@ -14,13 +14,16 @@ import torch
 from . import BLOCK_BYTES, BLOCK_VALUES, MatvecJob, call, lib
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # (not a public name)
+
+
 def _stream() -> int:
     """The current HIP stream.  A decode product takes 6-8 us on the device, so its wrapper must
-    not take longer: the raw handle, without the Stream object torch.cuda.current_stream()
-    builds."""
-    if not torch.cuda.is_initialized():
+    not take longer: the raw handle, where torch gives it, without the Stream object
+    torch.cuda.current_stream() builds."""
+    if _raw_stream is None or not torch.cuda.is_initialized():
         return torch.cuda.current_stream().cuda_stream
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:

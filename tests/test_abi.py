@@ -142,6 +142,18 @@ def test_missing_library_is_noticed_after_earlier_calls(monkeypatch, tmp_path):
             use()
 
 
+def test_stream_without_the_raw_handle(monkeypatch):
+    """A torch that does not give the raw handle: the public current stream."""
+    import types
+    import torch
+    from kadan_amd import ops
+    monkeypatch.setattr(ops, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream",
+                        lambda: types.SimpleNamespace(cuda_stream=77))
+    assert ops._stream() == 77
+
+
 def test_packed_sizes_looked_up_once_still_refuse_a_float():
     import ctypes
     from kadan_amd import ops
