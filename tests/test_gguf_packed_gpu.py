@@ -229,3 +229,51 @@ def test_gemv_long_rows_in_k_slices(device, oracle, enc, rows):
             assert_close(y.cpu().numpy(), want, what=f"sliced gemv enc={enc} rows={rows}")
             got.append(y.cpu().numpy())
         assert all(np.array_equal(got[0], g) for g in got)
+
+
+@pytest.mark.parametrize("enc", [8, 12, 14, 11, 23, 18])
+@pytest.mark.parametrize("rows", [2, 3, 4, 7])
+def test_gemv_k_slices_over_many_outputs(device, oracle, enc, rows):
+    """K slices of outputs that give a workgroup several 16-row tiles, the last a part: 16387
+    rows, 331 different ones in turn.  y is wider than its rows, and the gap stays as it is."""
+    import torch
+    from kadan_amd import ops
+    n_in, n_out, unique = 14336, 16387, 331
+    w = synth.gguf_weights(enc, 0x53 + rows, unique, n_in)
+    x = synth.normal(0x53 + rows, 5, rows * n_in).reshape(rows, n_in)
+    want = oracle.gemv(enc, w, x, n_in, unique)[:, np.arange(n_out) % unique]
+    wd = torch.from_numpy(w).to(device)[torch.arange(n_out, device=device) % unique].contiguous()
+    xd = torch.from_numpy(x).to(device)
+    forms = [lambda y: ops.gemv(enc, wd, xd, n_out, out=y)]
+    if enc in (8, 12, 14):
+        packed = ops.gguf_pack(enc, wd, n_in)
+        forms.append(lambda y: ops.gemv_packed(enc, packed, xd, n_out, out=y))
+    got = []
+    for product in forms:
+        y = torch.full((rows, n_out + 5), float("nan"), device=device)
+        product(y)
+        y = y.cpu().numpy()
+        assert np.isnan(y[:, n_out:]).all()
+        assert_close(y[:, :n_out], want, what=f"sliced gemv enc={enc} rows={rows}")
+        got.append(y[:, :n_out])
+    assert all(np.array_equal(got[0], g) for g in got)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_gemv_k_slices_flag_a_late_scale(device, packed):
+    """A non-finite scale in the last 256 values, which only the last slice reads."""
+    import torch
+    from kadan_amd import ops
+    n_in, n_out = 14336, 40
+    w = synth.gguf_weights(8, 0x54, n_out, n_in).copy()
+    w[17, -34:-32] = (0x00, 0x7C)
+    wd = torch.from_numpy(w).to(device)
+    x = torch.ones(4, n_in, device=device)
+    status = torch.zeros(1, dtype=torch.int32, device=device)
+    if packed:
+        y = ops.gemv_packed(8, ops.gguf_pack(8, wd, n_in), x, n_out, status=status)
+    else:
+        y = ops.gemv(8, wd, x, n_out, status=status)
+    assert int(status.item()) & 1
+    finite = torch.isfinite(y).cpu().numpy()
+    assert not finite[:, 17].any() and np.delete(finite, 17, 1).all()
