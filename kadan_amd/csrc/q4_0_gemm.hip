@@ -305,8 +305,10 @@ __device__ __forceinline__ f16x8 dequant_dword(unsigned w, f16x2 d, unsigned mag
     return f16x8{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
 }
 
+constexpr int kOperands = 2;          // 32-row weight operands per wavefront
+constexpr int kTiles = 8 * kOperands;  // 16-row weight tiles per workgroup
 // fp32 output row of a sliced tile in LDS (+16: banks)
-template <int NB> constexpr int sliced_pitch = 8 * NB * 16 * 4 + 16;
+constexpr int kSlicedPitch = kTiles * 16 * 4 + 16;
 
 // One group of a 32-row weight operand in a lane's registers: code pieces [j][p] and the
 // scale dwords [j] (d of blocks 4j + 2h and 4j + 2h + 1).
@@ -315,7 +317,7 @@ struct RowGroup {
     unsigned scale[2];
 };
 
-// Workgroup tile: 32 TB tokens x 64*NB weight rows; each of the 4 wavefronts owns NB
+// Workgroup tile: 32 TB tokens x 256 weight rows; each of the 4 wavefronts owns NB = 2
 // 32-row weight operands and all the tokens, so every weight byte is loaded and
 // dequantised once per workgroup, straight into operand registers.  The K loop runs
 // over 256-value groups: per group the workgroup stages its tokens x 512 bytes of
@@ -327,7 +329,7 @@ struct RowGroup {
 // workgroup per compute unit, smaller tiles two.
 // K slices: slice `ks` runs groups [ks * per, (ks + 1) * per) and writes its fp32 tile to
 // part + ks * part_stride, rows `pitch` apart.
-template <int NB, int TB>
+template <int TB>
 __global__ __launch_bounds__(256, TB == 4 ? 1 : 2) void packed_gemm_kernel(
     const uint16_t* __restrict__ xs, const uint8_t* __restrict__ w, unsigned m, unsigned n,
     unsigned k, unsigned slices, unsigned per, uint16_t* __restrict__ y,
@@ -335,7 +337,7 @@ __global__ __launch_bounds__(256, TB == 4 ? 1 : 2) void packed_gemm_kernel(
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr int PM = 32 * TB;                  // tokens per workgroup
     constexpr int kStageBytes = PM * kStageRow;  // one activation stage
-    constexpr int TILES = 8 * NB;                // 16-row weight tiles per workgroup
+    constexpr int NB = kOperands, TILES = kTiles;
     constexpr int DMAS = PM / kDmaRows / 4;      // DMA instructions per wavefront per group
 
     const unsigned groups = k / 256, wtiles = (n + 15) / 16;
@@ -530,7 +532,7 @@ __global__ __launch_bounds__(256, TB == 4 ? 1 : 2) void packed_gemm_kernel(
     __syncthreads();  // every wavefront is done reading the activation stages
     const unsigned f0 = n_tile * TILES * 16;  // first weight row of the tile
     if (slices > 1) {                         // fp32 partials
-        constexpr int kPitch = sliced_pitch<NB>, kChunks = TILES * 16 * 4 / 16;
+        constexpr int kPitch = kSlicedPitch, kChunks = TILES * 16 * 4 / 16;
 #pragma unroll
         for (int c = 0; c < NB; ++c)
 #pragma unroll
@@ -603,8 +605,6 @@ __global__ __launch_bounds__(256) void sum_kernel(const float* __restrict__ part
         out[j] = __builtin_bit_cast(uint16_t, _Float16(vals[j]));
 }
 
-constexpr int kOperands = 2;  // 32-row weight operands per wavefront
-
 // The token tile (TB blocks of 32), the K slices and the scratch of one call.
 struct Plan {
     unsigned blocks, per, slices, pitch;
@@ -624,7 +624,7 @@ struct Plan {
 Plan plan_of(size_t m, size_t n, size_t k) {
     Plan p;
     const size_t units = compute_units(), groups = k / 256;
-    const size_t wtiles = ((n + 15) / 16 + 8 * kOperands - 1) / (8 * kOperands);
+    const size_t wtiles = ((n + 15) / 16 + kTiles - 1) / kTiles;
     p.blocks = m <= 32 ? 1 : (m + 127) / 128 * wtiles * 2 > units ? 4 : 2;
     const size_t tokens = 32 * size_t(p.blocks), tiles = (m + tokens - 1) / tokens * wtiles;
     const size_t slots = units * (p.blocks == 4 ? 1 : 2);
@@ -644,10 +644,10 @@ int launch_tiles(const Plan& p, const uint16_t* xs, const uint8_t* w, unsigned m
                  unsigned k, uint16_t* y, float* part, hipStream_t stream) {
     const unsigned wtiles = (n + 15) / 16;
     const unsigned tiles =
-        unsigned(p.rows / (32 * TB)) * ((wtiles + 8 * kOperands - 1) / (8 * kOperands)) * p.slices;
+        unsigned(p.rows / (32 * TB)) * ((wtiles + kTiles - 1) / kTiles) * p.slices;
     constexpr size_t lds = std::max(size_t(2) * 32 * TB * kStageRow,
-                                    size_t(32) * TB * sliced_pitch<kOperands>);
-    auto kernel = packed_gemm_kernel<kOperands, TB>;
+                                    size_t(32) * TB * kSlicedPitch);
+    auto kernel = packed_gemm_kernel<TB>;
     static bool configured = false;  // one attribute call per instantiation
     if (!configured) {
         KDQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
