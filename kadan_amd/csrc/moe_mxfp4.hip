@@ -773,7 +773,8 @@ __device__ __forceinline__ WavePair wave_pair(const uint8_t* packed, const Packe
     return w;
 }
 
-// Steps per turn of the products' loop (staged_pair).
+// Steps per turn of the products' loop (staged_pair): whole rounds of its buffers and
+// registers.  Slices of up to four or eight steps run one turn of that many instead.
 constexpr unsigned kTurnSteps = 12;
 
 // Steps of a K slice when `steps` are cut into about `slices`: eight (two sets of scales) when
@@ -819,9 +820,9 @@ constexpr int kChunk = 2, kStages = 3, kAheadSteps = 4;
 template <int TERMS, int TILES> constexpr int chunk_bytes = TILES * kChunk * TERMS * 2048;
 
 // acc[m][t] += A(tile t, steps [q0, q1)) * B(group m), q0 % 4 == 0; weights with the
-// non-temporal policy when NT (weights read once per layer call).  Ends with no DMA in
-// flight and `stage` free.
-template <int TERMS, int TILES, bool NT, int WAVES>
+// non-temporal policy when NT (weights read once per layer call).  TURN is kTurnSteps, or
+// four or eight when there are no more steps.  Ends with no DMA in flight and `stage` free.
+template <int TERMS, int TILES, bool NT, int WAVES, unsigned TURN>
 __device__ __forceinline__ void staged_pair(const Tiles& l, unsigned item, unsigned wave,
                                             unsigned lane, const WavePair& w, unsigned q0,
                                             unsigned q1, bool active,
@@ -888,12 +889,17 @@ __device__ __forceinline__ void staged_pair(const Tiles& l, unsigned item, unsig
         }
         issue_order();
     };
-    // The chunk that the next products read has arrived, for every wavefront: behind its DMAs
-    // at least the loads of two chunks (four steps' codes, one set of scales) and the DMAs of
-    // the chunk after were issued.
-    constexpr int kBehind = 2 * kAheadSteps + 2 + TILES + kDmas;
-    static_assert(kBehind < 64, "vmcnt holds six bits");
-    auto arrive = [&]() {
+    // Loads of set i of scales: a turn of four or eight steps has no use for more than one or two
+    // sets (the compiler would drop the others).
+    constexpr auto set_loads = [](int i) {
+        return TURN == kTurnSteps || i * 4 < int(TURN) ? 2 + TILES : 0;
+    };
+    // Chunk C, which the next products read, has arrived, for every wavefront: behind its DMAs
+    // at least the codes of two chunks (four steps), one set of scales if the turn has it, and
+    // the DMAs of the chunk after were issued.
+    auto arrive = [&]<int C>() {
+        constexpr int kBehind = 2 * kAheadSteps + set_loads((C + 1) / 2) + kDmas;
+        static_assert(kBehind < 64, "vmcnt holds six bits");
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kBehind) : "memory");
         __builtin_amdgcn_s_barrier();
         issue_order();
@@ -917,14 +923,19 @@ __device__ __forceinline__ void staged_pair(const Tiles& l, unsigned item, unsig
     // around them would let the compiler move them away from where `arrive` counts them.
     // Chunks past q1 multiply nothing; within a chunk the A operands are read two ahead of
     // their products.
-    for (unsigned qt = q0; qt < q1; qt += kTurnSteps) {
-        static_for<kTurnSteps / kChunk>([&]<int C>() {
+    // Each of those chunks still costs a wait and a barrier, hence the turns of four and eight
+    // for slices of no more steps (1660 tokens, top 2 of 64 experts, 128 -> 4928, two steps:
+    // 90 us in turns of four, 112 in twelve).  They are loops too, though one turn is all:
+    // without a next turn that could read them the compiler drops loads of codes that `arrive`
+    // counts, or moves them past its waits.
+    for (unsigned qt = q0; qt < q1; qt += TURN) {
+        static_for<TURN / kChunk>([&]<int C>() {
             constexpr int kOperands = kChunk * TILES * TERMS, kReadAhead = 2;
             const unsigned qc = qt + C * kChunk;
-            arrive();
+            arrive.template operator()<C>();
             // two chunks ahead, into the buffer that the previous chunk's products have left
             stage_x(qc + 2 * kChunk, stage[(C + 2) % kStages]);
-            if constexpr (C % 2 == 0)
+            if constexpr (C % 2 == 0 && set_loads(C / 2 + 1) > 0)
                 load_scales(qc + 4, scales[(C / 2 + 1) % 3]);
             if (qc < q1) {
                 v8i32 av[kReadAhead + 1];
@@ -1082,7 +1093,7 @@ __device__ __forceinline__ ItemCell item_cell(unsigned cols) {
 // per (tile row, feature) (finalize_kernel).
 // Three workgroups per compute unit (168 registers, no spill): measured 187 -> 174 us at
 // T = 256 and 0.79 -> 0.75 ms at C5.  (down_kernel would spill at that cap.)
-template <bool NT>
+template <bool NT, unsigned TURN>
 __global__ __launch_bounds__(kGemmWaves * 64, 3) void gate_up_kernel(
     const uint8_t* __restrict__ xa, unsigned hidden, unsigned inter, unsigned experts,
     size_t tiles, const uint8_t* __restrict__ gate, const uint8_t* __restrict__ up,
@@ -1119,8 +1130,8 @@ __global__ __launch_bounds__(kGemmWaves * 64, 3) void gate_up_kernel(
 
     auto run = [&]<int TILES>() {
         f32x16 acc[2][TILES];
-        staged_pair<kXTerms, TILES, NT, kGemmWaves>(xl, cell.item, wave, lane, wp, q0, q1, active,
-                                                    stage, acc);
+        staged_pair<kXTerms, TILES, NT, kGemmWaves, TURN>(xl, cell.item, wave, lane, wp, q0, q1,
+                                                          active, stage, acc);
         if (!active)
             return;
         if (gridDim.z > 1) {
@@ -1177,7 +1188,7 @@ __global__ __launch_bounds__(256) void finalize_kernel(const float* __restrict__
 // down: grid (cells of item_cell: groups of row pairs of 64 x items, K slices); wavefront w
 // multiplies the down rows 64 (kDownWaves col + w) .. +63 (two groups of 32).  fp32 partial
 // sums of h x down per slice, indexed by the slot's position in the permutation.
-template <bool NT>
+template <bool NT, unsigned TURN>
 __global__ __launch_bounds__(kDownWaves * 64) void down_kernel(
     const uint8_t* __restrict__ ha, size_t tiles, unsigned hidden, unsigned inter,
     unsigned experts, const uint8_t* __restrict__ down, const int32_t* __restrict__ offsets,
@@ -1207,8 +1218,8 @@ __global__ __launch_bounds__(kDownWaves * 64) void down_kernel(
     const Tiles hl = tile_layout(const_cast<uint8_t*>(ha), tiles, inter / 64, kHTerms);
     auto run = [&]<int TILES>() {
         f32x16 acc[2][TILES];
-        staged_pair<kHTerms, TILES, NT, kDownWaves>(hl, cell.item, wave, lane, w, q0, q1, active,
-                                                    stage, acc);
+        staged_pair<kHTerms, TILES, NT, kDownWaves, TURN>(hl, cell.item, wave, lane, w, q0, q1,
+                                                          active, stage, acc);
         if (!active)
             return;
 #pragma unroll
@@ -2072,8 +2083,19 @@ int launch_layer(const uint16_t* x_bf16, const float* logits, size_t tokens, siz
     const unsigned items8 = (items + 7) / 8 * 8;
     const unsigned gu_cols = gate_up_columns(inter), d_cols = down_columns(hidden);
     const dim3 gu_grid(gu_cols * items8, 1, ks.gate_up);
-    const auto gate_up = nt ? gate_up_kernel<true> : gate_up_kernel<false>;
-    const auto down_product = nt ? down_kernel<true> : down_kernel<false>;
+    // the turn by the longest slice's steps
+    const auto by_turn = [](size_t steps, unsigned slices, auto four, auto eight, auto twelve) {
+        const size_t most = std::min<size_t>(steps, steps_per_slice(unsigned(steps), slices));
+        return most <= 4 ? four : most <= 8 ? eight : twelve;
+    };
+    const auto pick = [&]<bool NT>() {
+        return std::pair(by_turn(hidden / kStepK, ks.gate_up, gate_up_kernel<NT, 4>,
+                                 gate_up_kernel<NT, 8>, gate_up_kernel<NT, kTurnSteps>),
+                         by_turn(inter / kStepK, ks.down, down_kernel<NT, 4>,
+                                 down_kernel<NT, 8>, down_kernel<NT, kTurnSteps>));
+    };
+    const auto [gate_up, down_product] =
+        nt ? pick.template operator()<true>() : pick.template operator()<false>();
     hipLaunchKernelGGL(gate_up, gu_grid, dim3(kGemmWaves * 64), 0, st, s.xa,
                        unsigned(hidden), unsigned(inter), unsigned(experts), tiles, gate, up,
                        s.offsets, s.items, s.item_count, s.ha, s.part_g, s.part_u, part_gu,

@@ -192,6 +192,10 @@ def run_layer(device, oracle, tokens, hidden, inter, experts, top_k, seed, hot=0
     # K of 23, 13, 25 and 7 steps (part turns of the products' 12-step loop, in one slice and
     # in several), few experts with many rows each
     (70, 1472, 832, 8, 3), (20, 832, 1600, 4, 1), (700, 448, 320, 4, 2),
+    # K of 4, 5, 8 and 9 steps (the products' turns of four, eight and twelve), and slices of
+    # eight steps of a longer K
+    (70, 256, 512, 8, 3), (70, 320, 576, 4, 2), (200, 512, 256, 4, 2), (9, 576, 320, 8, 2),
+    (2, 1088, 1216, 64, 2),
     (16, 2880, 2880, 32, 4),
     # more than 4096 slots (the chunked permutation): heavy items first, and experts of
     # several work items each
