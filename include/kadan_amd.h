@@ -95,6 +95,9 @@ int kdq_dequantize(int encoding, const void* packed, size_t row_bytes, size_t ro
  * the activation operand is carried as 16-bit
  * block fixed point per 32 values (relative error below 2^-15 of the block maximum),
  * products exact in int32; every other shape and encoding runs kdq_gemv_exact.
+ * Rows of 12288 values and more that run together (2 to 4 to a pass, where their staged form
+ * does not fit a workgroup's LDS) are summed over K in parts: such a row's last bits may
+ * differ from the same row's alone.  Shorter rows give the same bits either way.
  * `status`: as kdq_dequantize, set when a block scale is not finite. */
 int kdq_gemv(int encoding, const void* weights, size_t row_bytes, const float* x, size_t rows,
              size_t in, size_t out, float* y, size_t stride, unsigned* status, void* stream);

@@ -18,13 +18,13 @@
 //                      group (the permutation depends on the format's packed lane image)
 //   stream_gemm_kernel<ENC, PAIR>  short chunks and grouped (MoE) layers: 64-token tiles,
 //                      the weights of two groups in flight
-//   gemm_kernel<ENC, W> 128 tokens x 256 weight rows per workgroup, W = 4 wavefronts
-//                      each owning two 32-row weight operands (W = 8: one) and all 128
-//                      tokens; weights go from HBM straight into operand registers
-//                      (16-byte loads of the packed lane images, issued one group
-//                      ahead) and are dequantised there; activations are staged into
-//                      swizzled LDS by global->LDS DMA; the fp32 output tile leaves
-//                      through LDS as whole rows.
+//   gemm_kernel<ENC, W, TB>  128 tokens (TB = 4; TB = 3: 96) x 256 weight rows per
+//                      workgroup, W = 4 wavefronts each owning two 32-row weight operands
+//                      (W = 8: one) and all the tokens; weights go from HBM straight
+//                      into operand registers (16-byte loads of the packed lane images,
+//                      issued one group ahead) and are dequantised there; activations
+//                      are staged into swizzled LDS by buffer->LDS DMA; the fp32 output
+//                      tile leaves through LDS as whole rows.
 #include "kdq_common.hpp"
 
 #include <algorithm>
@@ -651,8 +651,10 @@ __global__ __launch_bounds__(W * 64, 1) void gemm_kernel(
 // after the next as soon as each is read out (free_at), which keeps between one and two
 // groups per wavefront in flight in two groups' registers, and a group ends by waiting only
 // for its activation DMA, which goes out first (the counted wait below).  Past the last
-// group the loads go on, all lanes to one line: the count stays the same and nothing is read
-// twice.  (Before, the next group's loads were spread over a group and waited for at its
+// group the loads go on, so that the count stays the same: the DMAs to one address, the
+// weights to group 0 of the operand's first tile, up to two groups' worth that nothing reads
+// (with those to one address per wavefront too, 720 dense calls took 0.998 of the time, the
+// short ones as well).  (Before, the next group's loads were spread over a group and waited for at its
 // end, most of their latency showing; at 4096 slots over 128 experts, Q4_K gate / up 2048 ->
 // 768: 90 -> 68 us, the 226 MB of weights at 3.3 TB/s; Q6_K down 768 -> 2048: 72 -> 58.)
 // Only the tile's live tokens cost anything: the DMA of a dead one repeats token 0's lines,

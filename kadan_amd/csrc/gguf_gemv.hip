@@ -1724,7 +1724,10 @@ int launch_sliced(const uint8_t* w, size_t row_bytes, const float* x, size_t in,
 // 14336 -> 4096 42.7 us in two passes of 2 rows, 26.8 in two slices of 4.  Passes of 8 rows
 // gain nothing over two of 4 (Q8_0 7168 -> 16384: 54.7 us, in two slices of 8 57.2): the
 // products then outweigh the weights.  Nor do 4 rows of a shorter input (Q4_K 9216 -> 6562,
-// packed: 21.7 us in two passes of 2, 22.6 in slices; 14336 -> 4096 24.8 and 21.1).
+// packed: 21.7 us in two passes of 2, 22.6 in slices; 14336 -> 4096 24.8 and 21.1).  The line
+// was drawn by Q4_K and holds for every encoding: of 1500 products of 12288 to 28672 inputs and
+// 2 to 8 rows none was slower for its slices.  A row's sum is then in two parts, so its last
+// bits are not those of the row alone.
 constexpr size_t kSlicedInputs = 12288;
 
 template <int ENC, bool PACKED>

@@ -277,3 +277,18 @@ def test_gemv_k_slices_flag_a_late_scale(device, packed):
     assert int(status.item()) & 1
     finite = torch.isfinite(y).cpu().numpy()
     assert not finite[:, 17].any() and np.delete(finite, 17, 1).all()
+
+
+@pytest.mark.parametrize("enc", [2, 8, 12, 14, 11, 23, 20, 18, 21, 22])
+@pytest.mark.parametrize("n_in", [768, 4096, 11264])
+def test_gemv_row_bits_alone_and_together(device, enc, n_in):
+    """Below 12288 inputs a row gives the same bits alone as in a batch."""
+    import torch
+    from kadan_amd import ops
+    n_out, rows = 300, 7
+    w = torch.from_numpy(synth.gguf_weights(enc, 0x55, n_out, n_in)).to(device)
+    x = torch.from_numpy(synth.normal(0x55, 5, rows * n_in).reshape(rows, n_in)).to(device)
+    together = ops.gemv(enc, w, x, n_out)
+    for r in range(rows):
+        alone = ops.gemv(enc, w, x[r:r + 1].contiguous(), n_out)
+        assert torch.equal(alone[0].view(torch.int32), together[r].view(torch.int32)), r
