@@ -780,7 +780,7 @@ constexpr unsigned kTurnSteps = 12;
 // Steps of a K slice when `steps` are cut into about `slices`: eight (two sets of scales) when
 // they are short, else whole turns of the products' loop, unless that leaves the last slice
 // less than half a slice; then whole sets of scales.
-__host__ __device__ inline unsigned steps_per_slice(unsigned steps, unsigned slices) {
+inline unsigned steps_per_slice(unsigned steps, unsigned slices) {
     const unsigned even = (steps + slices - 1) / slices;
     if (even <= 8)
         return 8;
@@ -789,10 +789,9 @@ __host__ __device__ inline unsigned steps_per_slice(unsigned steps, unsigned sli
     return turns == kTurnSteps || last * 2 >= turns ? turns : (even + 3) / 4 * 4;
 }
 
-// K slice `slice` of `slices`: [begin, end) in steps, begin a multiple of 4.
-__device__ __forceinline__ void slice_steps(unsigned steps, unsigned slices, unsigned slice,
+// K slice `slice` of `per` steps (a multiple of 4): [begin, end) in steps.
+__device__ __forceinline__ void slice_steps(unsigned steps, unsigned per, unsigned slice,
                                             unsigned& begin, unsigned& end) {
-    const unsigned per = steps_per_slice(steps, slices);
     begin = min(steps, slice * per);
     end = min(steps, begin + per);
 }
@@ -1102,7 +1101,7 @@ __global__ __launch_bounds__(kGemmWaves * 64, 3) void gate_up_kernel(
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ items,
     const int32_t* __restrict__ item_count, uint8_t* __restrict__ ha,
     float* __restrict__ part_g, float* __restrict__ part_u, size_t part_stride,
-    unsigned cols) {
+    unsigned cols, unsigned per) {
     __shared__ __align__(16) uint8_t stage0[chunk_bytes<kXTerms, 2>],
         stage1[chunk_bytes<kXTerms, 2>], stage2[chunk_bytes<kXTerms, 2>];
     uint8_t* const stage[kStages] = {stage0, stage1, stage2};
@@ -1118,7 +1117,7 @@ __global__ __launch_bounds__(kGemmWaves * 64, 3) void gate_up_kernel(
     const bool active = fg < shape.groups;                // uniform per wavefront
     const unsigned f = (active ? fg : 0) * 32 + i32;
     unsigned q0, q1;
-    slice_steps(unsigned(shape.steps), gridDim.z, blockIdx.z, q0, q1);
+    slice_steps(unsigned(shape.steps), per, blockIdx.z, q0, q1);
     if (q0 >= q1)
         return;
     const Packed whole = packed_shape(experts, inter, hidden);
@@ -1195,7 +1194,7 @@ __global__ __launch_bounds__(kDownWaves * 64) void down_kernel(
     const uint8_t* __restrict__ ha, size_t tiles, unsigned hidden, unsigned inter,
     unsigned experts, const uint8_t* __restrict__ down, const int32_t* __restrict__ offsets,
     const int32_t* __restrict__ items, const int32_t* __restrict__ item_count,
-    float* __restrict__ part_d, size_t part_stride, unsigned cols) {
+    float* __restrict__ part_d, size_t part_stride, unsigned cols, unsigned per) {
     __shared__ __align__(16) uint8_t stage0[chunk_bytes<kHTerms, 2>],
         stage1[chunk_bytes<kHTerms, 2>], stage2[chunk_bytes<kHTerms, 2>];
     uint8_t* const stage[kStages] = {stage0, stage1, stage2};
@@ -1211,7 +1210,7 @@ __global__ __launch_bounds__(kDownWaves * 64) void down_kernel(
     const bool active = pair < shape.groups / 2;
     const unsigned g0 = (active ? pair : 0) * 2;
     unsigned q0, q1;
-    slice_steps(unsigned(shape.steps), gridDim.z, blockIdx.z, q0, q1);
+    slice_steps(unsigned(shape.steps), per, blockIdx.z, q0, q1);
     if (q0 >= q1)
         return;
     const Packed whole = packed_shape(experts, hidden, inter);
@@ -1723,7 +1722,8 @@ unsigned down_columns(size_t hidden) {
 // K slices of the grouped GEMMs: enough workgroups for about two per compute unit (two
 // fit at once) when the items are few (decode), one slice otherwise; none is empty.
 struct MoeSlices {
-    unsigned gate_up, down;
+    unsigned gate_up, down;              // K slices
+    unsigned gate_up_steps, down_steps;  // steps of each but the last
 };
 
 MoeSlices moe_slices(size_t tokens, size_t hidden, size_t inter, size_t experts,
@@ -1732,9 +1732,16 @@ MoeSlices moe_slices(size_t tokens, size_t hidden, size_t inter, size_t experts,
     // (4096 slots over 8 experts, counted as 8 items, ran gate / up in three slices: 420 us)
     const size_t slots = tokens * top_k;
     const size_t items = std::max(std::min(slots, experts), slots / kItemRows);
+    // and with rows spread around a mean near whole items or above, half of the experts have an
+    // item more
+    const size_t many = slots > 40 * experts
+                            ? std::max(items, slots / kItemRows + experts / 2) : items;
+    struct Slices {
+        unsigned count, steps;
+    };
     // workgroups for about two gate/up (four waves) or one down (eight waves) per compute
     // unit
-    auto slices = [&](size_t columns, size_t steps, size_t per_cu, bool round_up) {
+    auto slices = [&](size_t columns, size_t steps, size_t per_cu, bool round_up) -> Slices {
         const size_t target = per_cu * size_t(compute_units());
         size_t ks = round_up ? (target + columns * items - 1) / (columns * items)
                              : target / (columns * items);
@@ -1742,7 +1749,17 @@ MoeSlices moe_slices(size_t tokens, size_t hidden, size_t inter, size_t experts,
         const auto count = [&](size_t per) { return (steps + per - 1) / per; };
         // no more than slices of whole eights would give: the partials of more took layers
         // past the static scratch below (64 -> 2496, 64 experts, 4096 slots: 4 for 3)
-        const size_t even = (steps + ks - 1) / ks, eights = count((even + 7) / 8 * 8);
+        const size_t even = (steps + ks - 1) / ks, rounded = (even + 7) / 8 * 8,
+                     eights = count(rounded);
+        // Where down's workgroups leave an XCD less than a quarter of its compute units spare,
+        // some wait for a second round (those without an item take places in turn as well): then
+        // slices of whole eights, whose last one is short, and not equal ones (9 tokens over 8
+        // experts, 3584 -> 4672, 30 workgroups on each XCD's 32 units: 18.0 us in 24, 24 and 8
+        // steps, 26.1 in 20, 20 and 16; 70 tokens over 16 experts, 2240 -> 2048, 24 on each: 23.1
+        // in 16, 16 and 3, 20.4 in 12, 12 and 11).
+        if (per_cu == 1 && even > 8 &&
+            columns * ((many + 7) / 8) * eights * 8 * 4 > 3 * size_t(compute_units()))
+            return {unsigned(eights), unsigned(rounded)};
         // short slices: a whole turn each where that still gives three compute units in four
         // a workgroup (264 tokens, top 2 of 8, 1536 -> 1856: 62.9 us, with eights 65.2), else
         // eights (2 tokens, 64 experts, 1024 -> 2048: 25.1 us, with turns 27.7)
@@ -1754,12 +1771,13 @@ MoeSlices moe_slices(size_t tokens, size_t hidden, size_t inter, size_t experts,
         // and none empty: fewer slices may be longer ones, so until the count stands
         for (size_t n; (n = count(steps_per_slice(unsigned(steps), unsigned(ks)))) < ks;)
             ks = n;
-        return unsigned(ks);
+        return {unsigned(ks), steps_per_slice(unsigned(steps), unsigned(ks))};
     };
     // down rounds down: its workgroups (one per compute unit at its register count) then
     // run in one round rather than one and a part (C4 T=256: 1 slice, 192 workgroups)
-    return MoeSlices{slices(gate_up_columns(inter), hidden / kStepK, 2, true),
-                     slices(down_columns(hidden), inter / kStepK, 1, false)};
+    const Slices gate_up = slices(gate_up_columns(inter), hidden / kStepK, 2, true);
+    const Slices down = slices(down_columns(hidden), inter / kStepK, 1, false);
+    return MoeSlices{gate_up.count, down.count, gate_up.steps, down.steps};
 }
 
 size_t align256(size_t n) {
@@ -2086,14 +2104,14 @@ int launch_layer(const uint16_t* x_bf16, const float* logits, size_t tokens, siz
     const unsigned gu_cols = gate_up_columns(inter), d_cols = down_columns(hidden);
     const dim3 gu_grid(gu_cols * items8, 1, ks.gate_up);
     // the turn by the longest slice's steps
-    const auto by_turn = [](size_t steps, unsigned slices, auto four, auto eight, auto twelve) {
-        const size_t most = std::min<size_t>(steps, steps_per_slice(unsigned(steps), slices));
+    const auto by_turn = [](size_t steps, unsigned per, auto four, auto eight, auto twelve) {
+        const size_t most = std::min<size_t>(steps, per);
         return most <= 4 ? four : most <= 8 ? eight : twelve;
     };
     const auto pick = [&]<bool NT>() {
-        return std::pair(by_turn(hidden / kStepK, ks.gate_up, gate_up_kernel<NT, 4>,
+        return std::pair(by_turn(hidden / kStepK, ks.gate_up_steps, gate_up_kernel<NT, 4>,
                                  gate_up_kernel<NT, 8>, gate_up_kernel<NT, kTurnSteps>),
-                         by_turn(inter / kStepK, ks.down, down_kernel<NT, 4>,
+                         by_turn(inter / kStepK, ks.down_steps, down_kernel<NT, 4>,
                                  down_kernel<NT, 8>, down_kernel<NT, kTurnSteps>));
     };
     const auto [gate_up, down_product] =
@@ -2101,7 +2119,7 @@ int launch_layer(const uint16_t* x_bf16, const float* logits, size_t tokens, siz
     hipLaunchKernelGGL(gate_up, gu_grid, dim3(kGemmWaves * 64), 0, st, s.xa,
                        unsigned(hidden), unsigned(inter), unsigned(experts), tiles, gate, up,
                        s.offsets, s.items, s.item_count, s.ha, s.part_g, s.part_u, part_gu,
-                       gu_cols);
+                       gu_cols, ks.gate_up_steps);
     KDQ_HIP(hipGetLastError());
     if (ks.gate_up > 1) {
         hipLaunchKernelGGL(finalize_kernel, dim3(unsigned((inter + 255) / 256), unsigned(slots)),
@@ -2113,7 +2131,8 @@ int launch_layer(const uint16_t* x_bf16, const float* logits, size_t tokens, siz
     const dim3 d_grid(d_cols * items8, 1, ks.down);
     hipLaunchKernelGGL(down_product, d_grid, dim3(kDownWaves * 64), 0, st,
                        s.ha, tiles, unsigned(hidden), unsigned(inter), unsigned(experts), down,
-                       s.offsets, s.items, s.item_count, s.part_d, stride, d_cols);
+                       s.offsets, s.items, s.item_count, s.part_d, stride, d_cols,
+                       ks.down_steps);
     KDQ_HIP(hipGetLastError());
     const size_t n = tokens * hidden / 4;
     const dim3 grid(unsigned((n + 255) / 256));
