@@ -172,7 +172,8 @@ int kdq_gemv_packed_supported(int encoding, size_t in);
  * (amax/127, codes round-half-even(x*127/amax), G/src/ggml-cpu/arch/x86/quants.c:302-398).
  * y[m x n] fp16 = sum_b float(sumi_b) * d_w * d_x, fp32 accumulation.
  * k % 256 == 0; any m, n >= 1.  Weights of up to 256 MiB are packed into the library's
- * workspace first, on each call, where that is faster (and its memory can be had). */
+ * workspace first, on each call, where that is faster and its memory can be had (a call that
+ * is being captured takes only the workspace there is). */
 int kdq_gemm_q4_0(const void* weights, size_t n, size_t k, const uint16_t* x_f16, size_t m,
                   uint16_t* y_f16, void* stream);
 

@@ -56,6 +56,21 @@ void* workspace(size_t bytes, int* status) {
     return w.ptr;
 }
 
+bool workspace_usable(size_t bytes, hipStream_t stream) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;  // workspace() reports what is wrong
+    }
+    if (capture == hipStreamCaptureStatusNone)
+        return true;
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess)
+        return true;
+    std::lock_guard<std::mutex> lock(workspace_mutex);
+    return workspaces.size() > size_t(device) && workspaces[size_t(device)].bytes >= bytes;
+}
+
 unsigned compute_units() {
     static std::mutex mutex;
     static std::vector<unsigned> cached;

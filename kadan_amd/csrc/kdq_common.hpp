@@ -316,6 +316,10 @@ int hip_failure(hipError_t error);
 // Per-device cached workspace (grown on demand, released by kdq_release_scratch).
 void* workspace(size_t bytes, int* status);
 
+// Whether workspace(bytes) may be tried for work on `stream`: not where the stream is being
+// captured and the workspace would have to grow (it waits for the device, which ends a capture).
+bool workspace_usable(size_t bytes, hipStream_t stream);
+
 // Compute units of the current device (cached per device; 256 if the query fails).
 unsigned compute_units();
 

@@ -747,9 +747,13 @@ extern "C" int kdq_gemm_q4_0(const void* weights, size_t n, size_t k, const uint
     if (pack_first(m, n, k)) {
         const Plan p = plan_of(m, n, k);
         const size_t at = (p.total + 255) & ~size_t(255);
-        auto* base = static_cast<uint8_t*>(
-            workspace(at + kdq_gguf_packed_bytes(KDQ_Q4_0, k, n), &rc));
-        if (rc != KDQ_ERR_SCRATCH) {  // (no memory for the copy: from the rows)
+        const size_t total = at + kdq_gguf_packed_bytes(KDQ_Q4_0, k, n);
+        // no memory for the copy, or a capture, which cannot allocate it: from the rows
+        rc = KDQ_ERR_SCRATCH;
+        uint8_t* base = nullptr;
+        if (workspace_usable(total, st))
+            base = static_cast<uint8_t*>(workspace(total, &rc));
+        if (rc != KDQ_ERR_SCRATCH) {
             if (rc || (rc = kdq_gguf_pack(KDQ_Q4_0, weights, (k / 32) * 18, k, n, base + at, st)))
                 return rc;
             return run_packed(p, x_f16, base + at, m, n, k, y_f16, base, st);

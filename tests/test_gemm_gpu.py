@@ -184,3 +184,36 @@ def test_gemm_q4_0_rows_holds_no_copy_of_large_weights(device, m, k, n):
     torch.cuda.synchronize()
     assert before - torch.cuda.mem_get_info()[0] < 64 << 20
     assert not y.any()  # d = 0
+
+
+def test_gemm_q4_0_rows_captured_in_a_small_workspace(device):
+    """A shape that packs first, captured while the workspace holds its activations but not the
+    weights' copy (which a capture cannot allocate): taken from the rows.  Each replay is
+    within this file's tolerance of the eager result (the same fp16 weights and activations,
+    summed in another order)."""
+    torch = _torch()
+    import kadan_amd
+    from kadan_amd import ops
+    m, k, n = 70, 2304, 2000
+    _, _, wd, xd = _rows_case(device, m, k, n)
+    xs = [xd, (xd * 0.5).contiguous(), xd.flip(0).contiguous()]
+    eager = [ops.gemm_q4_0(wd, x, n).clone() for x in xs]
+    torch.cuda.synchronize()
+    kadan_amd.call("kdq_release_scratch")
+    _, _, ws, xsmall = _rows_case(device, m, 512, 300)
+    ops.gemm_q4_0(ws, xsmall, 300)  # the least workspace, 1 MiB: not the 2.6 MB copy
+    static = xs[0].clone()
+    out = torch.zeros(m, n, dtype=torch.float16, device=device)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ops.gemm_q4_0(wd, static, n, out=out)
+    for i in (1, 0, 2, 2, 1):
+        static.copy_(xs[i])
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close(out.float().cpu().numpy(), eager[i].float().cpu().numpy(), rel=1e-3,
+                     mabs=2e-2, what=f"replay of input {i}")
+        ops.gemm_q4_0(ws, xsmall, 300)  # eager work between replays, in the same workspace
