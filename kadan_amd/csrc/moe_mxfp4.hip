@@ -1751,15 +1751,6 @@ MoeSlices moe_slices(size_t tokens, size_t hidden, size_t inter, size_t experts,
         // past the static scratch below (64 -> 2496, 64 experts, 4096 slots: 4 for 3)
         const size_t even = (steps + ks - 1) / ks, rounded = (even + 7) / 8 * 8,
                      eights = count(rounded);
-        // Where down's workgroups leave an XCD less than a quarter of its compute units spare,
-        // some wait for a second round (those without an item take places in turn as well): then
-        // slices of whole eights, whose last one is short, and not equal ones (9 tokens over 8
-        // experts, 3584 -> 4672, 30 workgroups on each XCD's 32 units: 18.0 us in 24, 24 and 8
-        // steps, 26.1 in 20, 20 and 16; 70 tokens over 16 experts, 2240 -> 2048, 24 on each: 23.1
-        // in 16, 16 and 3, 20.4 in 12, 12 and 11).
-        if (per_cu == 1 && even > 8 &&
-            columns * ((many + 7) / 8) * eights * 8 * 4 > 3 * size_t(compute_units()))
-            return {unsigned(eights), unsigned(rounded)};
         // short slices: a whole turn each where that still gives three compute units in four
         // a workgroup (264 tokens, top 2 of 8, 1536 -> 1856: 62.9 us, with eights 65.2), else
         // eights (2 tokens, 64 experts, 1024 -> 2048: 25.1 us, with turns 27.7)
@@ -1771,7 +1762,23 @@ MoeSlices moe_slices(size_t tokens, size_t hidden, size_t inter, size_t experts,
         // and none empty: fewer slices may be longer ones, so until the count stands
         for (size_t n; (n = count(steps_per_slice(unsigned(steps), unsigned(ks)))) < ks;)
             ks = n;
-        return {unsigned(ks), steps_per_slice(unsigned(steps), unsigned(ks))};
+        const Slices equal{unsigned(ks), steps_per_slice(unsigned(steps), unsigned(ks))};
+        // Down runs one workgroup per compute unit.  Where those of an XCD pass its 32 units, the
+        // last slices run in a second round, and slices of whole eights with a last one of half
+        // or less are better than as many equal ones (385 such layers: 0.98 of the time at the
+        // median, 0.89 to 1.08; 353 tokens, top 4 of 8 experts, 3712 -> 1408, 36 workgroups: the
+        // layer 100 us in 24, 24 and 10 steps, 113 in 20, 20 and 18).  The same within an eighth
+        // of the units, where an item more than counted, or a cell without one, passes them, and
+        // equal slices save a sixth at most (236 layers: 1.009, 0.87 to 1.03; 18 tokens, top 8 of
+        // 8, 3712 -> 4992, 30 workgroups: 79 and 88 us).  Elsewhere equal ones: below, 0.95, and
+        // where they are fewer.
+        const size_t places = columns * ((many + 7) / 8) * eights * 8, units = compute_units();
+        const bool second = places > units ||
+                            (places * 8 > units * 7 && equal.steps * 6 >= rounded * 5);
+        if (per_cu == 1 && even > 8 && ks == eights &&
+            steps * 2 <= (2 * eights - 1) * rounded && second)
+            return {unsigned(eights), unsigned(rounded)};
+        return equal;
     };
     // down rounds down: its workgroups (one per compute unit at its register count) then
     // run in one round rather than one and a part (C4 T=256: 1 slice, 192 workgroups)

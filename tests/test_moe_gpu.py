@@ -196,8 +196,10 @@ def run_layer(device, oracle, tokens, hidden, inter, experts, top_k, seed, hot=0
     # eight steps of a longer K
     (70, 256, 512, 8, 3), (70, 320, 576, 4, 2), (200, 512, 256, 4, 2), (9, 576, 320, 8, 2),
     (2, 1088, 1216, 64, 2),
-    # down's K slices unequal (16 and 3 steps): its workgroups leave few compute units spare
+    # down's K slices where an XCD's workgroups come close to its compute units (two of 12 and 7
+    # steps) and where they pass them (16 and 3)
     (12, 2112, 1216, 24, 2),
+    (9, 2624, 1216, 17, 2),
     (16, 2880, 2880, 32, 4),
     # more than 4096 slots (the chunked permutation): heavy items first, and experts of
     # several work items each
